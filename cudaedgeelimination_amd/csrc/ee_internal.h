@@ -130,6 +130,16 @@ struct KoptLaunch {
   // deleted_cost (the cells TryReconnectFromCostRow rechecks)
   uint32_t* masks;
   uint32_t mask_words;
+  // packed_lo non-null: instead of int64 cells, write each cell's transfer
+  // form (ExpandCells): its low word to packed_lo[cell] and, on instances
+  // that are not near, its high byte to packed_hi[cell], both in host memory;
+  // once tile i's cells are there, `mark` goes to marks[i].  Task rows are
+  // then read as another agent's: node ids at or above bound_nodes read node 0.
+  uint32_t* packed_lo;
+  uint8_t* packed_hi;
+  uint64_t* marks;
+  uint64_t mark;
+  uint32_t bound_nodes;
   KoptKLayout layout[3];
   uint32_t wave_base;   // LDS offset of the first wave's tile arrays
   uint32_t wave_bytes;  // LDS bytes per wave
@@ -148,6 +158,15 @@ struct KoptTuning {
   uint32_t block = 256;
   bool non_temporal = false;
 };
+
+// A cell in transfer form: costs are below 2^35, so the low word and, where a
+// cost can reach 2^32 - 1 (an instance that is not near), the high byte hold
+// it exactly; an invalid cell (INT64_MAX) is all ones in the word, or in the
+// byte.  ExpandCells writes cells [0, count) back as int64 on the host; hi is
+// null for near instances, whose costs are below 5 x 2^26.
+constexpr uint32_t kPackedInvalid = 0xffffffffu;
+constexpr uint8_t kPackedInvalidHi = 0xff;
+void ExpandCells(const uint32_t* lo, const uint8_t* hi, size_t count, int64_t* cells);
 
 // Number of tiles the segments split into under `tuning`.
 uint64_t KoptCountTiles(const KoptSegment* segments, size_t count, const KoptTuning& tuning);

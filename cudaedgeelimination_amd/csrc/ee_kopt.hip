@@ -51,6 +51,11 @@ constexpr uint64_t kBadMask = (uint64_t{0xAAAAA} << kCounterBase) | (uint64_t{7}
 constexpr uint32_t kNearPortBytes = 16;
 constexpr uint32_t kFarPortBytes = 32;
 
+// What phase C writes: int64 cells, the rows' improving-template masks, or
+// cells in transfer form (KoptLaunch::packed_lo) straight to page-locked host
+// memory.
+enum KoptOut { kOutCells, kOutMasks, kOutPacked };
+
 // The launch's buffers, taken from the kernel arguments.
 struct KoptPointers {
   const longlong2* xy;
@@ -59,6 +64,8 @@ struct KoptPointers {
   const KoptPlan* plans;
   int64_t* costs;
   uint32_t* masks;
+  uint32_t* packed_lo;
+  uint8_t* packed_hi;
   // measurement only (null otherwise): wavefront w of the launch writes the
   // constant-rate device clock at its start to stamps[2w] and at its end to
   // stamps[2w + 1]
@@ -104,7 +111,7 @@ __device__ __forceinline__ void StoreCell(int64_t* out, uint32_t at, uint64_t su
 // free until phase B) and their coordinates, two gathers in flight per lane.
 // kBounded: node ids at or above node_count read node 0's coordinates (task
 // rows that another agent wrote, whose checks this kernel cannot see).
-template <int K, bool kNear, bool kMask, bool kBounded = false>
+template <int K, bool kNear, int kOut, bool kBounded = kOut == kOutPacked>
 __device__ __forceinline__ void StagePorts(const KoptLaunch& a, const KoptPointers& bufs, const KoptKLayout& L,
                                            const KoptTile& d, char* wave, int lane, uint32_t node_count = 0) {
   constexpr uint32_t kPorts = 2 * K;
@@ -148,7 +155,7 @@ __device__ __forceinline__ void StagePorts(const KoptLaunch& a, const KoptPointe
         if (p == 0) {
           w_row[r] = 0;
           // mask output: the row's deleted_cost (bytes 40..47 of the task row)
-          if (kMask) {
+          if (kOut == kOutMasks) {
             reinterpret_cast<int64_t*>(wave + L.dcost_off)[r] =
                 reinterpret_cast<const int64_t*>(ports + r * 12)[5];
           }
@@ -264,14 +271,21 @@ struct MaskOut {
   uint32_t g;            // lane group (its rows are g, g + G, ...)
 };
 
+// Packed mode: the tile's first cell in the low-word and high-byte planes.
+struct PackedOut {
+  uint32_t* lo;
+  uint8_t* hi;
+};
+
 __device__ __forceinline__ void WriteMaskRow(const MaskOut& m, uint32_t row, bool improving) {
   if (improving) atomicOr(m.stage + row * m.words + m.t / 32, 1u << (m.t % 32));
 }
 
-template <int K, bool kNear, bool kNonTemporal, uint32_t kG, bool kMask>
+template <int K, bool kNear, bool kNonTemporal, uint32_t kG, int kOut>
 __device__ __forceinline__ void CellSteps(const char* pairs, const uint32_t (&off)[K], int64_t* out,
-                                          uint32_t at, uint32_t step_bytes, uint32_t g_rows, uint32_t n,
-                                          bool extra_row, const MaskOut& m) {
+                                          const PackedOut& packed, uint32_t at, uint32_t step_bytes,
+                                          uint32_t g_rows, uint32_t n, bool extra_row, const MaskOut& m) {
+  constexpr bool kMask = kOut == kOutMasks;
   const uint32_t G = kG != 0 ? kG : g_rows;
   auto steps = [&](auto unroll, uint32_t i) {
     constexpr uint32_t U = decltype(unroll)::value;
@@ -331,6 +345,11 @@ __device__ __forceinline__ void CellSteps(const char* pairs, const uint32_t (&of
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u) {
         const bool bad = (hi[u] & static_cast<uint32_t>(kBadMask >> 32)) != 0;
+        if (kOut == kOutPacked) {
+          *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(packed.lo) + at) = bad ? kPackedInvalid : lo[u];
+          at += step_bytes;
+          continue;
+        }
         const int64_t value = bad ? kInvalid : static_cast<int64_t>(lo[u]);
         int64_t* dst = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(out) + at);
         if (kNonTemporal) {
@@ -352,7 +371,15 @@ __device__ __forceinline__ void CellSteps(const char* pairs, const uint32_t (&of
       }
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u) {
-        StoreCell<kNonTemporal>(out, at, sum[u]);
+        if (kOut == kOutPacked) {
+          const uint32_t hi = static_cast<uint32_t>(sum[u] >> 32);
+          const bool bad = (hi & static_cast<uint32_t>(kBadMask >> 32)) != 0;
+          *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(packed.lo) + at) =
+              bad ? kPackedInvalid : static_cast<uint32_t>(sum[u]);
+          packed.hi[at / 4] = bad ? kPackedInvalidHi : static_cast<uint8_t>(hi & 7u);
+        } else {
+          StoreCell<kNonTemporal>(out, at, sum[u]);
+        }
         at += step_bytes;
       }
     }
@@ -364,10 +391,12 @@ __device__ __forceinline__ void CellSteps(const char* pairs, const uint32_t (&of
 }
 
 // Phases A2, B and C of one staged tile.
-template <int K, bool kNear, bool kNonTemporal, bool kMask>
+template <int K, bool kNear, bool kNonTemporal, int kOut>
 __device__ void TileCells(const KoptLaunch& a, const KoptPointers& bufs, const KoptKLayout& L, const KoptTile& d,
                           const char* smem, char* wave, int lane) {
   constexpr uint32_t kPorts = 2 * K;
+  constexpr bool kMask = kOut == kOutMasks;
+  constexpr uint32_t kCellBytes = kOut == kOutPacked ? 4 : 8;
   const uint16_t* s_pq = reinterpret_cast<const uint16_t*>(smem + L.pq_off);
   const uint64_t* s_tpl = reinterpret_cast<const uint64_t*>(smem + L.tpl_off);
   uint32_t* w_row = reinterpret_cast<uint32_t*>(wave + L.row_off);
@@ -424,11 +453,13 @@ __device__ void TileCells(const KoptLaunch& a, const KoptPointers& bufs, const K
   // it walks every row once per pass of 64 templates.
   const uint64_t cost_index = Uniform64(d.cost_index);
   int64_t* const out = bufs.costs + cost_index;
+  PackedOut packed{};
+  if (kOut == kOutPacked) packed = PackedOut{bufs.packed_lo + cost_index, bufs.packed_hi + cost_index};
   const char* const pairs = reinterpret_cast<const char*>(w_pair);
   const uint32_t G = L.group;
   const uint32_t n = __builtin_amdgcn_readfirstlane(rows / G);  // rows every group has
   const uint32_t extra = rows - n * G;                          // groups g < extra have one more
-  const uint32_t step_bytes = G * T * 8;
+  const uint32_t step_bytes = G * T * kCellBytes;
   // mask mode: the tile's mask words are staged in the port records, which
   // phase C no longer reads (the layout sizes them for rows x mask words)
   uint32_t* const w_mask = reinterpret_cast<uint32_t*>(wave + L.xy_off);
@@ -449,7 +480,7 @@ __device__ void TileCells(const KoptLaunch& a, const KoptPointers& bufs, const K
 #pragma unroll
     for (int j = 0; j < K; ++j) off[j] = (static_cast<uint32_t>((tp >> (8 * j)) & 0xffu) * stride + g) * 8;
     // byte offset of the lane's next cell; a tile's cells stay below 2^24
-    const uint32_t at = (g * T + t) * 8;
+    const uint32_t at = (g * T + t) * kCellBytes;
     if (!active) continue;
     // the standard templates give T = 4 / 25 / 208, so G = 16 / 2 / 1: with G
     // a constant the rows of a step are immediate offsets of one address
@@ -462,14 +493,15 @@ __device__ void TileCells(const KoptLaunch& a, const KoptPointers& bufs, const K
       m.t = t;
       m.g = g;
       if (G == kStdG) {
-        CellSteps<K, kNear, kNonTemporal, kStdG, true>(pairs, off, out, at, step_bytes, G, n, g < extra, m);
+        CellSteps<K, kNear, kNonTemporal, kStdG, kOut>(pairs, off, out, packed, at, step_bytes, G, n, g < extra, m);
       } else {
-        CellSteps<K, kNear, kNonTemporal, 0, true>(pairs, off, out, at, step_bytes, G, n, g < extra, m);
+        CellSteps<K, kNear, kNonTemporal, 0, kOut>(pairs, off, out, packed, at, step_bytes, G, n, g < extra, m);
       }
     } else if (G == kStdG) {
-      CellSteps<K, kNear, kNonTemporal, kStdG, false>(pairs, off, out, at, step_bytes, G, n, g < extra, MaskOut{});
+      CellSteps<K, kNear, kNonTemporal, kStdG, kOut>(pairs, off, out, packed, at, step_bytes, G, n, g < extra,
+                                                     MaskOut{});
     } else {
-      CellSteps<K, kNear, kNonTemporal, 0, false>(pairs, off, out, at, step_bytes, G, n, g < extra, MaskOut{});
+      CellSteps<K, kNear, kNonTemporal, 0, kOut>(pairs, off, out, packed, at, step_bytes, G, n, g < extra, MaskOut{});
     }
   }
   WaveSync();
@@ -506,7 +538,7 @@ __device__ __forceinline__ KoptTile TileAt(const KoptLaunch& a, const KoptPointe
 // The tiles of one k handed to this workgroup, one per wavefront at a time.
 // The plan is fetched into registers first, so its latency overlaps the
 // first tile's gathers; it reaches LDS before the only block barrier.
-template <int K, bool kNonTemporal, bool kMask>
+template <int K, bool kNonTemporal, int kOut>
 __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* smem) {
   constexpr int ki = K - 3;
   // k = 5 tiles hold most of the cells and end the launch: their wavefronts
@@ -540,9 +572,9 @@ __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* sm
   if (tile < end) {
     d = TileAt<K>(a, bufs, L, tile);
     if (d.near != 0) {
-      StagePorts<K, true, kMask>(a, bufs, L, d, wave, lane);
+      StagePorts<K, true, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
     } else {
-      StagePorts<K, false, kMask>(a, bufs, L, d, wave, lane);
+      StagePorts<K, false, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
     }
   }
 
@@ -560,33 +592,41 @@ __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* sm
   for (bool first = true; tile < end; tile += stride, first = false) {
     if (!first) d = TileAt<K>(a, bufs, L, tile);
     if (d.near != 0) {
-      if (!first) StagePorts<K, true, kMask>(a, bufs, L, d, wave, lane);
-      TileCells<K, true, kNonTemporal, kMask>(a, bufs, L, d, smem, wave, lane);
+      if (!first) StagePorts<K, true, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+      TileCells<K, true, kNonTemporal, kOut>(a, bufs, L, d, smem, wave, lane);
     } else {
-      if (!first) StagePorts<K, false, kMask>(a, bufs, L, d, wave, lane);
-      TileCells<K, false, kNonTemporal, kMask>(a, bufs, L, d, smem, wave, lane);
+      if (!first) StagePorts<K, false, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+      TileCells<K, false, kNonTemporal, kOut>(a, bufs, L, d, smem, wave, lane);
+    }
+    if constexpr (kOut == kOutPacked) {
+      // the tile's cells, then its mark: the host takes a tile's cells once
+      // it sees the mark, while later tiles are still on their way
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+      if (lane == 0) {
+        __hip_atomic_store(a.marks + (tile - a.k_tile_begin[ki]), a.mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
   }
   if (bufs.stamps != nullptr && lane == 0) bufs.stamps[2 * static_cast<uint64_t>(wave_id) + 1] = __builtin_amdgcn_s_memrealtime();
 }
 
-template <bool kNonTemporal, bool kMask>
+template <bool kNonTemporal, int kOut>
 __device__ __forceinline__ void KoptBody(const KoptLaunch& a, const KoptPointers& bufs, char* smem) {
   if (blockIdx.x < a.k_block_first[1]) {
-    TileLoop<3, kNonTemporal, kMask>(a, bufs, smem);
+    TileLoop<3, kNonTemporal, kOut>(a, bufs, smem);
   } else if (blockIdx.x < a.k_block_first[2]) {
-    TileLoop<4, kNonTemporal, kMask>(a, bufs, smem);
+    TileLoop<4, kNonTemporal, kOut>(a, bufs, smem);
   } else {
-    TileLoop<5, kNonTemporal, kMask>(a, bufs, smem);
+    TileLoop<5, kNonTemporal, kOut>(a, bufs, smem);
   }
 }
 
 // The launch arguments by value, in the kernel argument segment.
-template <bool kNonTemporal, bool kMask>
+template <bool kNonTemporal, int kOut>
 __global__ void __launch_bounds__(256) KoptKernel(KoptLaunch a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const KoptPointers bufs{a.xy, a.tiles, a.tasks, a.plans, a.costs, a.masks, nullptr};
-  KoptBody<kNonTemporal, kMask>(a, bufs, smem);
+  const KoptPointers bufs{a.xy, a.tiles, a.tasks, a.plans, a.costs, a.masks, a.packed_lo, a.packed_hi, nullptr};
+  KoptBody<kNonTemporal, kOut>(a, bufs, smem);
 }
 
 // The launch arguments in ordinary device memory, for callers that launch
@@ -596,10 +636,10 @@ __global__ void __launch_bounds__(256) KoptKernel(KoptLaunch a) {
 // served from the caches after the first wavefront.  The buffer pointers
 // still come as arguments (one batch of independent reads), so the compiler
 // knows them as global memory.
-template <bool kNonTemporal, bool kMask>
+template <bool kNonTemporal, int kOut>
 __global__ void __launch_bounds__(256) KoptKernelResident(const KoptLaunch* __restrict__ ap, KoptPointers bufs) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  KoptBody<kNonTemporal, kMask>(*ap, bufs, smem);
+  KoptBody<kNonTemporal, kOut>(*ap, bufs, smem);
 }
 
 // ------------------------------------------------------------ work queue
@@ -777,11 +817,11 @@ __device__ __forceinline__ void QueueTile(const KoptLaunch& a, const KoptPointer
   d.distance_type = e.distance_type;
   d.near = e.near;
   if (d.near != 0) {
-    StagePorts<K, true, false, true>(a, bufs, L, d, wave, lane, e.node_count);
-    TileCells<K, true, false, false>(a, bufs, L, d, smem, wave, lane);
+    StagePorts<K, true, kOutCells, true>(a, bufs, L, d, wave, lane, e.node_count);
+    TileCells<K, true, false, kOutCells>(a, bufs, L, d, smem, wave, lane);
   } else {
-    StagePorts<K, false, false, true>(a, bufs, L, d, wave, lane, e.node_count);
-    TileCells<K, false, false, false>(a, bufs, L, d, smem, wave, lane);
+    StagePorts<K, false, kOutCells, true>(a, bufs, L, d, wave, lane, e.node_count);
+    TileCells<K, false, false, kOutCells>(a, bufs, L, d, smem, wave, lane);
   }
 }
 
@@ -847,7 +887,7 @@ __global__ void __launch_bounds__(kWave) KoptQueueKernel(KoptLaunch a, KoptQueue
     for (uint32_t t = lane; t < L.P; t += kWave) s_pq[t] = a.plans[i].pair_pq[t];
   }
   __syncthreads();
-  const KoptPointers bufs{a.xy, nullptr, a.tasks, a.plans, a.costs, nullptr, nullptr};
+  const KoptPointers bufs{a.xy, nullptr, a.tasks, a.plans, a.costs, nullptr, nullptr, nullptr, nullptr};
   char* const wave = smem + a.wave_base;
   // a poller that never ran ends nothing: every wait also ends on the launch's own clock
   const uint64_t limit = 2 * q.life_ticks + q.idle_ticks;
@@ -1117,11 +1157,13 @@ void LaunchKopt(const KoptLaunch& args, const KoptTuning& tuning, size_t shared_
   if (grid == 0) return;
   const dim3 g(grid), b(tuning.block);
   if (a.masks != nullptr) {
-    hipLaunchKernelGGL((KoptKernel<false, true>), g, b, shared_bytes, stream, a);
+    hipLaunchKernelGGL((KoptKernel<false, kOutMasks>), g, b, shared_bytes, stream, a);
+  } else if (a.packed_lo != nullptr) {
+    hipLaunchKernelGGL((KoptKernel<false, kOutPacked>), g, b, shared_bytes, stream, a);
   } else if (tuning.non_temporal) {
-    hipLaunchKernelGGL((KoptKernel<true, false>), g, b, shared_bytes, stream, a);
+    hipLaunchKernelGGL((KoptKernel<true, kOutCells>), g, b, shared_bytes, stream, a);
   } else {
-    hipLaunchKernelGGL((KoptKernel<false, false>), g, b, shared_bytes, stream, a);
+    hipLaunchKernelGGL((KoptKernel<false, kOutCells>), g, b, shared_bytes, stream, a);
   }
   CheckHip(hipGetLastError(), "k-opt kernel launch");
 }
@@ -1133,13 +1175,13 @@ void LaunchKoptResident(const KoptLaunch& finalized, const KoptLaunch* device_ar
   if (device_args == nullptr) throw std::invalid_argument("resident k-opt arguments are NULL");
   const dim3 gd(grid), b(tuning.block);
   const KoptPointers ptrs{finalized.xy, finalized.tiles, finalized.tasks, finalized.plans, finalized.costs,
-                          finalized.masks, stamps};
+                          finalized.masks, nullptr, nullptr, stamps};
   if (finalized.masks != nullptr) {
-    hipLaunchKernelGGL((KoptKernelResident<false, true>), gd, b, shared_bytes, stream, device_args, ptrs);
+    hipLaunchKernelGGL((KoptKernelResident<false, kOutMasks>), gd, b, shared_bytes, stream, device_args, ptrs);
   } else if (tuning.non_temporal) {
-    hipLaunchKernelGGL((KoptKernelResident<true, false>), gd, b, shared_bytes, stream, device_args, ptrs);
+    hipLaunchKernelGGL((KoptKernelResident<true, kOutCells>), gd, b, shared_bytes, stream, device_args, ptrs);
   } else {
-    hipLaunchKernelGGL((KoptKernelResident<false, false>), gd, b, shared_bytes, stream, device_args, ptrs);
+    hipLaunchKernelGGL((KoptKernelResident<false, kOutCells>), gd, b, shared_bytes, stream, device_args, ptrs);
   }
   CheckHip(hipGetLastError(), "k-opt kernel launch");
 }

@@ -200,6 +200,42 @@ struct KoptCache {
   DeviceArray<ee_kopt_task> d_tasks;
   DeviceArray<int64_t> d_costs;
   DeviceArray<KoptTile> d_tiles;
+  // largest evaluation through the ring so far, grown as the buffers are
+  size_t task_room = 0, cell_room = 0;
+  bool Reserve(size_t tasks, size_t cells);
+};
+
+// Page-locked host memory that kernels read and write in place, in up to
+// kSlots slots: while one is on the device the host fills or empties
+// another.  One per context, used by its thread between synchronisations.
+//
+// A kernel marks each tile's output with the launch's mark, a number no
+// earlier launch used, once the output is in host memory.  The marks have an
+// area of their own, so that a word there is never anything but a mark.
+class DirectIo {
+ public:
+  static constexpr size_t kSlots = 3;
+  static constexpr size_t kSlotTiles = 4096;
+  // reserved when the context is made: replacing page-locked memory costs a
+  // first call 0.4 ms, and most calls fit this
+  static constexpr size_t kFirstBytes = size_t{1} << 20;
+  // At least `bytes`; growing discards the contents (no kernel may be using them).
+  void Reserve(size_t bytes);
+  char* host() { return mem_.get(); }
+  char* device() { return device_; }
+  uint64_t* device_marks(size_t slot) { return device_marks_ + slot * kSlotTiles; }
+  uint64_t bytes() const { return mem_.count() + marks_.count() * sizeof(uint64_t); }
+  uint64_t NextMark() { return ++mark_; }
+  // Returns once tile `tile` of the slot's launch, on `stream`, carries
+  // `mark`; throws if the stream has ended without it.  Any host thread.
+  void WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t stream) const;
+
+ private:
+  Pinned<char> mem_;
+  Pinned<uint64_t> marks_;
+  char* device_ = nullptr;
+  uint64_t* device_marks_ = nullptr;
+  uint64_t mark_ = 0;
 };
 
 // Device copy of one tour context for the deletion-set producer, kept while
@@ -258,6 +294,7 @@ struct Context {
   KoptCache kopt;
   KoptCursorCache cursor;
   HtCache ht;
+  DirectIo io;
   // DownloadToCaller's two page-locked chunks and their events, made on
   // first use
   Pinned<char> stage[2];

@@ -91,6 +91,7 @@ Context::Context(int requested) {
   CheckHip(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
   CheckHip(hipEventCreate(&ev_begin), "hipEventCreate");
   CheckHip(hipEventCreate(&ev_end), "hipEventCreate");
+  io.Reserve(0);  // the first calls find their ring
   hipDeviceProp_t prop{};
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
     compute_units = prop.multiProcessorCount;
@@ -341,66 +342,95 @@ void FindJvCandidates(Context& ctx, const ee_graph_view& g, int32_t* witnesses, 
 }
 
 // ------------------------------------------------------------------- k-opt
-uint64_t KoptResidentBytes(const KoptCache& c) {
+// Device memory of the caches and the page-locked ring the kernels work in.
+uint64_t KoptResidentBytes(const Context& ctx) {
+  const KoptCache& c = ctx.kopt;
   return c.d_xy.bytes() + c.d_plans.bytes() + c.d_tasks.bytes() + c.d_costs.bytes() +
-         c.d_tiles.bytes();
+         c.d_tiles.bytes() + ctx.io.bytes();
+}
+
+// Whether an evaluation of this size found room, with the growth rule of the
+// other caches (the rows and cells themselves pass through the bounded ring).
+bool KoptCache::Reserve(size_t tasks, size_t cells) {
+  const bool hit = task_room >= tasks && cell_room >= cells;
+  task_room = Grow(task_room, tasks);
+  cell_room = Grow(cell_room, cells);
+  return hit;
+}
+
+void DirectIo::Reserve(size_t bytes) {
+  const auto device_of = [](void* host) {
+    void* d = nullptr;
+    CheckHip(hipHostGetDevicePointer(&d, host, 0), "hipHostGetDevicePointer");
+    return d;
+  };
+  if (marks_.count() == 0) {
+    marks_.Reserve(kSlots * kSlotTiles);
+    device_marks_ = static_cast<uint64_t*>(device_of(marks_.get()));
+  }
+  const size_t want = Grow(mem_.count(), std::max<size_t>(bytes, kFirstBytes));
+  if (want <= mem_.count()) return;
+  mem_.Reserve(want);
+  device_ = static_cast<char*>(device_of(mem_.get()));
+}
+
+void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t stream) const {
+  const uint64_t* at = marks_.get() + slot * kSlotTiles + tile;
+  const auto seen = [&] { return __atomic_load_n(at, __ATOMIC_ACQUIRE) == mark; };
+  for (uint64_t polls = 1; !seen(); ++polls) {
+    // a kernel that ended, or failed, without the mark: look now and then
+    if (polls % (uint64_t{1} << 20) != 0) continue;
+    const hipError_t status = hipStreamQuery(stream);
+    if (status == hipErrorNotReady || seen()) continue;
+    CheckHip(status, "k-opt kernel");
+    throw std::runtime_error("k-opt kernel ended without marking a tile");
+  }
 }
 
 uint32_t TileRows(const KoptTuning& tuning, uint32_t k) { return tuning.rows_per_tile[k - 3]; }
 
-void EvalKoptCosts(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
-                   uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
-                   uint64_t generator_hash, const ee_kopt_task* tasks, size_t task_count,
-                   int64_t* costs, ee_kopt_usage* usage) {
-  ctx.Activate();
-  if (task_count == 0) {
-    if (usage) *usage = ee_kopt_usage{};
-    return;
-  }
-  if (tasks == nullptr || costs == nullptr) throw std::invalid_argument("HIP k-opt NULL buffer");
-  ValidateTasks(n, k, tasks, task_count);
-  const KoptTaskSource upload = [&](ee_kopt_task* d_tasks) {
-    CheckHip(hipMemcpyAsync(d_tasks, tasks, task_count * sizeof(ee_kopt_task), hipMemcpyHostToDevice,
-                            ctx.stream),
-             "hipMemcpyAsync tasks");
-  };
-  EvalKoptCostsFrom(ctx, x, y, n, type, k, templates, template_count, generator_hash, task_count,
-                    upload, true, costs, nullptr, usage);
+namespace {
+
+// Which caches held what an evaluation needs.
+struct KoptHits {
+  bool snapshot, templates;
+};
+
+bool SnapshotMatches(const KoptCache& c, const int64_t* x, const int64_t* y, int32_t n, uint8_t type) {
+  const size_t nn = static_cast<size_t>(n);
+  return c.snapshot_valid && c.dimension == n && c.distance_type == type && c.x.size() == nn &&
+         std::memcmp(c.x.data(), x, nn * 8) == 0 && std::memcmp(c.y.data(), y, nn * 8) == 0;
 }
 
-void EvalKoptCostsFrom(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
-                       uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
-                       uint64_t generator_hash, size_t task_count, const KoptTaskSource& fill_tasks,
-                       bool sync_after_fill, int64_t* costs, uint32_t* masks, ee_kopt_usage* usage) {
-  ee_kopt_usage u{};
-  ctx.Activate();
-  if (task_count == 0) {
-    if (usage) *usage = u;
-    return;
-  }
+bool TemplatesMatch(const KoptCache& c, uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
+                    uint64_t generator_hash) {
+  const KoptCache::TemplateEntry& entry = c.templates[k - 3];
+  return entry.valid && entry.hash == generator_hash && entry.table.size() == template_count &&
+         std::memcmp(entry.table.data(), templates, template_count * sizeof(ee_endpoint_matching)) == 0;
+}
+
+void CheckKoptInputs(const int64_t* x, const int64_t* y, int32_t n, uint8_t type, uint32_t k,
+                     const ee_endpoint_matching* templates, uint32_t template_count, size_t task_count) {
   if (k < 3 || k > 5 || templates == nullptr || template_count == 0) {
     throw std::invalid_argument("HIP k-opt reconnect table is invalid");
   }
   if (x == nullptr || y == nullptr || n <= 0 || (type != EE_EUC_2D && type != EE_CEIL_2D)) {
     throw std::invalid_argument("HIP k-opt coordinates are invalid");
   }
-  if ((costs == nullptr) == (masks == nullptr)) {
-    throw std::invalid_argument("HIP k-opt needs exactly one of costs and masks");
-  }
   if (task_count > SIZE_MAX / template_count) throw std::overflow_error("k-opt cell count overflows");
-  const size_t cells = task_count * template_count;
-  const uint32_t mask_words = (template_count + 31) / 32;
-  KoptCache& c = ctx.kopt;
+}
 
-  // snapshot
-  const size_t nn = static_cast<size_t>(n);
-  const bool snapshot_hit = c.snapshot_valid && c.dimension == n && c.distance_type == type &&
-                            c.x.size() == nn && std::memcmp(c.x.data(), x, nn * 8) == 0 &&
-                            std::memcmp(c.y.data(), y, nn * 8) == 0;
-  if (!snapshot_hit) {
+KoptHits PrepareKoptCaches(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type, uint32_t k,
+                           const ee_endpoint_matching* templates, uint32_t template_count,
+                           uint64_t generator_hash) {
+  KoptCache& c = ctx.kopt;
+  KoptHits hits{};
+  hits.snapshot = SnapshotMatches(c, x, y, n, type);
+  if (!hits.snapshot) {
     if (!DistanceSafe(x, y, n)) {
       throw std::invalid_argument("k-opt cost needs distance-safe integer coordinates");
     }
+    const size_t nn = static_cast<size_t>(n);
     const std::vector<longlong2> xy = Interleave(x, y, n);
     DeviceArray<longlong2> d_xy(nn, ctx.device);
     d_xy.Upload(xy.data(), nn, ctx.stream);
@@ -413,22 +443,250 @@ void EvalKoptCostsFrom(Context& ctx, const int64_t* x, const int64_t* y, int32_t
     c.near = NearExtent(x, y, n);
     c.snapshot_valid = true;
   }
-
-  // templates (one plan slot per k)
-  KoptCache::TemplateEntry& entry = c.templates[k - 3];
-  const bool template_hit =
-      entry.valid && entry.hash == generator_hash && entry.table.size() == template_count &&
-      std::memcmp(entry.table.data(), templates, template_count * sizeof(ee_endpoint_matching)) == 0;
-  if (!template_hit) {
+  // one plan slot per k
+  hits.templates = TemplatesMatch(c, k, templates, template_count, generator_hash);
+  if (!hits.templates) {
     const KoptPlan plan = BuildPlan(k, templates, template_count);
     if (c.d_plans.count() < 3) c.d_plans.Allocate(3, ctx.device);
     c.host_plans[k - 3] = plan;
     c.d_plans.UploadAt(k - 3, &c.host_plans[k - 3], 1, ctx.stream);
     ctx.Sync();
+    KoptCache::TemplateEntry& entry = c.templates[k - 3];
     entry.table.assign(templates, templates + template_count);
     entry.hash = generator_hash;
     entry.valid = true;
   }
+  return hits;
+}
+
+// The rows of one evaluation, cut into launches that pass through the
+// context's page-locked ring: per launch its task rows, and the cells in
+// transfer form (low words, then high bytes on instances that are not near).
+struct KoptChunks {
+  static constexpr size_t kSlotBytes = size_t{4} << 20;
+
+  KoptChunks(size_t rows, size_t templates, uint32_t tile_rows, bool wide) : rows_(rows) {
+    const size_t per_row = sizeof(ee_kopt_task) + templates * (wide ? 5 : 4);
+    const size_t fit = std::min<size_t>(std::max<size_t>(kSlotBytes / per_row / tile_rows, 1), DirectIo::kSlotTiles);
+    count = (rows + fit * tile_rows - 1) / (fit * tile_rows);
+    // launches of equal size, whole tiles each
+    const size_t even = (rows + count - 1) / count;
+    chunk_rows = std::min(rows, (even + tile_rows - 1) / tile_rows * tile_rows);
+    count = (rows + chunk_rows - 1) / chunk_rows;
+    lo_off = Align256(chunk_rows * sizeof(ee_kopt_task));
+    hi_off = lo_off + Align256(chunk_rows * templates * 4);
+    slot_bytes = hi_off + (wide ? Align256(chunk_rows * templates) : 0);
+    slots = std::min<size_t>(count, DirectIo::kSlots);
+  }
+  static size_t Align256(size_t v) { return (v + 255) & ~size_t{255}; }
+  size_t First(size_t chunk) const { return chunk * chunk_rows; }
+  size_t Rows(size_t chunk) const { return std::min(chunk_rows, rows_ - First(chunk)); }
+
+  size_t count = 0, chunk_rows = 0, slots = 0;
+  size_t lo_off = 0, hi_off = 0, slot_bytes = 0;
+
+ private:
+  size_t rows_;
+};
+
+// body(first, end) over [0, n), in four parts on host threads from
+// `serial_below` up.
+template <typename F> void InParts(size_t n, size_t serial_below, F&& body) {
+  constexpr size_t kParts = 4;
+  if (n < serial_below) {
+    body(size_t{0}, n);
+    return;
+  }
+  ParallelFor(kParts, [&](size_t p) { body(n * p / kParts, n * (p + 1) / kParts); }, static_cast<unsigned>(kParts));
+}
+
+// Whether the caches look up to date, from their sizes and a sample of the
+// coordinates.
+bool LooksResident(const KoptCache& c, const int64_t* x, const int64_t* y, int32_t n, uint8_t type, uint32_t k,
+                   const ee_endpoint_matching* templates, uint32_t template_count, uint64_t generator_hash) {
+  if (!c.snapshot_valid || c.dimension != n || c.distance_type != type ||
+      !TemplatesMatch(c, k, templates, template_count, generator_hash)) {
+    return false;
+  }
+  const size_t sample = std::min<size_t>(static_cast<size_t>(n), 64) * sizeof(int64_t);
+  return std::memcmp(c.x.data(), x, sample) == 0 && std::memcmp(c.y.data(), y, sample) == 0;
+}
+
+// Cells expanded on host threads: groups of kGroupCells on kExpandThreads
+// threads from kSerialCells up (below, waking them costs more than it saves).
+constexpr size_t kGroupCells = 16384, kSerialCells = 65536;
+constexpr unsigned kExpandThreads = 8;
+
+// Tiles of the launches that write to host memory.  PCIe bounds them, so few
+// wavefronts with several small tiles each: 192 keep the link busy and their
+// first tiles arrive early, so the host expands while the rest crosses.  A
+// k = 5 block of 4,096 rows takes 120 us (rows 4, 192 wavefronts), 126 with
+// 256 and 158 with one tile per wavefront, whose tiles all end together;
+// k = 3 and 4, with less output per row, measured best at 256.
+KoptTuning DirectTuning(uint32_t k) {
+  KoptTuning t;
+  t.rows_per_tile[0] = 64;
+  t.rows_per_tile[1] = 16;
+  t.rows_per_tile[2] = 4;
+  t.block = 64;
+  t.grid = k == 5 ? 192 : 256;
+  return t;
+}
+
+// The kernel reads the task rows from page-locked host memory and writes the
+// cells back there in transfer form, tile by tile, so a call has no copy
+// command and no wait for the stream, and half the bytes of int64 cells
+// cross PCIe (56 GB/s here, which bounds a block: 61 us for 4,096 k = 5
+// rows).  Host threads expand tiles into the caller's buffer as their marks
+// arrive.  Against an upload, a launch and a download with a wait each: one
+// k = 5 row 56 -> 19 us, 1,237 k = 4 rows 63 -> 32 us, 4,096 k = 5 rows
+// 293 -> 121 us, 1,501 wide k = 5 rows 163 -> 83 us.
+// `check` runs on the host while the first launches are on the device; false
+// drops their output and returns false, with nothing delivered.
+bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t template_count,
+               const ee_kopt_task* tasks, size_t task_count, int64_t* costs, const std::function<bool()>& check,
+               ee_kopt_usage* usage) {
+  ee_kopt_usage u{};
+  KoptCache& c = ctx.kopt;
+  const KoptTuning tuning = DirectTuning(k);
+  const uint32_t tile_rows = tuning.rows_per_tile[k - 3];
+  const KoptChunks chunks(task_count, template_count, tile_rows, !c.near);
+  DirectIo& io = ctx.io;
+  io.Reserve(chunks.slots * chunks.slot_bytes);
+
+  KoptInstance inst{};
+  inst.n = static_cast<uint32_t>(n);
+  inst.distance_type = type;
+  inst.near = c.near ? 1 : 0;
+  bool present[3] = {false, false, false};
+  present[k - 3] = true;
+  uint64_t marks[DirectIo::kSlots] = {};
+  const auto slot_of = [&](size_t chunk) { return chunk % chunks.slots * chunks.slot_bytes; };
+  const auto launch = [&](size_t chunk) {
+    const size_t rows = chunks.Rows(chunk), slot = chunk % chunks.slots, at = slot_of(chunk);
+    const ee_kopt_task* from = tasks + chunks.First(chunk);
+    ee_kopt_task* staged = reinterpret_cast<ee_kopt_task*>(io.host() + at);
+    InParts(rows, 8192, [&](size_t b, size_t e) { std::memcpy(staged + b, from + b, (e - b) * sizeof(*from)); });
+    KoptSegment segment{0, k, 0, rows, 0, 0, tile_rows, 0};
+    KoptLaunch a{};
+    KoptAssignTiles(&segment, 1, &inst, c.host_plans.data(), tuning, nullptr, &a);
+    if (a.inline_count == 0) throw std::logic_error("a one-segment k-opt launch needs its inline table");
+    a.xy = c.d_xy.get();
+    a.tasks = reinterpret_cast<const ee_kopt_task*>(io.device() + at);
+    a.plans = c.d_plans.get();
+    a.packed_lo = reinterpret_cast<uint32_t*>(io.device() + at + chunks.lo_off);
+    a.packed_hi = c.near ? nullptr : reinterpret_cast<uint8_t*>(io.device() + at + chunks.hi_off);
+    a.marks = io.device_marks(slot);
+    a.mark = marks[slot] = io.NextMark();
+    a.bound_nodes = static_cast<uint32_t>(n);
+    const size_t shared = KoptPrepareLayout(&a, c.host_plans.data(), present, tuning, c.near);
+    LaunchKopt(a, tuning, shared, ctx.stream);
+  };
+  try {
+    auto t0 = std::chrono::steady_clock::now();
+    for (size_t i = 0; i < chunks.slots; ++i) launch(i);
+    u.h2d_ms = MsSince(t0);
+    t0 = std::chrono::steady_clock::now();
+    if (!check()) {
+      ctx.Sync();
+      return false;
+    }
+    for (size_t i = 0; i < chunks.count; ++i) {
+      const size_t slot = i % chunks.slots, rows = chunks.Rows(i);
+      const size_t tiles = (rows + tile_rows - 1) / tile_rows;
+      io.WaitTile(slot, 0, marks[slot], ctx.stream);
+      if (i == 0) {
+        u.kernel_ms = MsSince(t0);
+        t0 = std::chrono::steady_clock::now();
+      }
+      const char* from = io.host() + slot_of(i);
+      const uint32_t* lo = reinterpret_cast<const uint32_t*>(from + chunks.lo_off);
+      const uint8_t* hi = c.near ? nullptr : reinterpret_cast<const uint8_t*>(from + chunks.hi_off);
+      int64_t* to = costs + chunks.First(i) * template_count;
+      // groups of tiles, taken in order by the host threads as they arrive
+      const size_t group = std::max<size_t>(1, kGroupCells / (tile_rows * template_count));
+      const auto expand = [&](size_t g) {
+        const size_t t0 = g * group, t1 = std::min(tiles, t0 + group);
+        for (size_t t = t0; t < t1; ++t) io.WaitTile(slot, t, marks[slot], ctx.stream);
+        const size_t b = t0 * tile_rows * template_count;
+        const size_t e = std::min(rows, t1 * tile_rows) * template_count;
+        ExpandCells(lo + b, hi != nullptr ? hi + b : nullptr, e - b, to + b);
+      };
+      ParallelFor((tiles + group - 1) / group, expand, rows * template_count < kSerialCells ? 1 : kExpandThreads);
+      if (i + chunks.slots < chunks.count) launch(i + chunks.slots);
+    }
+    u.d2h_ms = MsSince(t0);
+  } catch (...) {
+    static_cast<void>(hipStreamSynchronize(ctx.stream));  // the ring is free again
+    throw;
+  }
+  u.snapshot_hit = u.template_hit = 1;
+  u.workspace_hit = c.Reserve(task_count, task_count * template_count) ? 1 : 0;
+  u.resident_bytes = KoptResidentBytes(ctx);
+  if (usage) *usage = u;
+  return true;
+}
+
+}  // namespace
+
+void EvalKoptCosts(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
+                   uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
+                   uint64_t generator_hash, const ee_kopt_task* tasks, size_t task_count,
+                   int64_t* costs, ee_kopt_usage* usage) {
+  ctx.Activate();
+  if (task_count == 0) {
+    if (usage) *usage = ee_kopt_usage{};
+    return;
+  }
+  if (tasks == nullptr || costs == nullptr) throw std::invalid_argument("HIP k-opt NULL buffer");
+  KoptCache& c = ctx.kopt;
+  // Where the caches look up to date, the launch goes out first, and the
+  // full comparison with them and the check of the rows run beside it: the
+  // kernel clamps node ids to the cached snapshot, and nothing reaches the
+  // caller before both passed.  Otherwise rows and caches come first.
+  const bool inputs = k >= 3 && k <= 5 && templates != nullptr && template_count > 0 && x != nullptr &&
+                      y != nullptr && n > 0 && task_count <= SIZE_MAX / template_count;
+  if (inputs && LooksResident(c, x, y, n, type, k, templates, template_count, generator_hash)) {
+    const auto check = [&] {
+      if (!SnapshotMatches(c, x, y, n, type)) return false;
+      try {
+        InParts(task_count, 1024, [&](size_t b, size_t e) { ValidateTasks(n, k, tasks + b, e - b); });
+      } catch (const std::invalid_argument&) {
+        ValidateTasks(n, k, tasks, task_count);  // the first refused row's message
+        throw;
+      }
+      return true;
+    };
+    if (RunDirect(ctx, n, type, k, template_count, tasks, task_count, costs, check, usage)) return;
+  }
+  ValidateTasks(n, k, tasks, task_count);
+  CheckKoptInputs(x, y, n, type, k, templates, template_count, task_count);
+  const KoptHits hits = PrepareKoptCaches(ctx, x, y, n, type, k, templates, template_count, generator_hash);
+  RunDirect(ctx, n, type, k, template_count, tasks, task_count, costs, [] { return true; }, usage);
+  if (usage) {
+    usage->snapshot_hit = hits.snapshot ? 1 : 0;
+    usage->template_hit = hits.templates ? 1 : 0;
+  }
+}
+
+void EvalKoptCostsFrom(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
+                       uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
+                       uint64_t generator_hash, size_t task_count, const KoptTaskSource& fill_tasks,
+                       bool sync_after_fill, int64_t* costs, uint32_t* masks, ee_kopt_usage* usage) {
+  ee_kopt_usage u{};
+  ctx.Activate();
+  if (task_count == 0) {
+    if (usage) *usage = u;
+    return;
+  }
+  CheckKoptInputs(x, y, n, type, k, templates, template_count, task_count);
+  if ((costs == nullptr) == (masks == nullptr)) {
+    throw std::invalid_argument("HIP k-opt needs exactly one of costs and masks");
+  }
+  const size_t cells = task_count * template_count;
+  const uint32_t mask_words = (template_count + 31) / 32;
+  KoptCache& c = ctx.kopt;
+  const KoptHits hits = PrepareKoptCaches(ctx, x, y, n, type, k, templates, template_count, generator_hash);
 
   // workspace
   // mask output needs task_count x mask_words words, held in the cost pool
@@ -483,10 +741,10 @@ void EvalKoptCostsFrom(Context& ctx, const int64_t* x, const int64_t* y, int32_t
   }
   ctx.Sync();
   u.d2h_ms = MsSince(t0);
-  u.snapshot_hit = snapshot_hit ? 1 : 0;
-  u.template_hit = template_hit ? 1 : 0;
+  u.snapshot_hit = hits.snapshot ? 1 : 0;
+  u.template_hit = hits.templates ? 1 : 0;
   u.workspace_hit = workspace_hit ? 1 : 0;
-  u.resident_bytes = KoptResidentBytes(c);
+  u.resident_bytes = KoptResidentBytes(ctx);
   if (usage) *usage = u;
 }
 

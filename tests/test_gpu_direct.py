@@ -1,0 +1,96 @@
+"""Leaf-cost calls whose kernel reads rows from and writes cells to host
+memory, at the sizes where their tiles and launches end: one row, one row
+either side of a tile, several launches through the ring's slots, and more
+launches than slots; near and wide coordinates (one and two planes of the
+transfer form).  Whole numbers, so every comparison is exact."""
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import pytest
+
+import _oracle as O
+from cudaedgeelimination_amd import _lib, backend
+from cudaedgeelimination_amd import workloads as W
+from cudaedgeelimination_amd.graph import CEIL_2D, EUC_2D
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def graph(seed, n, dtype, box):
+    rng = np.random.default_rng(seed)
+    return W.knn_graph(rng.integers(0, box, n), rng.integers(0, box, n), dtype, 8)
+
+
+@pytest.mark.parametrize("box", [1_000_000, 1 << 30])
+@pytest.mark.parametrize("k, rows", [(3, 1), (3, 63), (3, 65), (3, 70_000), (4, 15), (4, 17), (4, 2_731),
+                                     (5, 1), (5, 3), (5, 5), (5, 315), (5, 316), (5, 4_799), (5, 20_011)])
+def test_rows_match_oracle(ctx, k, rows, box):
+    say(f"direct k={k} rows={rows} box={box}")
+    dtype = CEIL_2D if rows % 2 else EUC_2D
+    g = graph(rows + k, 700, dtype, box)
+    tasks = W.kopt_tasks(rows, g, np.full(rows, k, np.uint8))
+    table = backend.build_kopt_reconnect_table(k)
+    want, _, _ = O.kopt_costs(g.x, g.y, dtype, k, tasks)
+    for _ in range(2):  # caches empty, then up to date (the launch before the checks)
+        got, _, usage = backend.evaluate_kopt_template_costs_cuda(g, table, tasks, ctx)
+        assert np.array_equal(got, want)
+    assert usage.snapshot_hit and usage.template_hit and usage.workspace_hit
+
+
+@pytest.mark.parametrize("rows", [7, 3_000])
+def test_checks_beside_the_launch(ctx, rows):
+    """A refused row leaves the caller's buffer alone and the next call right;
+    coordinates that differ from the cached ones in one late node are seen."""
+    say(f"direct checks rows={rows}")
+    k = 5
+    g = graph(rows, 900, EUC_2D, 1_000_000)
+    tasks = W.kopt_tasks(rows, g, np.full(rows, k, np.uint8))
+    table = backend.build_kopt_reconnect_table(k)
+    want, _, _ = O.kopt_costs(g.x, g.y, EUC_2D, k, tasks)
+    got, _, _ = backend.evaluate_kopt_template_costs_cuda(g, table, tasks, ctx)
+    assert np.array_equal(got, want)
+    for field, value in (((0, 3), 900), ((0, 3), -5), ((0, 1), None), ((2, 2), None)):
+        bad = tasks.copy()
+        row = bad["port_nodes"][rows - 1]
+        if value is not None:
+            row[field[1]] = value
+        elif field == (0, 1):
+            row[1] = row[0]  # a loop
+        else:
+            row[2], row[3] = row[1], row[0]  # the first deleted edge again
+        out = np.full(rows * 208, -7, np.int64)
+        status = _lib.lib().ee_kopt_eval_costs(
+            ctx.handle, _lib.ptr(g.x), _lib.ptr(g.y), g.dimension, EUC_2D, k, _lib.ptr(table.templates), 208,
+            table.generator_hash, _lib.ptr(bad), rows, _lib.ptr(out), None)
+        assert status == 1 and (out == -7).all()
+        got, _, usage = backend.evaluate_kopt_template_costs_cuda(g, table, tasks, ctx)
+        assert np.array_equal(got, want) and usage.snapshot_hit
+    moved = g.copy()
+    node = int(tasks["port_nodes"][0, 0])
+    moved.x[node] += 1000
+    got, _, usage = backend.evaluate_kopt_template_costs_cuda(moved, table, tasks, ctx)
+    want2, _, _ = O.kopt_costs(moved.x, moved.y, EUC_2D, k, tasks)
+    assert not usage.snapshot_hit and np.array_equal(got, want2) and not np.array_equal(want2, want)
+
+
+def test_wider_tables(ctx):
+    """Tables of other sizes than the canonical ones: one template (many
+    tiles per launch) and all 945 matchings of ten ports (wide rows)."""
+    k = 5
+    g = graph(11, 400, EUC_2D, 1 << 30)
+    canon = backend.build_kopt_reconnect_table(k)
+    tasks = W.kopt_tasks(3, g, np.full(30_000, k, np.uint8))
+    want, _, _ = O.kopt_costs(g.x, g.y, EUC_2D, k, tasks)
+    one = backend.KOptReconnectTable(k, canon.templates[17:18].copy(), 99)
+    got, _, _ = backend.evaluate_kopt_template_costs_cuda(g, one, tasks, ctx)
+    assert np.array_equal(got, want.reshape(-1, 208)[:, 17])
+    wide = backend.KOptReconnectTable(k, np.tile(canon.templates, 5)[:945].copy(), 98)
+    got, _, _ = backend.evaluate_kopt_template_costs_cuda(g, wide, tasks[:2_000], ctx)
+    assert np.array_equal(got.reshape(-1, 945), np.tile(want.reshape(-1, 208)[:2_000], 5)[:, :945])
