@@ -703,7 +703,7 @@ ee_status ee_kopt_batch_download(ee_kopt_batch* batch, uint64_t first_cell, uint
     }
     if (cell_count > 0 && costs == nullptr) throw std::invalid_argument("costs is NULL");
     b.ctx->Activate();
-    ee::DownloadRange(*b.ctx, b.d_costs, first_cell, cell_count, costs);
+    ee::DownloadCells(*b.ctx, b.d_costs.get() + first_cell, cell_count, !b.NearOnly(), costs);
   });
 }
 
@@ -720,12 +720,12 @@ ee_status ee_kopt_batch_download_pool(ee_kopt_batch* batch, uint32_t pool, uint6
     if (cell_count > 0 && costs == nullptr) throw std::invalid_argument("costs is NULL");
     b.ctx->Activate();
     if (pool == 0) {
-      ee::DownloadRange(*b.ctx, b.d_costs, first_cell, cell_count, costs);
+      ee::DownloadCells(*b.ctx, b.d_costs.get() + first_cell, cell_count, !b.NearOnly(), costs);
     } else {
       ee::Batch::PipeLane& l = b.lanes[pool - 1];
       // the lane's launches ran on its own stream; wait for them first
       ee::CheckHip(hipStreamSynchronize(l.stream), "hipStreamSynchronize");
-      ee::DownloadRange(*b.ctx, l.costs, first_cell, cell_count, costs);
+      ee::DownloadCells(*b.ctx, l.costs.get() + first_cell, cell_count, !b.NearOnly(), costs);
     }
   });
 }

@@ -36,8 +36,9 @@ int CountDevices();
 // Page-locked host staging of at least `count` elements (hipHostMalloc);
 // growing discards the contents.  The pages are written once when allocated:
 // the first host access to fresh page-locked memory faults every page in
-// (about 0.4 ms per MB), which would otherwise land on the first run that
-// fills or reads the staging.
+// (about 0.4 ms per MB, and no less on several threads, which wait for one
+// another there), which would otherwise land on the first run that fills or
+// reads the staging.
 template <typename T> class Pinned {
  public:
   Pinned() = default;
@@ -214,11 +215,12 @@ struct KoptCache {
 // area of their own, so that a word there is never anything but a mark.
 class DirectIo {
  public:
-  static constexpr size_t kSlots = 3;
+  static constexpr size_t kSlots = 2;
   static constexpr size_t kSlotTiles = 4096;
-  // reserved when the context is made: replacing page-locked memory costs a
-  // first call 0.4 ms, and most calls fit this
-  static constexpr size_t kFirstBytes = size_t{1} << 20;
+  // The sizes the ring takes: the first when the context is made, which most
+  // calls fit, the next for large results, and what a call asks for beyond.
+  // Few steps, since fresh page-locked memory costs about 0.4 ms per MB.
+  static constexpr size_t kSizes[2] = {size_t{1} << 20, size_t{4} << 20};
   // At least `bytes`; growing discards the contents (no kernel may be using them).
   void Reserve(size_t bytes);
   char* host() { return mem_.get(); }
@@ -229,6 +231,10 @@ class DirectIo {
   // Returns once tile `tile` of the slot's launch, on `stream`, carries
   // `mark`; throws if the stream has ended without it.  Any host thread.
   void WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t stream) const;
+  // Waits for the tiles of a launch that writes `count` cells in transfer
+  // form, tile_cells to a tile, and expands them to int64 as they arrive.
+  void TakeCells(size_t slot, uint64_t mark, hipStream_t stream, const uint32_t* lo, const uint8_t* hi,
+                 size_t count, size_t tile_cells, int64_t* cells) const;
 
  private:
   Pinned<char> mem_;
@@ -307,6 +313,11 @@ struct Context {
 // the other is copied out on host threads.  A copy straight into pageable
 // caller memory is staged by the runtime at about half that rate.
 void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes);
+
+// Device-resident cost cells [0, count) into caller memory, after the work
+// queued before on the context's stream, in transfer form through the
+// context's ring.  wide: some instance's coordinates are not near.
+void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide, int64_t* cells);
 
 // Elements [offset, offset + count) of a device array into caller memory, as
 // DownloadToCaller.

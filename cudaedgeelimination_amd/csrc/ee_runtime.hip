@@ -358,35 +358,6 @@ bool KoptCache::Reserve(size_t tasks, size_t cells) {
   return hit;
 }
 
-void DirectIo::Reserve(size_t bytes) {
-  const auto device_of = [](void* host) {
-    void* d = nullptr;
-    CheckHip(hipHostGetDevicePointer(&d, host, 0), "hipHostGetDevicePointer");
-    return d;
-  };
-  if (marks_.count() == 0) {
-    marks_.Reserve(kSlots * kSlotTiles);
-    device_marks_ = static_cast<uint64_t*>(device_of(marks_.get()));
-  }
-  const size_t want = Grow(mem_.count(), std::max<size_t>(bytes, kFirstBytes));
-  if (want <= mem_.count()) return;
-  mem_.Reserve(want);
-  device_ = static_cast<char*>(device_of(mem_.get()));
-}
-
-void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t stream) const {
-  const uint64_t* at = marks_.get() + slot * kSlotTiles + tile;
-  const auto seen = [&] { return __atomic_load_n(at, __ATOMIC_ACQUIRE) == mark; };
-  for (uint64_t polls = 1; !seen(); ++polls) {
-    // a kernel that ended, or failed, without the mark: look now and then
-    if (polls % (uint64_t{1} << 20) != 0) continue;
-    const hipError_t status = hipStreamQuery(stream);
-    if (status == hipErrorNotReady || seen()) continue;
-    CheckHip(status, "k-opt kernel");
-    throw std::runtime_error("k-opt kernel ended without marking a tile");
-  }
-}
-
 uint32_t TileRows(const KoptTuning& tuning, uint32_t k) { return tuning.rows_per_tile[k - 3]; }
 
 namespace {
@@ -512,11 +483,6 @@ bool LooksResident(const KoptCache& c, const int64_t* x, const int64_t* y, int32
   return std::memcmp(c.x.data(), x, sample) == 0 && std::memcmp(c.y.data(), y, sample) == 0;
 }
 
-// Cells expanded on host threads: groups of kGroupCells on kExpandThreads
-// threads from kSerialCells up (below, waking them costs more than it saves).
-constexpr size_t kGroupCells = 16384, kSerialCells = 65536;
-constexpr unsigned kExpandThreads = 8;
-
 // Tiles of the launches that write to host memory.  PCIe bounds them, so few
 // wavefronts with several small tiles each: 192 keep the link busy and their
 // first tiles arrive early, so the host expands while the rest crosses.  A
@@ -593,26 +559,15 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
     }
     for (size_t i = 0; i < chunks.count; ++i) {
       const size_t slot = i % chunks.slots, rows = chunks.Rows(i);
-      const size_t tiles = (rows + tile_rows - 1) / tile_rows;
       io.WaitTile(slot, 0, marks[slot], ctx.stream);
       if (i == 0) {
         u.kernel_ms = MsSince(t0);
         t0 = std::chrono::steady_clock::now();
       }
       const char* from = io.host() + slot_of(i);
-      const uint32_t* lo = reinterpret_cast<const uint32_t*>(from + chunks.lo_off);
-      const uint8_t* hi = c.near ? nullptr : reinterpret_cast<const uint8_t*>(from + chunks.hi_off);
-      int64_t* to = costs + chunks.First(i) * template_count;
-      // groups of tiles, taken in order by the host threads as they arrive
-      const size_t group = std::max<size_t>(1, kGroupCells / (tile_rows * template_count));
-      const auto expand = [&](size_t g) {
-        const size_t t0 = g * group, t1 = std::min(tiles, t0 + group);
-        for (size_t t = t0; t < t1; ++t) io.WaitTile(slot, t, marks[slot], ctx.stream);
-        const size_t b = t0 * tile_rows * template_count;
-        const size_t e = std::min(rows, t1 * tile_rows) * template_count;
-        ExpandCells(lo + b, hi != nullptr ? hi + b : nullptr, e - b, to + b);
-      };
-      ParallelFor((tiles + group - 1) / group, expand, rows * template_count < kSerialCells ? 1 : kExpandThreads);
+      io.TakeCells(slot, marks[slot], ctx.stream, reinterpret_cast<const uint32_t*>(from + chunks.lo_off),
+                   c.near ? nullptr : reinterpret_cast<const uint8_t*>(from + chunks.hi_off),
+                   rows * template_count, tile_rows * template_count, costs + chunks.First(i) * template_count);
       if (i + chunks.slots < chunks.count) launch(i + chunks.slots);
     }
     u.d2h_ms = MsSince(t0);

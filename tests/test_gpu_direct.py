@@ -14,6 +14,7 @@ import _oracle as O
 from cudaedgeelimination_amd import _lib, backend
 from cudaedgeelimination_amd import workloads as W
 from cudaedgeelimination_amd.graph import CEIL_2D, EUC_2D
+from cudaedgeelimination_amd.resident import KoptBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +95,27 @@ def test_wider_tables(ctx):
     wide = backend.KOptReconnectTable(k, np.tile(canon.templates, 5)[:945].copy(), 98)
     got, _, _ = backend.evaluate_kopt_template_costs_cuda(g, wide, tasks[:2_000], ctx)
     assert np.array_equal(got.reshape(-1, 945), np.tile(want.reshape(-1, 208)[:2_000], 5)[:, :945])
+
+
+@pytest.mark.parametrize("box", [1_000_000, 1 << 30])
+def test_batch_download_ranges(ctx, box):
+    """Resident cells read back in ranges that start and end on, before and
+    after the transfer kernel's tiles (512 cells) and slots (2^19 near cells,
+    419,328 wide ones), at odd offsets, and whole."""
+    say(f"batch download box={box}")
+    k, rows = 5, 5_300  # 1,102,400 cells: three slots near or wide
+    far = graph(5, 300, CEIL_2D, box)
+    near = graph(6, 500, EUC_2D, 1_000_000)
+    tasks = [W.kopt_tasks(7, far, np.full(rows, k, np.uint8)), W.kopt_tasks(8, near, np.full(40, 3, np.uint8))]
+    want, _, _ = O.kopt_costs(far.x, far.y, CEIL_2D, k, tasks[0])
+    small, _, _ = O.kopt_costs(near.x, near.y, EUC_2D, 3, tasks[1])
+    batch = KoptBatch(ctx)
+    a, b = batch.add_instance(far), batch.add_instance(near)
+    batch.set_work([(a, k, rows), (b, 3, 40)], np.concatenate(tasks))
+    batch.run()
+    assert np.array_equal(batch.segment_costs(1), small)
+    slot = 1 << 19 if box == 1_000_000 else 419_328
+    for first, count in ((0, len(want)), (0, 1), (1, 511), (3, 512), (511, 513), (7, 65_536), (0, slot),
+                         (5, slot + 1), (1, 2 * slot - 1), (9, 2 * slot + 3), (len(want) - 1, 1), (4, 0)):
+        assert np.array_equal(batch.download(first, count), want[first:first + count]), (first, count)
+    batch.close()
