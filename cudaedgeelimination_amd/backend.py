@@ -342,13 +342,13 @@ def evaluate_kopt_cursor_cuda(graph: GraphSnapshot | None, table: KOptReconnectT
     total = kopt_cursor_count(tour, k)
     rows = max(0, min(count, total - first))
     T = len(table.templates) if table is not None else 0
-    tasks = np.zeros(max(rows, 1), dtype=_lib.KOPT_TASK_DTYPE)
-    positions = np.zeros((max(rows, 1), k), dtype=np.uint32)
+    tasks = np.empty(max(rows, 1), dtype=_lib.KOPT_TASK_DTYPE)
+    positions = np.empty((max(rows, 1), k), dtype=np.uint32)
     costs = masks = None
     if output == "costs":
         costs = np.empty(max(rows * T, 1), dtype=np.int64)
     elif output == "masks":
-        masks = np.zeros((max(rows, 1), (T + 31) // 32), dtype=np.uint32)
+        masks = np.empty((max(rows, 1), (T + 31) // 32), dtype=np.uint32)
     elif output is not None:
         raise ValueError("output must be 'costs', 'masks' or None")
     templates = (np.ascontiguousarray(table.templates, dtype=_lib.MATCHING_DTYPE)

@@ -8,10 +8,10 @@
 // (kopt_search.cpp:736-752), BuildKOptCostTask (kopt_search.cpp:561-584).
 #include <algorithm>
 #include <cstring>
-#include <limits>
 #include <stdexcept>
 #include <vector>
 
+#include "ee_cursor_body.h"
 #include "ee_runtime.h"
 
 namespace ee {
@@ -22,21 +22,6 @@ namespace {
 constexpr uint32_t kMaxSelectable = 65536;
 constexpr uint32_t kCursorBlock = 256;
 
-// C(n, j) for j in 1..4 and n < 2^16, exact in 64 bits.
-__host__ __device__ inline uint64_t Binom(uint64_t n, uint32_t j) {
-  if (n < j) return 0;
-  switch (j) {
-    case 1:
-      return n;
-    case 2:
-      return n * (n - 1) / 2;
-    case 3:
-      return n * (n - 1) / 2 * (n - 2) / 3;
-    default:
-      return (n * (n - 1) / 2) * ((n - 2) * (n - 3) / 2) / 6;
-  }
-}
-
 // Sets the reference cursor enumerates for one k: AdvanceCombination never
 // moves index 0, so a set is selectable[0] plus k - 1 of the other
 // `labels` = |selectable| - 1 positions, in lexicographic order of their
@@ -46,63 +31,19 @@ uint64_t SetCount(uint32_t selectable_count, uint32_t k) {
   return Binom(selectable_count - 1, k - 1);
 }
 
-// One thread per set.  Set `first + i` is unranked in the combinatorial
-// number system: the index of slot s is the largest v whose preceding
-// choices (indices prev+1 .. v-1, each followed by C(labels - u, rem)
-// completions) number at most the remaining rank; by the hockey-stick
-// identity those number C(labels - prev, rem + 1) - C(labels - v + 1, rem + 1).
-// The positions are sorted (tour order) and turned into ports and the summed
-// deleted cost as BuildKOptCostTask does.
-__global__ __launch_bounds__(kCursorBlock) void KoptCursorKernel(
-    const int32_t* __restrict__ tour, const int64_t* __restrict__ edge_costs,
-    const uint64_t* __restrict__ selectable, uint32_t tour_length, uint32_t labels, uint32_t k,
-    uint64_t first, uint32_t count, ee_kopt_task* __restrict__ tasks,
-    uint32_t* __restrict__ positions, uint32_t* __restrict__ status) {
+// One thread per set.
+__global__ __launch_bounds__(kCursorBlock) void KoptCursorKernel(KoptCursor cursor, uint32_t k, uint64_t first,
+                                                                 uint32_t count, ee_kopt_task* __restrict__ tasks,
+                                                                 uint32_t* __restrict__ positions,
+                                                                 uint32_t* __restrict__ status) {
   const uint32_t i = blockIdx.x * kCursorBlock + threadIdx.x;
   if (i >= count) return;
-  uint64_t rank = first + i;
   uint64_t pos[kMaxK];
-  pos[0] = selectable[0];
-  uint32_t prev = 0;
-  for (uint32_t s = 1; s < k; ++s) {
-    const uint32_t rem = k - 1 - s;
-    const uint64_t total = Binom(labels - prev, rem + 1);
-    uint32_t lo = prev + 1, hi = labels - rem;
-    while (lo < hi) {
-      const uint32_t mid = lo + (hi - lo + 1) / 2;
-      if (total - Binom(labels - mid + 1, rem + 1) <= rank) {
-        lo = mid;
-      } else {
-        hi = mid - 1;
-      }
-    }
-    rank -= total - Binom(labels - lo + 1, rem + 1);
-    prev = lo;
-    pos[s] = selectable[lo];
-  }
-  for (uint32_t s = 1; s < k; ++s) {  // insertion sort, k <= 5
-    const uint64_t v = pos[s];
-    uint32_t t = s;
-    while (t > 0 && pos[t - 1] > v) {
-      pos[t] = pos[t - 1];
-      --t;
-    }
-    pos[t] = v;
-  }
   ee_kopt_task task{};
-  uint64_t sum = 0;
-  bool overflow = false;
-  for (uint32_t e = 0; e < k; ++e) {
-    const uint64_t p = pos[e];
-    const uint64_t next = p + 1 == tour_length ? 0 : p + 1;
-    task.port_nodes[2 * e] = tour[p];
-    task.port_nodes[2 * e + 1] = tour[next];
-    overflow |= __builtin_add_overflow(sum, static_cast<uint64_t>(edge_costs[p]), &sum);
-    if (positions != nullptr) positions[static_cast<uint64_t>(i) * k + e] = static_cast<uint32_t>(p);
+  if (!CursorRow(cursor, k, first + i, pos, &task)) atomicOr(status, 1u);
+  if (positions != nullptr) {
+    for (uint32_t e = 0; e < k; ++e) positions[static_cast<uint64_t>(i) * k + e] = static_cast<uint32_t>(pos[e]);
   }
-  overflow |= sum > static_cast<uint64_t>(std::numeric_limits<int64_t>::max());
-  if (overflow) atomicOr(status, 1u);
-  task.deleted_cost = overflow ? 0 : static_cast<int64_t>(sum);
   tasks[i] = task;
 }
 
@@ -140,15 +81,28 @@ void CheckTourView(const ee_tour_view* tour, int32_t n) {
   }
 }
 
-// Keeps the device copy of the tour view; returns whether it was resident.
-bool PrepareTour(Context& ctx, const ee_tour_view& t) {
-  KoptCursorCache& c = ctx.cursor;
+// Whether the device copy is of this very tour, which then passed
+// CheckTourView for snapshots of n nodes when it was uploaded.
+bool TourMatches(const KoptCursorCache& c, const ee_tour_view* tour, int32_t n) {
+  if (!c.valid || c.nodes != n || tour == nullptr || tour->tour == nullptr || tour->edge_costs == nullptr ||
+      (tour->selectable == nullptr && tour->selectable_count > 0)) {
+    return false;
+  }
+  const ee_tour_view& t = *tour;
   const size_t L = t.tour_length, S = t.selectable_count;
-  const bool hit = c.valid && c.tour.size() == L && c.selectable.size() == S &&
-                   std::memcmp(c.tour.data(), t.tour, L * sizeof(int32_t)) == 0 &&
-                   std::memcmp(c.edge_costs.data(), t.edge_costs, L * sizeof(int64_t)) == 0 &&
-                   (S == 0 || std::memcmp(c.selectable.data(), t.selectable, S * sizeof(uint64_t)) == 0);
-  if (hit) return true;
+  return c.tour.size() == L && c.selectable.size() == S &&
+         std::memcmp(c.tour.data(), t.tour, L * sizeof(int32_t)) == 0 &&
+         std::memcmp(c.edge_costs.data(), t.edge_costs, L * sizeof(int64_t)) == 0 &&
+         (S == 0 || std::memcmp(c.selectable.data(), t.selectable, S * sizeof(uint64_t)) == 0);
+}
+
+// Checks the tour view and keeps its device copy.
+void PrepareTour(Context& ctx, const ee_tour_view* tour, int32_t n) {
+  KoptCursorCache& c = ctx.cursor;
+  if (TourMatches(c, tour, n)) return;
+  CheckTourView(tour, n);
+  const ee_tour_view& t = *tour;
+  const size_t L = t.tour_length, S = t.selectable_count;
   c.valid = false;
   if (c.d_tour.count() < L) c.d_tour.Allocate(Grow(c.d_tour.count(), L), ctx.device);
   if (c.d_edge_costs.count() < L) c.d_edge_costs.Allocate(Grow(c.d_edge_costs.count(), L), ctx.device);
@@ -168,8 +122,13 @@ bool PrepareTour(Context& ctx, const ee_tour_view& t) {
   c.tour.assign(t.tour, t.tour + L);
   c.edge_costs.assign(t.edge_costs, t.edge_costs + L);
   c.selectable.assign(t.selectable, t.selectable + S);
+  c.nodes = n;
   c.valid = true;
-  return false;
+}
+
+KoptCursor DeviceTour(const KoptCursorCache& c, const ee_tour_view& t) {
+  return KoptCursor{c.d_tour.get(), c.d_edge_costs.get(), c.d_selectable.get(), t.tour_length,
+                    t.selectable_count - 1};
 }
 
 void LaunchCursor(Context& ctx, const ee_tour_view& t, uint32_t k, uint64_t first, uint32_t count,
@@ -179,10 +138,8 @@ void LaunchCursor(Context& ctx, const ee_tour_view& t, uint32_t k, uint64_t firs
     c.d_positions.Allocate(Grow(c.d_positions.count(), static_cast<size_t>(count) * k), ctx.device);
   }
   const uint32_t blocks = (count + kCursorBlock - 1) / kCursorBlock;
-  hipLaunchKernelGGL(KoptCursorKernel, dim3(blocks), dim3(kCursorBlock), 0, ctx.stream,
-                     c.d_tour.get(), c.d_edge_costs.get(), c.d_selectable.get(), t.tour_length,
-                     t.selectable_count - 1, k, first, count, d_tasks,
-                     want_positions ? c.d_positions.get() : nullptr, c.d_status.get());
+  hipLaunchKernelGGL(KoptCursorKernel, dim3(blocks), dim3(kCursorBlock), 0, ctx.stream, DeviceTour(c, t), k, first,
+                     count, d_tasks, want_positions ? c.d_positions.get() : nullptr, c.d_status.get());
   CheckHip(hipGetLastError(), "KoptCursorKernel launch");
 }
 
@@ -213,31 +170,26 @@ void CursorEval(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uin
     throw std::invalid_argument("k-opt cursor: costs and masks are exclusive");
   }
   if (k < 3 || k > 5) throw std::invalid_argument("k-opt cursor: k must lie in [3, 5]");
-  CheckTourView(tour, n);
+  const bool resident = TourMatches(ctx.cursor, tour, n);
+  if (!resident) CheckTourView(tour, n);
   const uint64_t total = SetCount(tour->selectable_count, k);
   const uint32_t rows = first >= total ? 0 : static_cast<uint32_t>(std::min<uint64_t>(count, total - first));
   if (rows == 0) return;
-  PrepareTour(ctx, *tour);
-  const bool want_positions = positions != nullptr;
-  try {
-    if (costs == nullptr && masks == nullptr) {  // producer only
-      KoptCache& kc = ctx.kopt;
-      if (kc.d_tasks.count() < rows) kc.d_tasks.Allocate(Grow(kc.d_tasks.count(), rows), ctx.device);
-      LaunchCursor(ctx, *tour, k, first, rows, kc.d_tasks.get(), want_positions);
-    } else {
-      const KoptTaskSource produce = [&](ee_kopt_task* d_tasks) {
-        LaunchCursor(ctx, *tour, k, first, rows, d_tasks, want_positions);
-      };
-      EvalKoptCostsFrom(ctx, x, y, n, type, k, templates, template_count, generator_hash, rows,
-                        produce, false, costs, masks, usage);
-    }
-  } catch (...) {
-    // a failed evaluation may leave the overflow flag set; clear it (best
-    // effort) so that the next call does not report this one's overflow
-    static_cast<void>(hipMemsetAsync(ctx.cursor.d_status.get(), 0, sizeof(uint32_t), ctx.stream));
-    static_cast<void>(hipStreamSynchronize(ctx.stream));
-    throw;
+  PrepareTour(ctx, tour, n);
+  if (costs != nullptr || masks != nullptr) {
+    KoptRows made;
+    made.cursor = DeviceTour(ctx.cursor, *tour);
+    made.first = first;
+    made.out_tasks = tasks;
+    made.out_positions = positions;
+    EvalKoptRows(ctx, x, y, n, type, k, templates, template_count, generator_hash, rows, made, costs, masks, usage);
+    if (produced) *produced = rows;
+    return;
   }
+  // the rows only
+  KoptCache& kc = ctx.kopt;
+  if (kc.d_tasks.count() < rows) kc.d_tasks.Allocate(Grow(kc.d_tasks.count(), rows), ctx.device);
+  LaunchCursor(ctx, *tour, k, first, rows, kc.d_tasks.get(), positions != nullptr);
   FinishCursor(ctx, k, rows, tasks, positions);
   if (produced) *produced = rows;
 }
@@ -263,9 +215,9 @@ void LaunchCursorRows(const int32_t* d_tour, const int64_t* d_edge_costs, const 
                       hipStream_t stream) {
   if (count == 0) return;
   const uint32_t blocks = (count + kCursorBlock - 1) / kCursorBlock;
-  hipLaunchKernelGGL(KoptCursorKernel, dim3(blocks), dim3(kCursorBlock), 0, stream, d_tour, d_edge_costs,
-                     d_selectable, tour_length, selectable_count - 1, k, first, count, d_tasks, d_positions,
-                     d_status);
+  hipLaunchKernelGGL(KoptCursorKernel, dim3(blocks), dim3(kCursorBlock), 0, stream,
+                     KoptCursor{d_tour, d_edge_costs, d_selectable, tour_length, selectable_count - 1}, k, first, count,
+                     d_tasks, d_positions, d_status);
   CheckHip(hipGetLastError(), "KoptCursorKernel launch");
 }
 

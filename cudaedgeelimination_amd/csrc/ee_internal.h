@@ -88,6 +88,7 @@ struct KoptKLayout {
   uint32_t pair_step_r, pair_step_p;  // 64 = pair_step_r * P + pair_step_p
   uint32_t pq_off, tpl_off;
   uint32_t xy_off, row_off, dcost_off, pair_off;
+  uint32_t made_off;  // rows made by the wavefront: their 48-byte rows, then their positions
 };
 
 // A segment carried in the kernel arguments: for launches of at most
@@ -108,6 +109,15 @@ constexpr uint32_t kInlineSegments = 8;
 // bytes, one L2 line): partial-line stores cost the memory system a
 // read-modify-write.
 constexpr uint64_t kSegmentAlignCells = 16;
+
+// A tour context on the device: the deletion sets of the cost cursor are
+// selectable[0] and k - 1 of the other `labels` selectable positions.
+struct KoptCursor {
+  const int32_t* tour;
+  const int64_t* edge_costs;
+  const uint64_t* selectable;
+  uint32_t tour_length, labels;
+};
 
 // Tiles are numbered k by k: tiles [k_tile_begin[i], k_tile_begin[i] +
 // k_tile_count[i]) belong to segments with k = 3 + i, and the k_block_count[i]
@@ -140,6 +150,16 @@ struct KoptLaunch {
   uint64_t* marks;
   uint64_t mark;
   uint32_t bound_nodes;
+  // row_status non-null: there are no task rows; row r is that of deletion
+  // set row_first + r of `cursor`, made by the wavefront that evaluates it,
+  // which also writes it to made_tasks[r] and its k positions to
+  // made_positions + k r, in host memory, and 1 to *row_status where the
+  // deleted cost overflows
+  KoptCursor cursor;
+  uint64_t row_first;
+  ee_kopt_task* made_tasks;
+  uint32_t* made_positions;
+  uint32_t* row_status;
   KoptKLayout layout[3];
   uint32_t wave_base;   // LDS offset of the first wave's tile arrays
   uint32_t wave_bytes;  // LDS bytes per wave

@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "ee_cursor_body.h"
 #include "ee_exact.h"
 #include "ee_internal.h"
 #include "ee_jv_body.h"
@@ -163,6 +164,54 @@ __device__ __forceinline__ void StagePorts(const KoptLaunch& a, const KoptPointe
       }
     }
   }
+  WaveSync();
+}
+
+// Phase A of a tile whose rows are deletion sets of the tour context: lane r
+// makes row r, then the ports' coordinates are gathered as in StagePorts.
+// The rows and positions are staged in LDS and written to host memory in
+// whole words, consecutive lanes to consecutive addresses.
+template <int K, bool kNear, int kOut>
+__device__ __forceinline__ void MakeRows(const KoptLaunch& a, const KoptPointers& bufs, const KoptKLayout& L,
+                                         const KoptTile& d, char* wave, int lane) {
+  constexpr uint32_t kPorts = 2 * K;
+  char* w_port = wave + L.xy_off;
+  int32_t* w_node = reinterpret_cast<int32_t*>(wave + L.pair_off);
+  uint32_t* w_task = reinterpret_cast<uint32_t*>(wave + L.made_off);
+  uint32_t* w_position = w_task + d.rows * 12;
+  const uint32_t r = static_cast<uint32_t>(lane);
+  if (r < d.rows) {
+    uint64_t pos[kMaxK];
+    ee_kopt_task row{};
+    if (!CursorRow(a.cursor, K, a.row_first + d.task_index + r, pos, &row)) {
+      __hip_atomic_store(a.row_status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < 10; ++p) w_task[r * 12 + p] = static_cast<uint32_t>(row.port_nodes[p]);
+    w_task[r * 12 + 10] = static_cast<uint32_t>(row.deleted_cost);
+    w_task[r * 12 + 11] = static_cast<uint32_t>(static_cast<uint64_t>(row.deleted_cost) >> 32);
+#pragma unroll
+    for (uint32_t p = 0; p < kPorts; ++p) w_node[r * kPorts + p] = row.port_nodes[p];
+#pragma unroll
+    for (uint32_t e = 0; e < K; ++e) w_position[r * K + e] = static_cast<uint32_t>(pos[e]);
+    reinterpret_cast<uint32_t*>(wave + L.row_off)[r] = 0;
+    if (kOut == kOutMasks) reinterpret_cast<int64_t*>(wave + L.dcost_off)[r] = row.deleted_cost;
+  }
+  WaveSync();
+  const longlong2* xy = bufs.xy + d.coord_base;
+  for (uint32_t s = static_cast<uint32_t>(lane); s < d.rows * kPorts; s += kWave) {
+    const longlong2 c = xy[w_node[s]];
+    if (kNear) {
+      *reinterpret_cast<uint2*>(w_port + s * kNearPortBytes) =
+          uint2{static_cast<uint32_t>(c.x), static_cast<uint32_t>(c.y)};
+    } else {
+      *reinterpret_cast<longlong2*>(w_port + s * kFarPortBytes) = c;
+    }
+  }
+  uint32_t* tasks = reinterpret_cast<uint32_t*>(a.made_tasks + d.task_index);
+  for (uint32_t q = static_cast<uint32_t>(lane); q < d.rows * 12; q += kWave) tasks[q] = w_task[q];
+  uint32_t* positions = a.made_positions + static_cast<uint64_t>(d.task_index) * K;
+  for (uint32_t q = static_cast<uint32_t>(lane); q < d.rows * K; q += kWave) positions[q] = w_position[q];
   WaveSync();
 }
 
@@ -538,7 +587,7 @@ __device__ __forceinline__ KoptTile TileAt(const KoptLaunch& a, const KoptPointe
 // The tiles of one k handed to this workgroup, one per wavefront at a time.
 // The plan is fetched into registers first, so its latency overlaps the
 // first tile's gathers; it reaches LDS before the only block barrier.
-template <int K, bool kNonTemporal, int kOut>
+template <int K, bool kNonTemporal, int kOut, bool kMade>
 __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* smem) {
   constexpr int ki = K - 3;
   // k = 5 tiles hold most of the cells and end the launch: their wavefronts
@@ -568,13 +617,21 @@ __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* sm
   const uint64_t stride = static_cast<uint64_t>(blocks) * waves_per_block;
   const uint64_t end = a.k_tile_begin[ki] + a.k_tile_count[ki];
   uint64_t tile = a.k_tile_begin[ki] + __builtin_amdgcn_readfirstlane(block * waves_per_block + wib);
+  const auto stage = [&](auto near, const KoptTile& d) {
+    constexpr bool kNear = decltype(near)::value;
+    if constexpr (kMade) {
+      MakeRows<K, kNear, kOut>(a, bufs, L, d, wave, lane);
+    } else {
+      StagePorts<K, kNear, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+    }
+  };
   KoptTile d{};
   if (tile < end) {
     d = TileAt<K>(a, bufs, L, tile);
     if (d.near != 0) {
-      StagePorts<K, true, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+      stage(std::true_type{}, d);
     } else {
-      StagePorts<K, false, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+      stage(std::false_type{}, d);
     }
   }
 
@@ -592,14 +649,14 @@ __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* sm
   for (bool first = true; tile < end; tile += stride, first = false) {
     if (!first) d = TileAt<K>(a, bufs, L, tile);
     if (d.near != 0) {
-      if (!first) StagePorts<K, true, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+      if (!first) stage(std::true_type{}, d);
       TileCells<K, true, kNonTemporal, kOut>(a, bufs, L, d, smem, wave, lane);
     } else {
-      if (!first) StagePorts<K, false, kOut>(a, bufs, L, d, wave, lane, a.bound_nodes);
+      if (!first) stage(std::false_type{}, d);
       TileCells<K, false, kNonTemporal, kOut>(a, bufs, L, d, smem, wave, lane);
     }
-    if constexpr (kOut == kOutPacked) {
-      // the tile's cells, then its mark: the host takes a tile's cells once
+    if constexpr (kOut == kOutPacked || kMade) {
+      // the tile's output, then its mark: the host takes a tile's output once
       // it sees the mark, while later tiles are still on their way
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
       if (lane == 0) {
@@ -610,14 +667,14 @@ __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* sm
   if (bufs.stamps != nullptr && lane == 0) bufs.stamps[2 * static_cast<uint64_t>(wave_id) + 1] = __builtin_amdgcn_s_memrealtime();
 }
 
-template <bool kNonTemporal, int kOut>
+template <bool kNonTemporal, int kOut, bool kMade = false>
 __device__ __forceinline__ void KoptBody(const KoptLaunch& a, const KoptPointers& bufs, char* smem) {
   if (blockIdx.x < a.k_block_first[1]) {
-    TileLoop<3, kNonTemporal, kOut>(a, bufs, smem);
+    TileLoop<3, kNonTemporal, kOut, kMade>(a, bufs, smem);
   } else if (blockIdx.x < a.k_block_first[2]) {
-    TileLoop<4, kNonTemporal, kOut>(a, bufs, smem);
+    TileLoop<4, kNonTemporal, kOut, kMade>(a, bufs, smem);
   } else {
-    TileLoop<5, kNonTemporal, kOut>(a, bufs, smem);
+    TileLoop<5, kNonTemporal, kOut, kMade>(a, bufs, smem);
   }
 }
 
@@ -627,6 +684,15 @@ __global__ void __launch_bounds__(256) KoptKernel(KoptLaunch a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const KoptPointers bufs{a.xy, a.tiles, a.tasks, a.plans, a.costs, a.masks, a.packed_lo, a.packed_hi, nullptr};
   KoptBody<kNonTemporal, kOut>(a, bufs, smem);
+}
+
+// Rows made by the wavefronts that evaluate them (KoptLaunch::row_status),
+// everything written to host memory.
+template <int kOut>
+__global__ void __launch_bounds__(256) KoptCursorCostKernel(KoptLaunch a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const KoptPointers bufs{a.xy, a.tiles, a.tasks, a.plans, a.costs, a.masks, a.packed_lo, a.packed_hi, nullptr};
+  KoptBody<false, kOut, true>(a, bufs, smem);
 }
 
 // The launch arguments in ordinary device memory, for callers that launch
@@ -1038,8 +1104,11 @@ size_t KoptPrepareLayout(KoptLaunch* a, const KoptPlan plans[3], const bool pres
     L.row_off = Align16(std::max(port_bytes, stage_bytes));
     L.dcost_off = L.row_off + Align16(rows * 4);
     L.pair_off = L.dcost_off + (a->masks != nullptr ? Align16(rows * 8) : 0u);
-    // the port node ids of phase A share the pair record area
-    const uint32_t pair_bytes = std::max(L.P * L.pair_stride * 8, rows * ports * 4);
+    // the port node ids of phase A share the pair record area, and so do rows
+    // made by the wavefront (behind the node ids)
+    L.made_off = L.pair_off + Align16(rows * ports * 4);
+    const uint32_t made_bytes = a->row_status != nullptr ? rows * (48 + 4 * k) : 0u;
+    const uint32_t pair_bytes = std::max(L.P * L.pair_stride * 8, Align16(rows * ports * 4) + made_bytes);
     wave_bytes = std::max<uint32_t>(wave_bytes, L.pair_off + Align16(pair_bytes));
   }
   a->wave_base = plan_bytes;
@@ -1156,7 +1225,11 @@ void LaunchKopt(const KoptLaunch& args, const KoptTuning& tuning, size_t shared_
   const uint32_t grid = KoptFinalize(&a, tuning, shared_bytes);
   if (grid == 0) return;
   const dim3 g(grid), b(tuning.block);
-  if (a.masks != nullptr) {
+  if (a.row_status != nullptr && a.masks != nullptr) {
+    hipLaunchKernelGGL((KoptCursorCostKernel<kOutMasks>), g, b, shared_bytes, stream, a);
+  } else if (a.row_status != nullptr) {
+    hipLaunchKernelGGL((KoptCursorCostKernel<kOutPacked>), g, b, shared_bytes, stream, a);
+  } else if (a.masks != nullptr) {
     hipLaunchKernelGGL((KoptKernel<false, kOutMasks>), g, b, shared_bytes, stream, a);
   } else if (a.packed_lo != nullptr) {
     hipLaunchKernelGGL((KoptKernel<false, kOutPacked>), g, b, shared_bytes, stream, a);

@@ -198,9 +198,7 @@ struct KoptCache {
   std::array<TemplateEntry, 3> templates;
   std::array<KoptPlan, 3> host_plans;
   DeviceArray<KoptPlan> d_plans;
-  DeviceArray<ee_kopt_task> d_tasks;
-  DeviceArray<int64_t> d_costs;
-  DeviceArray<KoptTile> d_tiles;
+  DeviceArray<ee_kopt_task> d_tasks;  // rows made without an evaluation
   // largest evaluation through the ring so far, grown as the buffers are
   size_t task_room = 0, cell_room = 0;
   bool Reserve(size_t tasks, size_t cells);
@@ -235,6 +233,10 @@ class DirectIo {
   // form, tile_cells to a tile, and expands them to int64 as they arrive.
   void TakeCells(size_t slot, uint64_t mark, hipStream_t stream, const uint32_t* lo, const uint8_t* hi,
                  size_t count, size_t tile_cells, int64_t* cells) const;
+  // Waits for tiles [0, tiles) in groups, in order, and calls take(first,
+  // last) for each group as it arrives, on up to `threads` host threads.
+  void TakeTiles(size_t slot, uint64_t mark, hipStream_t stream, size_t tiles, size_t group, unsigned threads,
+                 const std::function<void(size_t, size_t)>& take) const;
 
  private:
   Pinned<char> mem_;
@@ -248,6 +250,7 @@ class DirectIo {
 // the caller passes the same tour, edge costs and selectable positions.
 struct KoptCursorCache {
   bool valid = false;
+  int32_t nodes = 0;  // node count of the snapshots the tour was checked for
   std::vector<int32_t> tour;
   std::vector<int64_t> edge_costs;
   std::vector<uint64_t> selectable;
@@ -350,21 +353,25 @@ void ValidateTasks(int32_t n, uint32_t k, const ee_kopt_task* tasks, size_t coun
 // Null arrays, dimensions, distance type and integer coordinates of a view.
 void CheckGraphView(const ee_graph_view* g);
 
-// Writes the task rows of one plain evaluation into the device task pool
-// (`d_tasks`, room for the evaluation's rows), enqueued on the context's
-// stream.  The rows must pass ValidateTasks.
-using KoptTaskSource = std::function<void(ee_kopt_task* d_tasks)>;
+// The task rows of one plain evaluation: the caller's (which must pass
+// ValidateTasks), or, with `tasks` null, those of the deletion sets from rank
+// `first` of a checked tour context on the device, delivered to out_tasks
+// and out_positions where these are not null.
+struct KoptRows {
+  const ee_kopt_task* tasks = nullptr;
+  KoptCursor cursor{};
+  uint64_t first = 0;
+  ee_kopt_task* out_tasks = nullptr;
+  uint32_t* out_positions = nullptr;
+};
 
-// The plain synchronous k-opt evaluation (snapshot, template and workspace
-// caches, one launch, download) with its task rows taken from `fill_tasks`.
-// Exactly one of `costs` (task_count x template_count cells) and `masks`
-// (task_count x ceil(template_count / 32) improving-template words) is
-// non-null.  sync_after_fill: wait for the rows before the launch (usage's
-// h2d_ms is then their transfer); rows made by a kernel on the context's
-// stream need no wait, and their time falls into kernel_ms.
-void EvalKoptCostsFrom(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
-                       uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
-                       uint64_t generator_hash, size_t task_count, const KoptTaskSource& fill_tasks,
-                       bool sync_after_fill, int64_t* costs, uint32_t* masks, ee_kopt_usage* usage);
+// The plain synchronous k-opt evaluation (snapshot and template caches, rows
+// and output through the context's ring).  Exactly one of `costs`
+// (task_count x template_count cells) and `masks` (task_count x
+// ceil(template_count / 32) improving-template words) is non-null, masks only
+// with made rows.
+void EvalKoptRows(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type, uint32_t k,
+                  const ee_endpoint_matching* templates, uint32_t template_count, uint64_t generator_hash,
+                  size_t task_count, const KoptRows& rows, int64_t* costs, uint32_t* masks, ee_kopt_usage* usage);
 
 }  // namespace ee

@@ -345,8 +345,7 @@ void FindJvCandidates(Context& ctx, const ee_graph_view& g, int32_t* witnesses, 
 // Device memory of the caches and the page-locked ring the kernels work in.
 uint64_t KoptResidentBytes(const Context& ctx) {
   const KoptCache& c = ctx.kopt;
-  return c.d_xy.bytes() + c.d_plans.bytes() + c.d_tasks.bytes() + c.d_costs.bytes() +
-         c.d_tiles.bytes() + ctx.io.bytes();
+  return c.d_xy.bytes() + c.d_plans.bytes() + c.d_tasks.bytes() + ctx.io.bytes();
 }
 
 // Whether an evaluation of this size found room, with the growth rule of the
@@ -357,8 +356,6 @@ bool KoptCache::Reserve(size_t tasks, size_t cells) {
   cell_room = Grow(cell_room, cells);
   return hit;
 }
-
-uint32_t TileRows(const KoptTuning& tuning, uint32_t k) { return tuning.rows_per_tile[k - 3]; }
 
 namespace {
 
@@ -431,22 +428,26 @@ KoptHits PrepareKoptCaches(Context& ctx, const int64_t* x, const int64_t* y, int
 }
 
 // The rows of one evaluation, cut into launches that pass through the
-// context's page-locked ring: per launch its task rows, and the cells in
-// transfer form (low words, then high bytes on instances that are not near).
+// context's page-locked ring.  A launch's slot holds an overflow flag, its
+// task rows (the caller's, or made ones on their way out) and positions, and
+// its output: mask words, or cells in transfer form (low words, then high
+// bytes on instances that are not near).
 struct KoptChunks {
   static constexpr size_t kSlotBytes = size_t{4} << 20;
 
-  KoptChunks(size_t rows, size_t templates, uint32_t tile_rows, bool wide) : rows_(rows) {
-    const size_t per_row = sizeof(ee_kopt_task) + templates * (wide ? 5 : 4);
+  KoptChunks(size_t rows, uint32_t tile_rows, size_t position_bytes, size_t low_bytes, size_t high_bytes)
+      : rows_(rows) {
+    const size_t per_row = sizeof(ee_kopt_task) + position_bytes + low_bytes + high_bytes;
     const size_t fit = std::min<size_t>(std::max<size_t>(kSlotBytes / per_row / tile_rows, 1), DirectIo::kSlotTiles);
     count = (rows + fit * tile_rows - 1) / (fit * tile_rows);
     // launches of equal size, whole tiles each
     const size_t even = (rows + count - 1) / count;
     chunk_rows = std::min(rows, (even + tile_rows - 1) / tile_rows * tile_rows);
     count = (rows + chunk_rows - 1) / chunk_rows;
-    lo_off = Align256(chunk_rows * sizeof(ee_kopt_task));
-    hi_off = lo_off + Align256(chunk_rows * templates * 4);
-    slot_bytes = hi_off + (wide ? Align256(chunk_rows * templates) : 0);
+    positions_off = rows_off + Align256(chunk_rows * sizeof(ee_kopt_task));
+    lo_off = positions_off + Align256(chunk_rows * position_bytes);
+    hi_off = lo_off + Align256(chunk_rows * low_bytes);
+    slot_bytes = hi_off + Align256(chunk_rows * high_bytes);
     slots = std::min<size_t>(count, DirectIo::kSlots);
   }
   static size_t Align256(size_t v) { return (v + 255) & ~size_t{255}; }
@@ -454,7 +455,8 @@ struct KoptChunks {
   size_t Rows(size_t chunk) const { return std::min(chunk_rows, rows_ - First(chunk)); }
 
   size_t count = 0, chunk_rows = 0, slots = 0;
-  size_t lo_off = 0, hi_off = 0, slot_bytes = 0;
+  static constexpr size_t rows_off = 256;
+  size_t positions_off = 0, lo_off = 0, hi_off = 0, slot_bytes = 0;
 
  private:
   size_t rows_;
@@ -483,40 +485,45 @@ bool LooksResident(const KoptCache& c, const int64_t* x, const int64_t* y, int32
   return std::memcmp(c.x.data(), x, sample) == 0 && std::memcmp(c.y.data(), y, sample) == 0;
 }
 
-// Tiles of the launches that write to host memory.  PCIe bounds them, so few
-// wavefronts with several small tiles each: 192 keep the link busy and their
-// first tiles arrive early, so the host expands while the rest crosses.  A
-// k = 5 block of 4,096 rows takes 120 us (rows 4, 192 wavefronts), 126 with
-// 256 and 158 with one tile per wavefront, whose tiles all end together;
-// k = 3 and 4, with less output per row, measured best at 256.
-KoptTuning DirectTuning(uint32_t k) {
+// Tiles of the launches that write to host memory.  Where cells go out, PCIe
+// bounds them, so few wavefronts take several small tiles each: they keep
+// the link busy and their first tiles arrive early, so the host expands while
+// the rest crosses.  A k = 5 block of 4,096 rows takes 120 us (rows 4, 192
+// wavefronts), 126 with 256 and 158 with one tile per wavefront, whose tiles
+// all end together; k = 3 and 4, with less output per row, measured best at
+// 256.  Masks are small, so the wavefronts' own chain bounds them: one short
+// tile each (4,096 k = 5 sets: 59 us with 8 rows, 61 with 16, 64 with 4).
+KoptTuning DirectTuning(uint32_t k, bool masks) {
+  constexpr uint32_t kCellRows[3] = {64, 16, 4}, kMaskRows[3] = {32, 8, 8};
   KoptTuning t;
-  t.rows_per_tile[0] = 64;
-  t.rows_per_tile[1] = 16;
-  t.rows_per_tile[2] = 4;
+  std::copy_n(masks ? kMaskRows : kCellRows, 3, t.rows_per_tile);
   t.block = 64;
-  t.grid = k == 5 ? 192 : 256;
+  t.grid = masks ? 0 : k == 5 ? 192 : 256;
   return t;
 }
 
-// The kernel reads the task rows from page-locked host memory and writes the
-// cells back there in transfer form, tile by tile, so a call has no copy
-// command and no wait for the stream, and half the bytes of int64 cells
-// cross PCIe (56 GB/s here, which bounds a block: 61 us for 4,096 k = 5
-// rows).  Host threads expand tiles into the caller's buffer as their marks
-// arrive.  Against an upload, a launch and a download with a wait each: one
-// k = 5 row 56 -> 19 us, 1,237 k = 4 rows 63 -> 32 us, 4,096 k = 5 rows
-// 293 -> 121 us, 1,501 wide k = 5 rows 163 -> 83 us.
+// The kernel reads the task rows from page-locked host memory, or makes them
+// itself, and writes its output (and made rows) back there, cells in transfer
+// form, tile by tile.  So a call has no copy command and no wait for the
+// stream, and half the bytes of int64 cells cross PCIe (56 GB/s here, which
+// bounds a block: 61 us for 4,096 k = 5 rows).  Host threads take tiles into
+// the caller's buffers as their marks arrive.  Against an upload, a launch
+// and a download with a wait each: one k = 5 row 56 -> 19 us, 1,237 k = 4
+// rows 63 -> 32 us, 4,096 k = 5 rows 293 -> 121 us, 1,501 wide k = 5 rows
+// 163 -> 83 us, 4,096 made k = 5 rows with their masks 125 -> 60 us.
 // `check` runs on the host while the first launches are on the device; false
 // drops their output and returns false, with nothing delivered.
-bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t template_count,
-               const ee_kopt_task* tasks, size_t task_count, int64_t* costs, const std::function<bool()>& check,
+bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t template_count, size_t task_count,
+               const KoptRows& rows, int64_t* costs, uint32_t* masks, const std::function<bool()>& check,
                ee_kopt_usage* usage) {
   ee_kopt_usage u{};
   KoptCache& c = ctx.kopt;
-  const KoptTuning tuning = DirectTuning(k);
+  const bool made = rows.tasks == nullptr, wide = !c.near && masks == nullptr;
+  const uint32_t mask_words = (template_count + 31) / 32;
+  const KoptTuning tuning = DirectTuning(k, masks != nullptr);
   const uint32_t tile_rows = tuning.rows_per_tile[k - 3];
-  const KoptChunks chunks(task_count, template_count, tile_rows, !c.near);
+  const KoptChunks chunks(task_count, tile_rows, made ? 4 * k : 0, 4 * (masks ? mask_words : template_count),
+                          wide ? template_count : 0);
   DirectIo& io = ctx.io;
   io.Reserve(chunks.slots * chunks.slot_bytes);
 
@@ -529,25 +536,56 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
   uint64_t marks[DirectIo::kSlots] = {};
   const auto slot_of = [&](size_t chunk) { return chunk % chunks.slots * chunks.slot_bytes; };
   const auto launch = [&](size_t chunk) {
-    const size_t rows = chunks.Rows(chunk), slot = chunk % chunks.slots, at = slot_of(chunk);
-    const ee_kopt_task* from = tasks + chunks.First(chunk);
-    ee_kopt_task* staged = reinterpret_cast<ee_kopt_task*>(io.host() + at);
-    InParts(rows, 8192, [&](size_t b, size_t e) { std::memcpy(staged + b, from + b, (e - b) * sizeof(*from)); });
-    KoptSegment segment{0, k, 0, rows, 0, 0, tile_rows, 0};
+    const size_t count = chunks.Rows(chunk), slot = chunk % chunks.slots, at = slot_of(chunk);
+    char* const device = io.device() + at;
+    KoptSegment segment{0, k, 0, count, 0, 0, tile_rows, 0};
     KoptLaunch a{};
     KoptAssignTiles(&segment, 1, &inst, c.host_plans.data(), tuning, nullptr, &a);
     if (a.inline_count == 0) throw std::logic_error("a one-segment k-opt launch needs its inline table");
     a.xy = c.d_xy.get();
-    a.tasks = reinterpret_cast<const ee_kopt_task*>(io.device() + at);
     a.plans = c.d_plans.get();
-    a.packed_lo = reinterpret_cast<uint32_t*>(io.device() + at + chunks.lo_off);
-    a.packed_hi = c.near ? nullptr : reinterpret_cast<uint8_t*>(io.device() + at + chunks.hi_off);
+    if (made) {
+      *reinterpret_cast<uint32_t*>(io.host() + at) = 0;
+      a.row_status = reinterpret_cast<uint32_t*>(device);
+      a.cursor = rows.cursor;
+      a.row_first = rows.first + chunks.First(chunk);
+      a.made_tasks = reinterpret_cast<ee_kopt_task*>(device + chunks.rows_off);
+      a.made_positions = reinterpret_cast<uint32_t*>(device + chunks.positions_off);
+    } else {
+      const ee_kopt_task* from = rows.tasks + chunks.First(chunk);
+      ee_kopt_task* staged = reinterpret_cast<ee_kopt_task*>(io.host() + at + chunks.rows_off);
+      InParts(count, 8192, [&](size_t b, size_t e) { std::memcpy(staged + b, from + b, (e - b) * sizeof(*from)); });
+      a.tasks = reinterpret_cast<const ee_kopt_task*>(device + chunks.rows_off);
+      a.bound_nodes = static_cast<uint32_t>(n);
+    }
+    if (masks) {
+      a.masks = reinterpret_cast<uint32_t*>(device + chunks.lo_off);
+      a.mask_words = mask_words;
+    } else {
+      a.packed_lo = reinterpret_cast<uint32_t*>(device + chunks.lo_off);
+      a.packed_hi = wide ? reinterpret_cast<uint8_t*>(device + chunks.hi_off) : nullptr;
+    }
     a.marks = io.device_marks(slot);
     a.mark = marks[slot] = io.NextMark();
-    a.bound_nodes = static_cast<uint32_t>(n);
     const size_t shared = KoptPrepareLayout(&a, c.host_plans.data(), present, tuning, c.near);
     LaunchKopt(a, tuning, shared, ctx.stream);
   };
+  // made rows, their positions and mask words of tiles [first, last)
+  const auto take_rows = [&](size_t chunk, size_t first, size_t last) {
+    const size_t b = first * tile_rows, count = std::min(chunks.Rows(chunk), last * tile_rows) - b;
+    const size_t row = chunks.First(chunk) + b;
+    const char* at = io.host() + slot_of(chunk);
+    if (rows.out_tasks != nullptr) {
+      std::memcpy(rows.out_tasks + row, at + chunks.rows_off + b * sizeof(ee_kopt_task), count * sizeof(ee_kopt_task));
+    }
+    if (rows.out_positions != nullptr) {
+      std::memcpy(rows.out_positions + row * k, at + chunks.positions_off + b * 4 * k, count * 4 * k);
+    }
+    if (masks != nullptr) {
+      std::memcpy(masks + row * mask_words, at + chunks.lo_off + b * 4 * mask_words, count * 4 * mask_words);
+    }
+  };
+  bool overflow = false;
   try {
     auto t0 = std::chrono::steady_clock::now();
     for (size_t i = 0; i < chunks.slots; ++i) launch(i);
@@ -558,16 +596,26 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
       return false;
     }
     for (size_t i = 0; i < chunks.count; ++i) {
-      const size_t slot = i % chunks.slots, rows = chunks.Rows(i);
+      const size_t slot = i % chunks.slots, count = chunks.Rows(i);
       io.WaitTile(slot, 0, marks[slot], ctx.stream);
       if (i == 0) {
         u.kernel_ms = MsSince(t0);
         t0 = std::chrono::steady_clock::now();
       }
       const char* from = io.host() + slot_of(i);
-      io.TakeCells(slot, marks[slot], ctx.stream, reinterpret_cast<const uint32_t*>(from + chunks.lo_off),
-                   c.near ? nullptr : reinterpret_cast<const uint8_t*>(from + chunks.hi_off),
-                   rows * template_count, tile_rows * template_count, costs + chunks.First(i) * template_count);
+      if (masks == nullptr) {
+        io.TakeCells(slot, marks[slot], ctx.stream, reinterpret_cast<const uint32_t*>(from + chunks.lo_off),
+                     wide ? reinterpret_cast<const uint8_t*>(from + chunks.hi_off) : nullptr,
+                     count * template_count, tile_rows * template_count, costs + chunks.First(i) * template_count);
+      }
+      if (made) {
+        const size_t tiles = (count + tile_rows - 1) / tile_rows;
+        // 256 rows at a time on this thread: a block's rows and words are a few
+        // hundred KB, and four threads took 20 us where one takes 13
+        io.TakeTiles(slot, marks[slot], ctx.stream, tiles, std::max<size_t>(1, 256 / tile_rows), 1,
+                     [&](size_t first, size_t last) { take_rows(i, first, last); });
+        overflow = overflow || *reinterpret_cast<const uint32_t*>(from) != 0;
+      }
       if (i + chunks.slots < chunks.count) launch(i + chunks.slots);
     }
     u.d2h_ms = MsSince(t0);
@@ -575,14 +623,57 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
     static_cast<void>(hipStreamSynchronize(ctx.stream));  // the ring is free again
     throw;
   }
+  if (overflow) throw std::runtime_error("k-opt cursor: deleted cost sum overflows int64_t");
   u.snapshot_hit = u.template_hit = 1;
-  u.workspace_hit = c.Reserve(task_count, task_count * template_count) ? 1 : 0;
+  const size_t out_cells = masks ? (task_count * mask_words + 1) / 2 : task_count * template_count;
+  u.workspace_hit = c.Reserve(task_count, out_cells) ? 1 : 0;
   u.resident_bytes = KoptResidentBytes(ctx);
   if (usage) *usage = u;
   return true;
 }
 
 }  // namespace
+
+void EvalKoptRows(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type, uint32_t k,
+                  const ee_endpoint_matching* templates, uint32_t template_count, uint64_t generator_hash,
+                  size_t task_count, const KoptRows& rows, int64_t* costs, uint32_t* masks, ee_kopt_usage* usage) {
+  ctx.Activate();
+  if ((costs == nullptr) == (masks == nullptr)) {
+    throw std::invalid_argument("HIP k-opt needs exactly one of costs and masks");
+  }
+  KoptCache& c = ctx.kopt;
+  const auto validate = [&] {
+    if (rows.tasks != nullptr) ValidateTasks(n, k, rows.tasks, task_count);
+  };
+  // Where the caches look up to date, the launch goes out first, and the
+  // full comparison with them and the check of the rows run beside it: the
+  // kernel clamps node ids to the cached snapshot, and nothing reaches the
+  // caller before both passed.  Otherwise rows and caches come first.
+  const bool inputs = k >= 3 && k <= 5 && templates != nullptr && template_count > 0 && x != nullptr &&
+                      y != nullptr && n > 0 && task_count <= SIZE_MAX / template_count;
+  if (inputs && LooksResident(c, x, y, n, type, k, templates, template_count, generator_hash)) {
+    const auto check = [&] {
+      if (!SnapshotMatches(c, x, y, n, type)) return false;
+      if (rows.tasks == nullptr) return true;
+      try {
+        InParts(task_count, 1024, [&](size_t b, size_t e) { ValidateTasks(n, k, rows.tasks + b, e - b); });
+      } catch (const std::invalid_argument&) {
+        validate();  // the first refused row's message
+        throw;
+      }
+      return true;
+    };
+    if (RunDirect(ctx, n, type, k, template_count, task_count, rows, costs, masks, check, usage)) return;
+  }
+  validate();
+  CheckKoptInputs(x, y, n, type, k, templates, template_count, task_count);
+  const KoptHits hits = PrepareKoptCaches(ctx, x, y, n, type, k, templates, template_count, generator_hash);
+  RunDirect(ctx, n, type, k, template_count, task_count, rows, costs, masks, [] { return true; }, usage);
+  if (usage) {
+    usage->snapshot_hit = hits.snapshot ? 1 : 0;
+    usage->template_hit = hits.templates ? 1 : 0;
+  }
+}
 
 void EvalKoptCosts(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
                    uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
@@ -594,113 +685,10 @@ void EvalKoptCosts(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, 
     return;
   }
   if (tasks == nullptr || costs == nullptr) throw std::invalid_argument("HIP k-opt NULL buffer");
-  KoptCache& c = ctx.kopt;
-  // Where the caches look up to date, the launch goes out first, and the
-  // full comparison with them and the check of the rows run beside it: the
-  // kernel clamps node ids to the cached snapshot, and nothing reaches the
-  // caller before both passed.  Otherwise rows and caches come first.
-  const bool inputs = k >= 3 && k <= 5 && templates != nullptr && template_count > 0 && x != nullptr &&
-                      y != nullptr && n > 0 && task_count <= SIZE_MAX / template_count;
-  if (inputs && LooksResident(c, x, y, n, type, k, templates, template_count, generator_hash)) {
-    const auto check = [&] {
-      if (!SnapshotMatches(c, x, y, n, type)) return false;
-      try {
-        InParts(task_count, 1024, [&](size_t b, size_t e) { ValidateTasks(n, k, tasks + b, e - b); });
-      } catch (const std::invalid_argument&) {
-        ValidateTasks(n, k, tasks, task_count);  // the first refused row's message
-        throw;
-      }
-      return true;
-    };
-    if (RunDirect(ctx, n, type, k, template_count, tasks, task_count, costs, check, usage)) return;
-  }
-  ValidateTasks(n, k, tasks, task_count);
-  CheckKoptInputs(x, y, n, type, k, templates, template_count, task_count);
-  const KoptHits hits = PrepareKoptCaches(ctx, x, y, n, type, k, templates, template_count, generator_hash);
-  RunDirect(ctx, n, type, k, template_count, tasks, task_count, costs, [] { return true; }, usage);
-  if (usage) {
-    usage->snapshot_hit = hits.snapshot ? 1 : 0;
-    usage->template_hit = hits.templates ? 1 : 0;
-  }
-}
-
-void EvalKoptCostsFrom(Context& ctx, const int64_t* x, const int64_t* y, int32_t n, uint8_t type,
-                       uint32_t k, const ee_endpoint_matching* templates, uint32_t template_count,
-                       uint64_t generator_hash, size_t task_count, const KoptTaskSource& fill_tasks,
-                       bool sync_after_fill, int64_t* costs, uint32_t* masks, ee_kopt_usage* usage) {
-  ee_kopt_usage u{};
-  ctx.Activate();
-  if (task_count == 0) {
-    if (usage) *usage = u;
-    return;
-  }
-  CheckKoptInputs(x, y, n, type, k, templates, template_count, task_count);
-  if ((costs == nullptr) == (masks == nullptr)) {
-    throw std::invalid_argument("HIP k-opt needs exactly one of costs and masks");
-  }
-  const size_t cells = task_count * template_count;
-  const uint32_t mask_words = (template_count + 31) / 32;
-  KoptCache& c = ctx.kopt;
-  const KoptHits hits = PrepareKoptCaches(ctx, x, y, n, type, k, templates, template_count, generator_hash);
-
-  // workspace
-  // mask output needs task_count x mask_words words, held in the cost pool
-  const size_t out_cells = masks ? (task_count * mask_words + 1) / 2 : cells;
-  const bool workspace_hit = c.d_tasks.count() >= task_count && c.d_costs.count() >= out_cells;
-  if (c.d_tasks.count() < task_count) c.d_tasks.Allocate(Grow(c.d_tasks.count(), task_count), ctx.device);
-  if (c.d_costs.count() < out_cells) c.d_costs.Allocate(Grow(c.d_costs.count(), out_cells), ctx.device);
-
-  KoptInstance inst{};
-  inst.n = static_cast<uint32_t>(n);
-  inst.distance_type = type;
-  inst.near = c.near ? 1 : 0;
-  KoptSegment segment{0, k, 0, task_count, 0, 0, TileRows(ctx.kopt_tuning, k), 0};
-  const uint64_t n_tiles = KoptCountTiles(&segment, 1, ctx.kopt_tuning);
-  std::vector<KoptTile> tiles(n_tiles);
-  KoptLaunch a{};
-  KoptAssignTiles(&segment, 1, &inst, c.host_plans.data(), ctx.kopt_tuning, tiles.data(), &a);
-  // a one-segment launch derives its tiles from the kernel arguments
-  const bool descriptors = a.inline_count == 0;
-  if (descriptors && c.d_tiles.count() < n_tiles) c.d_tiles.Allocate(Grow(c.d_tiles.count(), n_tiles), ctx.device);
-  auto t0 = std::chrono::steady_clock::now();
-  fill_tasks(c.d_tasks.get());
-  if (descriptors) c.d_tiles.Upload(tiles.data(), n_tiles, ctx.stream);
-  if (sync_after_fill) ctx.Sync();
-  u.h2d_ms = MsSince(t0);
-
-  a.xy = c.d_xy.get();
-  a.tiles = c.d_tiles.get();
-  a.tasks = c.d_tasks.get();
-  a.plans = c.d_plans.get();
-  a.costs = c.d_costs.get();
-  if (masks) {
-    a.masks = reinterpret_cast<uint32_t*>(c.d_costs.get());
-    a.mask_words = mask_words;
-  }
-  bool present[3] = {false, false, false};
-  present[k - 3] = true;
-  const size_t shared = KoptPrepareLayout(&a, c.host_plans.data(), present, ctx.kopt_tuning, c.near);
-  t0 = std::chrono::steady_clock::now();
-  LaunchKopt(a, ctx.kopt_tuning, shared, ctx.stream);
-  ctx.Sync();
-  u.kernel_ms = MsSince(t0);
-
-  t0 = std::chrono::steady_clock::now();
-  if (masks) {
-    CheckHip(hipMemcpyAsync(masks, c.d_costs.get(), task_count * mask_words * sizeof(uint32_t),
-                            hipMemcpyDeviceToHost, ctx.stream),
-             "hipMemcpyAsync masks");
-  } else {
-    if (cells > c.d_costs.count()) throw std::logic_error("D2H beyond device buffer");
-    DownloadToCaller(ctx, costs, c.d_costs.get(), cells * sizeof(int64_t));
-  }
-  ctx.Sync();
-  u.d2h_ms = MsSince(t0);
-  u.snapshot_hit = hits.snapshot ? 1 : 0;
-  u.template_hit = hits.templates ? 1 : 0;
-  u.workspace_hit = workspace_hit ? 1 : 0;
-  u.resident_bytes = KoptResidentBytes(ctx);
-  if (usage) *usage = u;
+  KoptRows rows;
+  rows.tasks = tasks;
+  EvalKoptRows(ctx, x, y, n, type, k, templates, template_count, generator_hash, task_count, rows, costs, nullptr,
+               usage);
 }
 
 }  // namespace ee

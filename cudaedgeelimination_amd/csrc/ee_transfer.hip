@@ -75,21 +75,27 @@ void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t str
   }
 }
 
-// Groups of tiles, in order, on the host threads from kSerialCells up (below,
-// waking them costs more than it saves; the expansion of a large result
-// needs about twelve to keep pace with PCIe).
+void DirectIo::TakeTiles(size_t slot, uint64_t mark, hipStream_t stream, size_t tiles, size_t group,
+                         unsigned threads, const std::function<void(size_t, size_t)>& take) const {
+  ParallelFor((tiles + group - 1) / group, [&](size_t g) {
+    const size_t first = g * group, last = std::min(tiles, first + group);
+    for (size_t t = first; t < last; ++t) WaitTile(slot, t, mark, stream);
+    take(first, last);
+  }, threads);
+}
+
+// On the host threads from kSerialCells up (below, waking them costs more
+// than it saves; the expansion of a large result needs about twelve to keep
+// pace with PCIe).
 void DirectIo::TakeCells(size_t slot, uint64_t mark, hipStream_t stream, const uint32_t* lo, const uint8_t* hi,
                          size_t count, size_t tile_cells, int64_t* cells) const {
   constexpr size_t kGroupCells = 16384, kSerialCells = 65536;
   constexpr unsigned kThreads = 12;
-  const size_t tiles = (count + tile_cells - 1) / tile_cells;
-  const size_t group = std::max<size_t>(1, kGroupCells / tile_cells);
-  ParallelFor((tiles + group - 1) / group, [&](size_t g) {
-    const size_t first = g * group, last = std::min(tiles, first + group);
-    for (size_t t = first; t < last; ++t) WaitTile(slot, t, mark, stream);
+  TakeTiles(slot, mark, stream, (count + tile_cells - 1) / tile_cells, std::max<size_t>(1, kGroupCells / tile_cells),
+            count < kSerialCells ? 1 : kThreads, [&](size_t first, size_t last) {
     const size_t b = first * tile_cells, e = std::min(count, last * tile_cells);
     ExpandCells(lo + b, hi != nullptr ? hi + b : nullptr, e - b, cells + b);
-  }, count < kSerialCells ? 1 : kThreads);
+  });
 }
 
 // Half the bytes of a copy of the int64 cells (five eighths with high bytes)

@@ -311,7 +311,7 @@ ee_status ee_kopt_cursor_count(const ee_tour_view* tour, uint32_t k, uint64_t* c
  * EE_ERR_RUNTIME where a deleted cost sum overflows int64 or a selectable
  * position's cost is negative or out of the tour, as BuildKOptCostTask
  * throws; the positions are checked up front, not as the sets reach them.
- * usage->h2d_ms covers building the rows on the device. */
+ * usage->kernel_ms covers building the rows on the device. */
 ee_status ee_kopt_cursor_eval(ee_ctx* ctx, const int64_t* x, const int64_t* y, int32_t dimension,
                               uint8_t distance_type, const ee_tour_view* tour, uint32_t k,
                               const ee_endpoint_matching* templates, uint32_t template_count,

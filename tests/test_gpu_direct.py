@@ -119,3 +119,33 @@ def test_batch_download_ranges(ctx, box):
                          (5, slot + 1), (1, 2 * slot - 1), (9, 2 * slot + 3), (len(want) - 1, 1), (4, 0)):
         assert np.array_equal(batch.download(first, count), want[first:first + count]), (first, count)
     batch.close()
+
+
+@pytest.mark.parametrize("box", [1_000_000, 1 << 30])
+@pytest.mark.parametrize("output", ["costs", "masks"])
+@pytest.mark.parametrize("k, rows", [(3, 1), (3, 31), (3, 1_225), (4, 7), (4, 9), (4, 18_424), (5, 1), (5, 9),
+                                     (5, 255), (5, 257), (5, 14_001), (5, 44_000)])
+def test_made_rows_match_oracle(ctx, k, rows, output, box):
+    """Rows made by the wavefronts that evaluate them, at the edges of tiles,
+    of the host's groups of 256 rows, and of launches (several slots)."""
+    if output == "costs" and rows > 14_001:
+        rows = 9_400  # three launches of cells
+    say(f"made rows k={k} rows={rows} {output} box={box}")
+    g = graph(rows + k, 900, CEIL_2D if rows % 2 else EUC_2D, box)
+    tour = W.tour_context(rows, g, 120, 51)
+    table = backend.build_kopt_reconnect_table(k)
+    first = backend.kopt_cursor_count(tour, k) - rows if rows < 1_000 else 0
+    want, positions = O.cursor_tasks(tour.tour, tour.edge_costs, tour.selectable, k, first, rows)
+    cells, _, _ = O.kopt_costs(g.x, g.y, g.distance_type, k, want)
+    for _ in range(2):  # caches empty, then up to date
+        block = backend.evaluate_kopt_cursor_cuda(g, table, tour, k, first, rows, output, ctx)
+        assert np.array_equal(block.tasks["port_nodes"], want["port_nodes"])
+        assert np.array_equal(block.tasks["deleted_cost"], want["deleted_cost"])
+        assert np.array_equal(block.positions, positions)
+        if output == "costs":
+            assert np.array_equal(block.costs, cells)
+        else:
+            bits = np.unpackbits(block.masks.view(np.uint8), axis=1, bitorder="little")
+            improving = cells.reshape(rows, -1) < want["deleted_cost"][:, None]
+            assert np.array_equal(bits[:, :improving.shape[1]].astype(bool), improving)
+            assert not bits[:, improving.shape[1]:].any()
