@@ -250,7 +250,7 @@ def evaluate_ht_hamilton_replies_cuda(graph: GraphSnapshot, target, centers,
     (center, first, second), usage)."""
     ctx = _ctx(ctx)
     centers = np.ascontiguousarray(centers, dtype=np.int32)
-    offsets = np.zeros(len(centers) + 1, dtype=np.uint64)
+    offsets = np.empty(len(centers) + 1, dtype=np.uint64)
     total, usage = C.c_uint64(), _lib.HtUsage()
     view = graph.view()
     # the reply count is known after the device's count pass: size the

@@ -13,15 +13,24 @@
 // the center edge's exact distance and its 2-opt verdict into LDS (the
 // reference recomputes both per pair); then each lane takes one neighbour
 // pair (pairs numbered in the reference's first-major order), and a ballot
-// plus a popcount prefix place the surviving pairs in order.  The count and
-// write passes run the same wave body.
+// plus a popcount prefix place the surviving pairs in order.
+//
+// Two forms of the output.  Where every row is short (kBitsDegree), one pass
+// writes each pair's verdict as a bit into host memory, and the host writes
+// the replies from the bits into the caller's buffer: a reply is its center
+// and two neighbours, 12 bytes that the host has, against one bit.
+// Otherwise a count pass, an offset scan and a write pass leave the replies
+// on the device, which then never holds more than the replies themselves.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 #include "ee_exact.h"
+#include "ee_jvhost.h"
 #include "ee_runtime.h"
 
 namespace ee {
@@ -146,6 +155,145 @@ __global__ __launch_bounds__(kHtBlock) void HtHamiltonKernel(
     if (kWrite) out += __popcll(ballot);
   }
   if (!kWrite && lane == 0) counts[item] = found;
+}
+
+// Rows of up to this many neighbours (2,016 pairs in LDS, then up to 130,816
+// recomputed per pair) take the verdict bits, if all centers' words fit
+// kBitsBytes of host memory.
+constexpr uint32_t kBitsDegree = 512;
+constexpr size_t kBitsBytes = size_t{32} << 20;
+
+// A neighbour of the center under test: what the pair test needs of it.  x
+// and y are the low words on near snapshots (differences stay exact).
+template <bool kNear> struct HtRow {
+  int64_t cost;
+  typename std::conditional<kNear, uint32_t, int64_t>::type x, y;
+  int32_t node;
+  int32_t survives;
+};
+
+template <bool kNear>
+__device__ inline int64_t RowDist(const HtRow<kNear>& a, const HtRow<kNear>& b, int type) {
+  if constexpr (kNear) {
+    return ExactDistanceNear(static_cast<int32_t>(a.x - b.x), static_cast<int32_t>(a.y - b.y), type);
+  } else {
+    return ExactDistance(a.x, a.y, b.x, b.y, type);
+  }
+}
+
+// Neighbours per center in a wavefront's first phase, and its centers.
+constexpr uint32_t kVerdictGroup = 16;
+constexpr uint32_t kVerdictCenters = 64 / kVerdictGroup;
+
+// Verdict bits of each center's pairs, `stride` words per center (zero past
+// its pairs), and their counts.  A wavefront takes 4 consecutive centers, so
+// its reads of centers and writes of words and counts are whole stretches of
+// host memory.  The centers gather their neighbours on 16 lanes each (rows
+// of up to 16, the usual case; otherwise they take the wavefront one by one),
+// then each center's pairs take the 64 lanes, out of LDS.  Bound by those
+// gathers and the pair arithmetic: 41 us for the 30,000-node graph's 1.56
+// million pairs.  One center per wavefront, reading its id and writing its
+// words over PCIe by itself, took 64 us; 8 and 16 centers 41 and 50 us, and
+// 7 and 19 us more where few centers leave the chip to single wavefronts.
+template <bool kNear>
+__global__ __launch_bounds__(kHtBlock) void HtVerdictKernel(
+    const longlong2* __restrict__ xy, const int32_t* __restrict__ row_offsets,
+    const int32_t* __restrict__ neighbors, int32_t nodes, int type, int32_t tu, int32_t tv,
+    const int32_t* __restrict__ centers, uint32_t center_count, uint32_t stride, uint64_t* __restrict__ bits,
+    uint32_t* __restrict__ counts) {
+  __shared__ HtRow<kNear> rows[kHtWaves][kHtLdsNeighbors];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t first = (blockIdx.x * kHtWaves + wave) * kVerdictCenters;
+  if (first >= center_count) return;  // whole wavefronts leave together
+  const uint32_t here = min(kVerdictCenters, center_count - first);
+  HtRow<kNear>* const mine = rows[wave];
+  const int64_t target_cost = Dist<kNear>(xy, tu, tv, type);
+  // lane i < here: center i of the wavefront, its row (empty for an id out of
+  // range: the host refuses the call) and its distance to the target's ends
+  int32_t my_center = 0, my_begin = 0, my_degree = 0;
+  int64_t my_target = 0;
+  if (lane < here) {
+    const int32_t c = centers[first + lane];
+    if (static_cast<uint32_t>(c) < static_cast<uint32_t>(nodes)) {
+      my_center = c;
+      my_begin = row_offsets[c];
+      my_degree = row_offsets[c + 1] - my_begin;
+      my_target = Dist<kNear>(xy, tu, c, type) + Dist<kNear>(xy, tv, c, type);
+    }
+  }
+  const auto neighbor = [&](int32_t c, int32_t begin, uint32_t i) {
+    HtRow<kNear> r;
+    r.node = neighbors[begin + static_cast<int32_t>(i)];
+    const longlong2 p = xy[r.node];
+    r.x = static_cast<decltype(r.x)>(p.x);
+    r.y = static_cast<decltype(r.y)>(p.y);
+    r.cost = Dist<kNear>(xy, c, r.node, type);
+    r.survives = Survives<kNear>(xy, tu, tv, target_cost, c, r.node, r.cost, type) ? 1 : 0;
+    return r;
+  };
+  const auto lds = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  uint64_t word = 0;       // lane l: word l of the stretch being filled
+  uint32_t at = 0;         // words of the wavefront so far
+  uint32_t my_count = 0;   // lane i: surviving pairs of center i
+  uint64_t* const out = bits + static_cast<uint64_t>(first) * stride;
+  const uint32_t q = lane / kVerdictGroup;
+  const int32_t q_degree = __shfl(my_degree, static_cast<int>(q));
+  const bool together = __ballot(q_degree > static_cast<int32_t>(kVerdictGroup)) == 0;
+  if (together) {
+    const int32_t c = __shfl(my_center, static_cast<int>(q)), begin = __shfl(my_begin, static_cast<int>(q));
+    const uint32_t i = lane % kVerdictGroup;
+    if (static_cast<int32_t>(i) < q_degree) mine[lane] = neighbor(c, begin, i);
+    lds();
+  }
+  for (uint32_t k = 0; k < here; ++k) {  // uniform
+    const int32_t c = __builtin_amdgcn_readlane(my_center, static_cast<int>(k));
+    const int32_t begin = __builtin_amdgcn_readlane(my_begin, static_cast<int>(k));
+    const uint32_t d = static_cast<uint32_t>(__builtin_amdgcn_readlane(my_degree, static_cast<int>(k)));
+    const int64_t center_target = __shfl(static_cast<long long>(my_target), static_cast<int>(k));
+    const bool cached = d <= kHtLdsNeighbors;
+    const HtRow<kNear>* row = mine + (together ? k * kVerdictGroup : 0);
+    if (!together) {
+      if (cached && lane < d) mine[lane] = neighbor(c, begin, lane);
+      lds();
+    }
+    const uint32_t pairs = d < 2 ? 0 : d * (d - 1) / 2;
+    uint32_t found = 0;
+    for (uint32_t w = 0; w < stride; ++w) {
+      const uint32_t p = w * 64 + lane;
+      bool keep = false;
+      if (p < pairs) {
+        // row i of pair p: the root estimate (its argument is exact in
+        // float), then exact corrections
+        const float b = static_cast<float>(2 * d - 1);
+        uint32_t i = static_cast<uint32_t>(fmaxf(0.0f, (b - sqrtf(b * b - 8.0f * static_cast<float>(p))) * 0.5f));
+        if (i > d - 2) i = d - 2;
+        while (i > 0 && i * (2 * d - i - 1) / 2 > p) --i;
+        while (i + 1 <= d - 2 && (i + 1) * (2 * d - i - 2) / 2 <= p) ++i;
+        const uint32_t j = p - i * (2 * d - i - 1) / 2 + i + 1;
+        const HtRow<kNear> f = cached ? row[i] : neighbor(c, begin, i);
+        const HtRow<kNear> s = cached ? row[j] : neighbor(c, begin, j);
+        const bool is_target = min(f.node, s.node) == tu && max(f.node, s.node) == tv;
+        if (!is_target && f.survives && s.survives) {
+          const int64_t original = target_cost + f.cost + s.cost;
+          const int64_t replacement = RowDist<kNear>(f, s, type) + center_target;
+          keep = original <= replacement;
+        }
+      }
+      const uint64_t ballot = __ballot(keep);
+      found += static_cast<uint32_t>(__popcll(ballot));
+      if (lane == (at & 63u)) word = ballot;
+      ++at;
+      if ((at & 63u) == 0) out[at - 64 + lane] = word;  // uniform
+    }
+    if (lane == k) my_count = found;
+    if (!together) lds();  // the row is read before the next one replaces it
+  }
+  if (lane < (at & 63u)) out[(at & ~63u) + lane] = word;
+  if (lane < here) counts[first + lane] = my_count;
 }
 
 // chunk_sums[c] = counts of chunk c (kScanChunk centers), one workgroup per
@@ -281,25 +429,50 @@ void ValidateHtGraph(const ee_graph_view& g) {
   }
 }
 
-// Keeps the device copy of the snapshot.  A snapshot equal to the resident
-// one (coordinates, CSR and active flags) passed the HT checks when it was
-// uploaded, so only a new one is checked (ValidateHtGraph) and uploaded.
-bool PrepareHtGraph(Context& ctx, const ee_graph_view& g) {
+// Whether the resident snapshot is this one (coordinates, CSR and active
+// flags); it then passed the HT checks when it was uploaded.
+bool HtGraphMatches(const HtCache& c, const ee_graph_view& g) {
+  const size_t n = static_cast<size_t>(g.dimension), m = static_cast<size_t>(g.edge_count);
+  if (!c.valid || c.dimension != g.dimension || c.distance_type != g.distance_type || c.active.size() != m ||
+      c.row_offsets.size() != n + 1 || std::memcmp(c.row_offsets.data(), g.row_offsets, (n + 1) * 4) != 0) {
+    return false;
+  }
+  const struct {
+    const void *cached, *given;
+    size_t bytes;
+  } arrays[] = {{c.x.data(), g.x, n * 8},
+                {c.y.data(), g.y, n * 8},
+                {c.neighbors.data(), g.neighbors, c.neighbors.size() * 4},
+                {c.active.data(), g.edge_active, m}};
+  // in pieces of 64 KiB; large snapshots on four host threads
+  constexpr size_t kPiece = size_t{64} << 10;
+  size_t pieces = 0;
+  for (const auto& a : arrays) pieces += (a.bytes + kPiece - 1) / kPiece;
+  std::atomic<bool> equal{true};
+  ParallelFor(pieces, [&](size_t i) {
+    for (const auto& a : arrays) {
+      const size_t count = (a.bytes + kPiece - 1) / kPiece;
+      if (i < count) {
+        const size_t at = i * kPiece;
+        if (std::memcmp(static_cast<const char*>(a.cached) + at, static_cast<const char*>(a.given) + at,
+                        std::min(kPiece, a.bytes - at)) != 0) {
+          equal = false;
+        }
+        return;
+      }
+      i -= count;
+    }
+  }, pieces < 8 ? 1 : 4);
+  return equal;
+}
+
+// Keeps a device copy of a checked snapshot.
+void UploadHtGraph(Context& ctx, const ee_graph_view& g) {
   HtCache& c = ctx.ht;
-  const size_t n = static_cast<size_t>(g.dimension);
-  const size_t m = static_cast<size_t>(g.edge_count);
-  const bool hit = c.valid && c.dimension == g.dimension && c.distance_type == g.distance_type &&
-                   c.active.size() == m && c.row_offsets.size() == n + 1 &&
-                   std::memcmp(c.row_offsets.data(), g.row_offsets, (n + 1) * 4) == 0 &&
-                   std::memcmp(c.x.data(), g.x, n * 8) == 0 &&
-                   std::memcmp(c.y.data(), g.y, n * 8) == 0 &&
-                   (c.neighbors.empty() ||
-                    std::memcmp(c.neighbors.data(), g.neighbors, c.neighbors.size() * 4) == 0) &&
-                   (m == 0 || std::memcmp(c.active.data(), g.edge_active, m) == 0);
-  if (hit) return true;
-  ValidateHtGraph(g);
+  const size_t n = static_cast<size_t>(g.dimension), m = static_cast<size_t>(g.edge_count);
   const size_t a = static_cast<size_t>(g.row_offsets[g.dimension]);
   c.valid = false;
+  c.last_kind = 0;  // verdict bits go with their snapshot
   std::vector<longlong2> xy(n);
   for (size_t i = 0; i < n; ++i) xy[i] = make_longlong2(g.x[i], g.y[i]);
   c.d_xy.Allocate(n, ctx.device);
@@ -315,10 +488,13 @@ bool PrepareHtGraph(Context& ctx, const ee_graph_view& g) {
   c.neighbors.assign(g.neighbors, g.neighbors + a);
   c.active.assign(g.edge_active, g.edge_active + m);
   c.near = NearExtent(g.x, g.y, g.dimension);
+  c.max_degree = 0;
+  for (size_t v = 0; v < n; ++v) {
+    c.max_degree = std::max(c.max_degree, static_cast<uint32_t>(g.row_offsets[v + 1] - g.row_offsets[v]));
+  }
   c.dimension = g.dimension;
   c.distance_type = g.distance_type;
   c.valid = true;
-  return false;
 }
 
 template <typename T> bool Reserve(DeviceArray<T>& a, size_t count, int device) {
@@ -328,8 +504,150 @@ template <typename T> bool Reserve(DeviceArray<T>& a, size_t count, int device) 
 }
 
 uint64_t HtResidentBytes(const HtCache& c) {
-  return c.d_xy.bytes() + c.d_row_offsets.bytes() + c.d_neighbors.bytes() + c.d_items.bytes() +
+  uint64_t host = 0;
+  for (const HtCache::Verdicts& v : c.verdicts) host += v.centers.count() * 4 + v.bits.count() * 8;
+  return host + c.d_xy.bytes() + c.d_row_offsets.bytes() + c.d_neighbors.bytes() + c.d_items.bytes() +
          c.d_counts.bytes() + c.d_offsets.bytes() + c.d_chunk_sums.bytes() + c.d_replies.bytes();
+}
+
+// Replies of centers [b, e) from their verdict bits, in order, to `out`.
+int32_t* WriteReplies(const HtCache& c, const HtCache::Verdicts& v, size_t b, size_t e, int32_t* out) {
+  for (size_t item = b; item < e; ++item) {
+    const int32_t center = v.centers.get()[item];
+    const int32_t* row = c.neighbors.data() + c.row_offsets[static_cast<size_t>(center)];
+    const uint32_t d = static_cast<uint32_t>(c.row_offsets[static_cast<size_t>(center) + 1] -
+                                             c.row_offsets[static_cast<size_t>(center)]);
+    if (d < 2) continue;
+    const uint64_t* bits = v.bits.get() + item * v.stride;
+    const uint32_t pairs = d * (d - 1) / 2;
+    bool all = true;  // the usual case: every pair survives
+    for (uint32_t w = 0; w * 64 < pairs; ++w) {
+      const uint32_t left = pairs - w * 64;
+      all = all && bits[w] == (left >= 64 ? ~uint64_t{0} : (uint64_t{1} << left) - 1);
+    }
+    uint32_t p = 0;
+    for (uint32_t i = 0; i + 1 < d; ++i) {
+      for (uint32_t j = i + 1; j < d; ++j, ++p) {
+        if (!all && ((bits[p / 64] >> (p % 64)) & 1u) == 0) continue;
+        out[0] = center;
+        out[1] = row[i];
+        out[2] = row[j];
+        out += 3;
+      }
+    }
+  }
+  return out;
+}
+
+// Centers per group of the reply counts and of the host's work.
+constexpr size_t kGroupCenters = 256;
+// Host threads: writing 19 MB of replies takes 12 about 0.15 ms.
+constexpr unsigned kReplyThreads = 12;
+
+// Replies [first, first + count) of the last verdicts.
+void CopyVerdictReplies(const HtCache& c, uint64_t first, uint64_t count, int32_t* out) {
+  const HtCache::Verdicts& v = c.verdicts[c.current];
+  const auto group_of = [&](uint64_t reply) {
+    return static_cast<size_t>(std::upper_bound(v.group_first.begin(), v.group_first.end(), reply) -
+                               v.group_first.begin()) - 1;
+  };
+  const size_t g0 = group_of(first), g1 = group_of(first + count - 1) + 1;
+  ParallelFor(g1 - g0, [&](size_t i) {
+    const size_t g = g0 + i;
+    const size_t b = g * kGroupCenters, e = std::min(v.count, b + kGroupCenters);
+    const uint64_t from = v.group_first[g], to = v.group_first[g + 1];
+    if (from >= first && to <= first + count) {
+      WriteReplies(c, v, b, e, out + 3 * (from - first));
+      return;
+    }
+    std::vector<int32_t> whole(3 * (to - from));  // a group the range cuts
+    WriteReplies(c, v, b, e, whole.data());
+    const uint64_t lo = std::max(from, first), hi = std::min(to, first + count);
+    std::copy(whole.begin() + 3 * (lo - from), whole.begin() + 3 * (hi - from), out + 3 * (lo - first));
+  }, g1 - g0 < 8 ? 1 : kReplyThreads);
+}
+
+void CheckHamilton(const ee_graph_view& g, int32_t tu, int32_t tv, const int32_t* centers, size_t count) {
+  if (tu < 0 || tv >= g.dimension || tu == tv || !RowHas(g, tu, tv)) {
+    throw std::invalid_argument("HT Hamilton replies: the target is not an active edge");
+  }
+  bool bad = false;
+  for (size_t i = 0; i < count; ++i) {
+    const int32_t c = centers[i];
+    bad |= static_cast<uint32_t>(c) >= static_cast<uint32_t>(g.dimension) || c == tu || c == tv;
+  }
+  if (bad) throw std::invalid_argument("HT Hamilton replies: invalid center");
+}
+
+// Whether the call's verdict bits fit host memory, on the resident snapshot.
+size_t VerdictStride(const HtCache& c) {
+  const size_t d = c.max_degree;
+  return std::max<size_t>(1, (d * (d - std::min<size_t>(d, 1)) / 2 + 63) / 64);
+}
+bool TakesVerdicts(const HtCache& c, size_t count) {
+  return c.max_degree <= kBitsDegree && count <= UINT32_MAX && count * VerdictStride(c) * 8 <= kBitsBytes;
+}
+
+// Starts the verdict pass on the resident snapshot into the buffer that does
+// not hold the last call's; returns whether the buffers had room.
+bool LaunchVerdicts(Context& ctx, int type, int32_t tu, int32_t tv, const int32_t* centers, size_t count) {
+  HtCache& c = ctx.ht;
+  HtCache::Verdicts& v = c.verdicts[c.current ^ 1];
+  v.stride = VerdictStride(c);
+  v.count = count;
+  const bool room = v.centers.count() >= 2 * count && v.bits.count() >= count * v.stride;
+  for (HtCache::Verdicts& b : c.verdicts) {
+    if (&b != &v && c.last_kind == 1 && c.last_bits) continue;  // growing would drop the last call's replies
+    b.centers.Reserve(Grow(b.centers.count(), 2 * count));
+    b.bits.Reserve(Grow(b.bits.count(), count * v.stride));
+  }
+  std::memcpy(v.centers.get(), centers, count * sizeof(int32_t));
+  const auto kernel = c.near ? HtVerdictKernel<true> : HtVerdictKernel<false>;
+  const size_t per_block = kHtWaves * kVerdictCenters;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((count + per_block - 1) / per_block)), dim3(kHtBlock), 0,
+                     ctx.stream, c.d_xy.get(), c.d_row_offsets.get(), c.d_neighbors.get(), c.dimension, type, tu, tv,
+                     v.centers.device(), static_cast<uint32_t>(count), static_cast<uint32_t>(v.stride),
+                     v.bits.device(), reinterpret_cast<uint32_t*>(v.centers.device() + count));
+  CheckHip(hipGetLastError(), "HtVerdictKernel launch");
+  return room;
+}
+
+// Offsets and group totals from the finished verdict pass's counts.
+uint64_t CountVerdicts(HtCache& c, uint64_t* offsets) {
+  HtCache::Verdicts& v = c.verdicts[c.current ^ 1];
+  const uint32_t* counts = reinterpret_cast<const uint32_t*>(v.centers.get() + v.count);
+  const size_t groups = (v.count + kGroupCenters - 1) / kGroupCenters;
+  v.group_first.assign(groups + 1, 0);
+  uint64_t run = 0;
+  for (size_t g = 0; g < groups; ++g) {
+    for (size_t i = g * kGroupCenters, e = std::min(v.count, i + kGroupCenters); i < e; ++i) {
+      run += counts[i];
+      offsets[i + 1] = run;
+    }
+    v.group_first[g + 1] = run;
+  }
+  return run;
+}
+
+// As HamiltonReplies below, by verdict bits.  started: the pass is under way.
+void VerdictReplies(Context& ctx, const ee_graph_view& g, int32_t tu, int32_t tv, const int32_t* centers,
+                    size_t count, bool started, uint64_t* offsets, ee_ht_neighbor_pair* replies, uint64_t capacity,
+                    uint64_t* total, ee_ht_usage* u) {
+  HtCache& c = ctx.ht;
+  auto t0 = std::chrono::steady_clock::now();
+  if (!started) u->workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count) ? 1 : 0;
+  ctx.Sync();
+  *total = CountVerdicts(c, offsets);
+  u->kernel_ms = MsSince(t0);
+  c.current ^= 1;
+  c.last_kind = 1;
+  c.last_bits = true;
+  c.last_total = *total;
+  t0 = std::chrono::steady_clock::now();
+  const uint64_t copy = std::min(*total, capacity);
+  if (copy > 0) CopyVerdictReplies(c, 0, copy, reinterpret_cast<int32_t*>(replies));
+  u->d2h_ms = MsSince(t0);
+  u->resident_bytes = HtResidentBytes(c);
 }
 
 void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u, int32_t target_v,
@@ -345,16 +663,32 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
     throw std::invalid_argument("HT Hamilton replies: NULL argument");
   }
   auto t0 = std::chrono::steady_clock::now();
-  u.graph_hit = PrepareHtGraph(ctx, g) ? 1 : 0;  // checks a new snapshot
   const int32_t tu = std::min(target_u, target_v), tv = std::max(target_u, target_v);
-  if (tu < 0 || tv >= g.dimension || tu == tv || !RowHas(g, tu, tv)) {
-    throw std::invalid_argument("HT Hamilton replies: the target is not an active edge");
+  // Where the snapshot looks like the resident one, the verdict pass goes out
+  // first and the comparison runs beside it (the kernel leaves centers out of
+  // range alone; nothing reaches the caller before the checks).
+  const bool likely = count > 0 && tu >= 0 && tu != tv && tv < g.dimension && ctx.ht.valid &&
+                      ctx.ht.dimension == g.dimension && ctx.ht.distance_type == g.distance_type &&
+                      ctx.ht.active.size() == static_cast<size_t>(g.edge_count) &&
+                      std::memcmp(ctx.ht.x.data(), g.x, std::min<size_t>(ctx.ht.x.size(), 64) * 8) == 0 &&
+                      TakesVerdicts(ctx.ht, count);
+  bool started = false;
+  if (likely) {
+    u.workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count) ? 1 : 0;
+    started = true;
   }
-  for (size_t i = 0; i < count; ++i) {
-    const int32_t c = centers[i];
-    if (c < 0 || c >= g.dimension || c == tu || c == tv) {
-      throw std::invalid_argument("HT Hamilton replies: invalid center");
-    }
+  try {
+    u.graph_hit = HtGraphMatches(ctx.ht, g) ? 1 : 0;
+    if (!u.graph_hit) ValidateHtGraph(g);
+    CheckHamilton(g, tu, tv, centers, count);
+  } catch (...) {
+    if (started) static_cast<void>(hipStreamSynchronize(ctx.stream));
+    throw;
+  }
+  if (!u.graph_hit) {
+    if (started) ctx.Sync();
+    started = false;
+    UploadHtGraph(ctx, g);
   }
   offsets[0] = 0;
   *total = 0;
@@ -362,6 +696,12 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
   c.last_kind = 0;
   c.last_total = 0;
   if (count == 0) {
+    if (usage) *usage = u;
+    return;
+  }
+  if (started || TakesVerdicts(c, count)) {
+    u.h2d_ms = MsSince(t0);
+    VerdictReplies(ctx, g, tu, tv, centers, count, started, offsets, replies, capacity, total, &u);
     if (usage) *usage = u;
     return;
   }
@@ -412,6 +752,7 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
   ctx.Sync();
   u.kernel_ms = MsSince(t0);
   c.last_kind = 1;
+  c.last_bits = false;
   c.last_total = *total;
 
   t0 = std::chrono::steady_clock::now();
@@ -431,6 +772,10 @@ void CopyReplies(Context& ctx, uint64_t first, uint64_t count, void* out) {
   }
   if (count == 0) return;
   if (out == nullptr) throw std::invalid_argument("HT copy replies: NULL buffer");
+  if (c.last_kind == 1 && c.last_bits) {
+    CopyVerdictReplies(c, first, count, static_cast<int32_t*>(out));
+    return;
+  }
   ctx.Activate();
   const size_t record = c.last_kind == 1 ? sizeof(ee_ht_neighbor_pair) : sizeof(ee_node_edge);
   DownloadToCaller(ctx, out, reinterpret_cast<const char*>(c.d_replies.get()) + first * record, count * record);
@@ -448,7 +793,8 @@ void EndReplies(Context& ctx, const ee_graph_view* graph, const ee_ht_end_task* 
     throw std::invalid_argument("HT end replies: NULL argument");
   }
   auto t0 = std::chrono::steady_clock::now();
-  u.graph_hit = PrepareHtGraph(ctx, g) ? 1 : 0;  // checks a new snapshot
+  u.graph_hit = HtGraphMatches(ctx.ht, g) ? 1 : 0;
+  if (!u.graph_hit) ValidateHtGraph(g);
   offsets[0] = 0;
   for (size_t i = 0; i < count; ++i) {
     const int32_t e = tasks[i].endpoint, in = tasks[i].internal_neighbor;
@@ -459,6 +805,7 @@ void EndReplies(Context& ctx, const ee_graph_view* graph, const ee_ht_end_task* 
     offsets[i + 1] = offsets[i] + static_cast<uint64_t>(g.row_offsets[e + 1] - g.row_offsets[e] - 1);
   }
   *total = offsets[count];
+  if (!u.graph_hit) UploadHtGraph(ctx, g);
   HtCache& c = ctx.ht;
   c.last_kind = 0;
   c.last_total = 0;

@@ -71,6 +71,12 @@ template <typename T> class Pinned {
   }
   T* get() { return ptr_; }
   const T* get() const { return ptr_; }
+  // The address kernels use.
+  T* device() const {
+    void* d = nullptr;
+    CheckHip(hipHostGetDevicePointer(&d, ptr_, 0), "hipHostGetDevicePointer");
+    return static_cast<T*>(d);
+  }
   size_t count() const { return count_; }
 
  private:
@@ -272,6 +278,7 @@ struct HtCache {
   std::vector<int32_t> row_offsets, neighbors;
   std::vector<uint8_t> active;  // the snapshot passed the HT checks with these flags
   bool near = false;            // NearExtent: the FP64 distance path applies
+  uint32_t max_degree = 0;
   DeviceArray<longlong2> d_xy;
   DeviceArray<int32_t> d_row_offsets, d_neighbors;
   DeviceArray<int32_t> d_items;      // centers, or (endpoint, internal) task pairs
@@ -281,6 +288,18 @@ struct HtCache {
   DeviceArray<int32_t> d_replies;    // triples or pairs, exactly the last call's replies
   int last_kind = 0;                 // last completed call: 1 Hamilton, 2 end replies
   uint64_t last_total = 0;           // its reply count
+  // Hamilton replies as verdict bits: per center `stride` words in host
+  // memory, bit p set where pair p survives.  The call under way uses the
+  // other buffer, so that a refused one leaves the last one's replies.
+  struct Verdicts {
+    Pinned<int32_t> centers;  // the centers, then their reply counts
+    Pinned<uint64_t> bits;
+    size_t count = 0, stride = 0;
+    std::vector<uint64_t> group_first;  // replies before each group of centers, and in all
+  };
+  Verdicts verdicts[2];
+  int current = 0;
+  bool last_bits = false;            // the last Hamilton replies are verdicts[current]
 };
 
 struct Context {

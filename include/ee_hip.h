@@ -246,9 +246,10 @@ typedef struct {
  * (src/cpu/hamilton_tutte.cpp:230-262).  The target may be given in either
  * order.  offsets receives center_count + 1 entries (center i's replies are
  * [offsets[i], offsets[i+1])), replies the first min(*total, capacity)
- * replies (ee_ht_copy_replies copies the rest), *total their count.  A count
- * pass runs first, so the device holds exactly *total replies, never the
- * sum over centers of C(degree, 2).  The snapshot must pass the reference's HT graph checks
+ * replies (ee_ht_copy_replies copies the rest), *total their count.  What is
+ * kept for ee_ht_copy_replies is one bit per neighbour pair where every row
+ * is short (at most 512 entries, 32 MiB of bits in all), else, after a count
+ * pass, exactly *total replies on the device.  The snapshot must pass the reference's HT graph checks
  * (ht_replies.cu:521-553): a symmetric CSR of exactly the active edges,
  * rows strictly ascending. */
 ee_status ee_ht_hamilton_replies(ee_ctx* ctx, const ee_graph_view* graph, int32_t target_u,
@@ -265,7 +266,7 @@ ee_status ee_ht_end_replies(ee_ctx* ctx, const ee_graph_view* graph, const ee_ht
 /* Copies replies [first, first + count) of the context's last completed
  * ee_ht_hamilton_replies (12-byte ee_ht_neighbor_pair records) or
  * ee_ht_end_replies (8-byte ee_node_edge records) call into `replies`; they
- * stay on the device until the next reply call.  A caller that does not know
+ * are kept until the next completed reply call.  A caller that does not know
  * the reply count beforehand passes capacity 0 (or a guess) to the reply
  * call, sizes its buffer from *total and copies the rest here, as the
  * reference sizes its vector from the scanned offsets

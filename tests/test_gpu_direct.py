@@ -149,3 +149,53 @@ def test_made_rows_match_oracle(ctx, k, rows, output, box):
             improving = cells.reshape(rows, -1) < want["deleted_cost"][:, None]
             assert np.array_equal(bits[:, :improving.shape[1]].astype(bool), improving)
             assert not bits[:, improving.shape[1]:].any()
+
+
+def star(n, hub_degree, seed=3):
+    """A k-NN graph with one hub joined to `hub_degree` further nodes."""
+    g = graph(seed, n, EUC_2D, 1_000_000)
+    have = set(zip(g.edge_u.tolist(), g.edge_v.tolist()))
+    extra = [(0, v) for v in range(1, n) if (0, v) not in have][:hub_degree]
+    u = np.concatenate([g.edge_u, [e[0] for e in extra]]).astype(np.int32)
+    v = np.concatenate([g.edge_v, [e[1] for e in extra]]).astype(np.int32)
+    order = np.lexsort((v, u))
+    return type(g).from_edges(g.x, g.y, EUC_2D, u[order], v[order])
+
+
+@pytest.mark.parametrize("degree", [55, 90, 500, 700])
+def test_hamilton_verdicts(ctx, degree):
+    """Hub rows below and above the 64 neighbours cached in LDS and the 512
+    that take verdict bits; replies copied in ranges that cut the groups of
+    256 centers; a refused call leaves the last call's replies."""
+    say(f"ht verdicts hub degree {degree}")
+    g = star(800, degree)
+    backend.clear_ht_reply_cuda_cache(ctx)
+    e = len(g.edge_u) // 2
+    target = (int(g.edge_u[e]), int(g.edge_v[e]))
+    centers = np.setdiff1d(np.arange(g.dimension, dtype=np.int32), np.array(target, np.int32))
+    deg = np.diff(g.row_offsets).astype(np.int64)[centers]
+    woff, wrep = O.ht_hamilton_replies(O.OGraph.from_snapshot(g), target, centers,
+                                       int((deg * (deg - 1) // 2).sum()))
+    for _ in range(2):
+        off, rep, _ = backend.evaluate_ht_hamilton_replies_cuda(g, target, centers, ctx)
+        assert np.array_equal(off, woff) and np.array_equal(rep, wrep)
+    total = len(wrep)
+    for first, count in ((0, 1), (1, 7), (total // 3, total // 2), (total - 1, 1), (5, 0)):
+        part = np.full((count, 3), -1, np.int32)
+        _lib.check(_lib.lib().ee_ht_copy_replies(ctx.handle, first, count, _lib.ptr(part) if count else None))
+        assert np.array_equal(part, wrep[first:first + count])
+    with pytest.raises(_lib.InvalidArgument):
+        backend.evaluate_ht_hamilton_replies_cuda(g, target, np.array([0, target[1]], np.int32), ctx)
+    with pytest.raises(_lib.InvalidArgument):
+        backend.evaluate_ht_hamilton_replies_cuda(g, target, np.array([0, g.dimension], np.int32), ctx)
+    part = np.empty((total, 3), np.int32)
+    _lib.check(_lib.lib().ee_ht_copy_replies(ctx.handle, 0, total, _lib.ptr(part)))
+    assert np.array_equal(part, wrep)
+    # the same sizes with one node moved: not the resident snapshot
+    moved = g.copy()
+    moved.x[g.dimension - 1] += 5000
+    moved = type(g).from_edges(moved.x, moved.y, EUC_2D, moved.edge_u, moved.edge_v)
+    off, rep, usage = backend.evaluate_ht_hamilton_replies_cuda(moved, target, centers, ctx)
+    woff, wrep = O.ht_hamilton_replies(O.OGraph.from_snapshot(moved), target, centers,
+                                       int((deg * (deg - 1) // 2).sum()))
+    assert not usage.graph_hit and np.array_equal(off, woff) and np.array_equal(rep, wrep)
