@@ -39,11 +39,16 @@ struct Batch {
   // work
   std::vector<KoptSegment> segments;
   DeviceArray<ee_kopt_task> d_tasks;
+  // the next work's rows, checked there before they replace d_tasks; and the
+  // segments they are checked against
+  DeviceArray<ee_kopt_task> d_next_tasks;
+  DeviceArray<KoptRowSegment> d_row_segments;
   DeviceArray<int64_t> d_costs;
   // improving-template masks instead of cells (ee_kopt_batch_set_output)
   bool mask_output = false;
   DeviceArray<uint32_t> d_masks;
-  std::vector<KoptTile> tiles;
+  std::vector<KoptTileSource> sources;
+  DeviceArray<KoptTileSource> d_sources;
   DeviceArray<KoptTile> d_tiles;
   KoptLaunch ranges{};  // per-k tile ranges of the current tiles
   uint64_t task_count = 0, cell_count = 0, tile_count = 0;
@@ -106,14 +111,26 @@ struct Batch {
       instances_dirty = false;
     }
     if (!layout_dirty) return;
-    tiles.assign(KoptCountTiles(segments.data(), segments.size(), tuning), KoptTile{});
-    KoptAssignTiles(segments.data(), segments.size(), instances.data(), plans.data(), tuning,
-                    tiles.data(), &ranges);
+    KoptAssignTiles(segments.data(), segments.size(), instances.data(), plans.data(), tuning, nullptr, &ranges);
     tile_count = ranges.tile_count;
     if (SharedBytes() > 65536) throw std::invalid_argument("k-opt tuning needs more than 64 KiB of LDS");
     if (ranges.inline_count == 0) {  // otherwise the kernel derives tiles from its arguments
-      d_tiles.Allocate(std::max<size_t>(tiles.size(), 1), ctx->device);
-      d_tiles.Upload(tiles.data(), tiles.size(), ctx->stream);
+      // the descriptors are made on the device, from a source per segment
+      sources.clear();
+      for (uint32_t k = 3; k <= 5; ++k) {
+        for (const KoptSegment& seg : segments) {
+          if (seg.k != k || seg.task_count == 0) continue;
+          const KoptInstance& inst = instances[seg.instance];
+          sources.push_back({seg.tile_begin, seg.task_offset, seg.task_count, seg.cost_offset, inst.coord_base,
+                             seg.rows_per_tile, plans[k - 3].templates, inst.distance_type, inst.near, 0});
+        }
+      }
+      if (d_tiles.count() < std::max<uint64_t>(tile_count, 1)) {
+        d_tiles.Allocate(std::max<uint64_t>(tile_count, 1), ctx->device);
+      }
+      if (d_sources.count() < sources.size()) d_sources.Allocate(sources.size(), ctx->device);
+      d_sources.Upload(sources.data(), sources.size(), ctx->stream);
+      LaunchKoptTiles(d_sources.get(), static_cast<uint32_t>(sources.size()), tile_count, d_tiles.get(), ctx->stream);
       ctx->Sync();
     }
     layout_dirty = false;
@@ -250,8 +267,8 @@ struct Batch {
   uint64_t ResidentBytes() const {
     uint64_t pools = 0;
     for (const PipeLane& l : lanes) pools += l.costs.bytes();
-    return d_xy.bytes() + d_tasks.bytes() + d_costs.bytes() + pools + d_masks.bytes() + d_tiles.bytes() +
-           d_plans.bytes();
+    return d_xy.bytes() + d_tasks.bytes() + d_next_tasks.bytes() + d_row_segments.bytes() + d_costs.bytes() + pools +
+           d_masks.bytes() + d_tiles.bytes() + d_sources.bytes() + d_plans.bytes();
   }
 };
 
@@ -568,37 +585,57 @@ ee_status ee_kopt_batch_set_work(ee_kopt_batch* batch, const ee_kopt_segment_des
     ee::Batch& b = ee::AsBatch(batch);
     if (segment_count > 0 && segments == nullptr) throw std::invalid_argument("segments is NULL");
     std::vector<ee::KoptSegment> segs;
+    std::vector<ee::KoptRowSegment> checks;  // with rows, and where the last one ends
     uint64_t rows = 0, cells = 0;
     bool present[3] = {false, false, false};
+    // the host's check of the rows of the segments so far, for the message
+    const auto refuse_rows = [&] {
+      for (const ee::KoptSegment& s : segs) {
+        ee::ValidateTasks(static_cast<int32_t>(b.instances[s.instance].n), s.k, tasks + s.task_offset, s.task_count);
+      }
+    };
+    const auto refuse = [&](const char* why) {
+      refuse_rows();
+      throw std::invalid_argument(why);
+    };
     for (uint32_t s = 0; s < segment_count; ++s) {
       const ee_kopt_segment_desc& d = segments[s];
-      if (d.instance >= b.instances.size()) throw std::invalid_argument("segment instance id");
-      if (d.k < 3 || d.k > 5) throw std::invalid_argument("segment k must be in [3,5]");
-      if (d.task_count > 0 && tasks == nullptr) throw std::invalid_argument("tasks is NULL");
-      ee::ValidateTasks(static_cast<int32_t>(b.instances[d.instance].n), d.k, tasks + rows,
-                        d.task_count);
+      if (d.instance >= b.instances.size()) refuse("segment instance id");
+      if (d.k < 3 || d.k > 5) refuse("segment k must be in [3,5]");
+      if (d.task_count > 0 && tasks == nullptr) refuse("tasks is NULL");
       // every segment starts on a 128-byte boundary, so whole-line stores of
       // its rows stay line-aligned
       cells = (cells + ee::kSegmentAlignCells - 1) / ee::kSegmentAlignCells * ee::kSegmentAlignCells;
       if (cell_offsets) cell_offsets[s] = cells;
       ee::KoptSegment seg{d.instance, d.k, rows, d.task_count, cells, 0, 1, 0};
       segs.push_back(seg);
+      if (d.task_count > 0) checks.push_back({rows, d.k, static_cast<int32_t>(b.instances[d.instance].n)});
       present[d.k - 3] = present[d.k - 3] || d.task_count > 0;
       rows += d.task_count;
       cells += d.task_count * ee::kTemplateCount[d.k - 3];
     }
     if (cell_offsets) cell_offsets[segment_count] = cells;
+    checks.push_back({rows, 0, 0});
     b.ctx->Activate();
+    const auto room = [&](auto& array, uint64_t count) {
+      if (array.count() < std::max<uint64_t>(count, 1)) array.Allocate(std::max<uint64_t>(count, 1), b.ctx->device);
+    };
+    room(b.d_next_tasks, rows);
+    room(b.d_row_segments, checks.size());
+    b.d_row_segments.Upload(checks.data(), checks.size(), b.ctx->stream);
+    if (!ee::UploadRows(*b.ctx, tasks, rows, b.d_row_segments.get(), checks.size() - 1, b.d_next_tasks.get())) {
+      refuse_rows();
+      throw std::logic_error("the device refused task rows that the host accepts");
+    }
     b.DropGraph();
     b.ClearWritten();
-    b.d_tasks.Allocate(std::max<uint64_t>(rows, 1), b.ctx->device);
-    b.d_tasks.Upload(tasks, rows, b.ctx->stream);
-    b.d_costs.Allocate(std::max<uint64_t>(cells, 1), b.ctx->device);
+    std::swap(b.d_tasks, b.d_next_tasks);
+    room(b.d_costs, cells);
     b.segments = std::move(segs);
     b.task_count = rows;
     b.cell_count = cells;
     for (int i = 0; i < 3; ++i) b.k_present[i] = present[i];
-    if (b.mask_output) b.d_masks.Allocate(std::max<uint64_t>(rows * b.MaskWords(), 1), b.ctx->device);
+    if (b.mask_output) room(b.d_masks, rows * b.MaskWords());
     b.ctx->Sync();
     b.layout_dirty = true;
   });
@@ -738,7 +775,8 @@ ee_status ee_kopt_batch_set_output(ee_kopt_batch* batch, uint32_t mode) {
     b.mask_output = mode == 1;
     b.ClearWritten();
     if (b.mask_output) {
-      b.d_masks.Allocate(std::max<uint64_t>(b.task_count * b.MaskWords(), 1), b.ctx->device);
+      const uint64_t words = std::max<uint64_t>(b.task_count * b.MaskWords(), 1);
+      if (b.d_masks.count() < words) b.d_masks.Allocate(words, b.ctx->device);
     }
     b.DropGraph();  // the launch arguments change
   });

@@ -188,6 +188,18 @@ constexpr uint32_t kPackedInvalid = 0xffffffffu;
 constexpr uint8_t kPackedInvalidHi = 0xff;
 void ExpandCells(const uint32_t* lo, const uint8_t* hi, size_t count, int64_t* cells);
 
+// What the tiles of one segment are made from on the device; sources in tile
+// order, each with at least one tile.
+struct KoptTileSource {
+  uint64_t tile_begin, task_offset, task_count, cost_offset, coord_base;
+  uint32_t rows_per_tile, templates;
+  uint16_t distance_type, near;
+  uint32_t reserved;
+};
+// Writes descriptors [0, tile_count) from `count` sources (device memory).
+void LaunchKoptTiles(const KoptTileSource* sources, uint32_t count, uint64_t tile_count, KoptTile* tiles,
+                     hipStream_t stream);
+
 // Number of tiles the segments split into under `tuning`.
 uint64_t KoptCountTiles(const KoptSegment* segments, size_t count, const KoptTuning& tuning);
 // Sets rows_per_tile and tile_begin of every segment, numbering tiles k by k,

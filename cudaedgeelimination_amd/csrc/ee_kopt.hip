@@ -1026,9 +1026,45 @@ __global__ void __launch_bounds__(kWave) KoptQueueKernel(KoptLaunch a, KoptQueue
   }
 }
 
+// One tile descriptor per thread, its source found by bisection.
+__global__ void __launch_bounds__(256) KoptTilesKernel(const KoptTileSource* __restrict__ sources, uint32_t count,
+                                                       uint64_t tile_count, KoptTile* __restrict__ tiles) {
+  const uint64_t tile = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (tile >= tile_count) return;
+  uint32_t lo = 0, hi = count - 1;  // the last source that begins at or before the tile
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo + 1) / 2;
+    if (sources[mid].tile_begin <= tile) {
+      lo = mid;
+    } else {
+      hi = mid - 1;
+    }
+  }
+  const KoptTileSource s = sources[lo];
+  const uint64_t row0 = (tile - s.tile_begin) * s.rows_per_tile;
+  KoptTile d;
+  d.task_index = s.task_offset + row0;
+  d.cost_index = s.cost_offset + row0 * s.templates;
+  d.coord_base = s.coord_base;
+  const uint64_t left = s.task_count - row0;
+  d.rows = left < s.rows_per_tile ? static_cast<uint32_t>(left) : s.rows_per_tile;
+  d.distance_type = s.distance_type;
+  d.near = s.near;
+  tiles[tile] = d;
+}
+
 uint32_t Align16(uint32_t v) { return (v + 15u) & ~15u; }
 
 }  // namespace
+
+void LaunchKoptTiles(const KoptTileSource* sources, uint32_t count, uint64_t tile_count, KoptTile* tiles,
+                     hipStream_t stream) {
+  if (count == 0 || tile_count == 0) return;
+  if (tile_count > (uint64_t{1} << 38)) throw std::invalid_argument("k-opt launch has too many tiles");
+  const uint32_t blocks = static_cast<uint32_t>((tile_count + 255) / 256);
+  hipLaunchKernelGGL(KoptTilesKernel, dim3(blocks), dim3(256), 0, stream, sources, count, tile_count, tiles);
+  CheckHip(hipGetLastError(), "KoptTilesKernel launch");
+}
 
 size_t KoptQueueLayout(KoptLaunch* a, const KoptPlan plans[3], const KoptTuning& tuning) {
   KoptTuning t = tuning;

@@ -323,18 +323,28 @@ struct Context {
   KoptCursorCache cursor;
   HtCache ht;
   DirectIo io;
-  // DownloadToCaller's two page-locked chunks and their events, made on
-  // first use
-  Pinned<char> stage[2];
-  hipEvent_t stage_ready[2] = {nullptr, nullptr};
 };
 
-// Copies `bytes` of device memory to caller memory and waits, after the work
-// queued before it on the context's stream.  A large copy goes through the
-// context's two page-locked chunks: while one chunk is in flight over PCIe
-// the other is copied out on host threads.  A copy straight into pageable
-// caller memory is staged by the runtime at about half that rate.
+// Copies `bytes` (whole 4-byte words) of device memory to caller memory and
+// waits, after the work queued before it on the context's stream: a kernel
+// writes the words into the context's ring and host threads copy them out
+// as they arrive.
 void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes);
+
+// The rows from row_begin to the next entry's are checked as k-opt task rows
+// of this k on n nodes.
+struct KoptRowSegment {
+  uint64_t row_begin;
+  uint32_t k;
+  int32_t n;
+};
+
+// Copies task rows [0, count) into device memory through the context's ring,
+// checking them on the way as ValidateTasks does, against `segments` entries
+// on the device (and one more, where the last ends).  Returns once all rows
+// are in place; false if some row is refused.
+bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const KoptRowSegment* d_segments,
+                size_t segments, ee_kopt_task* d_rows);
 
 // Device-resident cost cells [0, count) into caller memory, after the work
 // queued before on the context's stream, in transfer form through the

@@ -105,52 +105,7 @@ Context::~Context() {
   kopt = KoptCache{};
   static_cast<void>(hipEventDestroy(ev_begin));
   static_cast<void>(hipEventDestroy(ev_end));
-  for (hipEvent_t e : stage_ready) {
-    if (e != nullptr) static_cast<void>(hipEventDestroy(e));
-  }
   static_cast<void>(hipStreamDestroy(stream));
-}
-
-void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes) {
-  // below kDirect the runtime's own copy costs no more; chunks of kChunk
-  // copied out by kParts host threads kept pace with PCIe on the MI355X host
-  constexpr size_t kDirect = size_t{1} << 20, kChunk = size_t{4} << 20, kParts = 4;
-  if (bytes == 0) return;
-  if (dst == nullptr || src == nullptr) throw std::logic_error("download with a NULL buffer");
-  if (bytes < kDirect) {
-    CheckHip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx.stream), "hipMemcpyAsync D2H");
-    ctx.Sync();
-    return;
-  }
-  for (int b = 0; b < 2; ++b) {
-    ctx.stage[b].Reserve(kChunk);
-    if (ctx.stage_ready[b] == nullptr) {
-      CheckHip(hipEventCreateWithFlags(&ctx.stage_ready[b], hipEventDisableTiming), "hipEventCreate");
-    }
-  }
-  char* const out = static_cast<char*>(dst);
-  const char* const in = static_cast<const char*>(src);
-  const size_t chunks = (bytes + kChunk - 1) / kChunk;
-  // chunk i goes to stage i % 2; the chunk before it is copied out meanwhile,
-  // so a stage is refilled only after its previous chunk has left it
-  for (size_t i = 0; i <= chunks; ++i) {
-    if (i < chunks) {
-      const size_t at = i * kChunk;
-      CheckHip(hipMemcpyAsync(ctx.stage[i % 2].get(), in + at, std::min(kChunk, bytes - at), hipMemcpyDeviceToHost,
-                              ctx.stream),
-               "hipMemcpyAsync D2H chunk");
-      CheckHip(hipEventRecord(ctx.stage_ready[i % 2], ctx.stream), "hipEventRecord");
-    }
-    if (i > 0) {
-      const size_t j = i - 1, at = j * kChunk, len = std::min(kChunk, bytes - at);
-      CheckHip(hipEventSynchronize(ctx.stage_ready[j % 2]), "hipEventSynchronize");
-      const char* const from = ctx.stage[j % 2].get();
-      ParallelFor(kParts, [&](size_t p) {
-        const size_t a = len * p / kParts, b = len * (p + 1) / kParts;
-        std::memcpy(out + at + a, from + a, b - a);
-      }, static_cast<unsigned>(kParts));
-    }
-  }
 }
 
 void Context::Activate() const { CheckHip(hipSetDevice(device), "hipSetDevice"); }

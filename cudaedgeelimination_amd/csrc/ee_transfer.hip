@@ -1,7 +1,9 @@
-// Results that reach the caller through page-locked host memory which kernels
-// write in place: the ring itself (DirectIo), the host's side of taking
-// cells out of it, and the download of device-resident cells.
+// Transfers between caller memory and the device through page-locked host
+// memory which kernels read and write in place: the ring itself (DirectIo),
+// the host's side of taking tiles out of it, the download of device-resident
+// cells and words, and the upload of task rows.
 #include <algorithm>
+#include <cstring>
 #include <stdexcept>
 
 #include "ee_internal.h"
@@ -38,6 +40,104 @@ __global__ __launch_bounds__(kWave) void PackCells(const int64_t* __restrict__ c
     if (threadIdx.x == 0) __hip_atomic_store(marks + tile, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
+
+// Words [0, count) to host memory, tile by tile, as PackCells.
+__global__ __launch_bounds__(kWave) void CopyWords(const uint32_t* __restrict__ words, uint32_t count,
+                                                   uint32_t* __restrict__ out, uint64_t* __restrict__ marks,
+                                                   uint64_t mark) {
+  const uint32_t tiles = (count + kPackTile - 1) / kPackTile;
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint32_t end = min(count, (tile + 1) * kPackTile);
+#pragma unroll 4
+    for (uint32_t i = tile * kPackTile + threadIdx.x; i < end; i += kWave) out[i] = words[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    if (threadIdx.x == 0) __hip_atomic_store(marks + tile, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// ValidateTasks' rule for one row (12 words) of a segment.
+__device__ inline bool RowIsValid(const int32_t* row, uint32_t k, int32_t n) {
+  bool ok = row[11] >= 0;  // the high word of deleted_cost
+  uint64_t deleted[kMaxK];
+  for (uint32_t e = 0; e < static_cast<uint32_t>(kMaxK); ++e) {
+    if (e >= k) break;
+    const int32_t a = row[2 * e], b = row[2 * e + 1];
+    ok = ok && a >= 0 && b >= 0 && a < n && b < n && a != b;
+    deleted[e] = (static_cast<uint64_t>(min(a, b)) << 32) | static_cast<uint32_t>(max(a, b));
+    for (uint32_t f = 0; f < e; ++f) ok = ok && deleted[f] != deleted[e];
+  }
+  return ok;
+}
+
+// One workgroup per 256 rows: it reads them from host memory in whole words,
+// stores them to the row pool, and checks a row per thread out of LDS.  PCIe
+// bounds it (56 GB/s: 12.6 MB in 225 us); the host's check of as many rows
+// took 1.2 ms.  marks[i] once group i is done, *refused = 1 on a bad row.
+constexpr uint32_t kIngestRows = 256;
+constexpr uint32_t kRowWords = sizeof(ee_kopt_task) / 4;
+
+__global__ __launch_bounds__(kIngestRows) void IngestRows(const uint32_t* __restrict__ staged, uint64_t first,
+                                                          uint32_t count, const KoptRowSegment* __restrict__ segments,
+                                                          uint32_t segment_count, uint32_t* __restrict__ rows,
+                                                          uint32_t* __restrict__ refused, uint64_t* __restrict__ marks,
+                                                          uint64_t mark) {
+  __shared__ int32_t words[kIngestRows * kRowWords];
+  const uint32_t row0 = blockIdx.x * kIngestRows;
+  const uint32_t here = min(kIngestRows, count - row0);
+  const uint32_t* from = staged + static_cast<uint64_t>(row0) * kRowWords;
+  uint32_t* to = rows + (first + row0) * kRowWords;
+#pragma unroll 4
+  for (uint32_t q = threadIdx.x; q < here * kRowWords; q += kIngestRows) {
+    const uint32_t v = from[q];
+    words[q] = static_cast<int32_t>(v);
+    to[q] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < here) {
+    const uint64_t row = first + row0 + threadIdx.x;
+    uint32_t lo = 0, hi = segment_count - 1;  // the last segment that begins at or before the row
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo + 1) / 2;
+      if (segments[mid].row_begin <= row) {
+        lo = mid;
+      } else {
+        hi = mid - 1;
+      }
+    }
+    if (!RowIsValid(words + threadIdx.x * kRowWords, segments[lo].k, segments[lo].n)) {
+      __hip_atomic_store(refused, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    __hip_atomic_store(marks + blockIdx.x, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// Passes items [0, count) through the ring in launches of at most
+// `slot_items`, each with a slot of slot_bytes: start(i, slot) stages and
+// launches number i, finish(i, slot) takes what it left.
+template <typename Start, typename Finish>
+void ThroughRing(Context& ctx, size_t launches, Start&& start, Finish&& finish) {
+  const size_t slots = std::min<size_t>(launches, DirectIo::kSlots);
+  try {
+    for (size_t i = 0; i < slots; ++i) start(i, i);
+    for (size_t i = 0; i < launches; ++i) {
+      finish(i, i % slots);
+      if (i + slots < launches) start(i + slots, i % slots);
+    }
+  } catch (...) {
+    static_cast<void>(hipStreamSynchronize(ctx.stream));  // the ring is free again
+    throw;
+  }
+}
+
+// A launch's share of the ring's second size.
+constexpr size_t kSlotBytes = size_t{2} << 20;
+static_assert(kSlotBytes / 4 / kPackTile <= DirectIo::kSlotTiles, "a slot's tiles have marks");
+static_assert(kSlotBytes * DirectIo::kSlots <= DirectIo::kSizes[1], "the slots fit");
 
 }  // namespace
 
@@ -107,45 +207,102 @@ void DirectIo::TakeCells(size_t slot, uint64_t mark, hipStream_t stream, const u
 void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide, int64_t* cells) {
   if (count == 0) return;
   if (d_cells == nullptr || cells == nullptr) throw std::logic_error("download with a NULL buffer");
-  // whole tiles, 2 MiB to a slot: the ring's second size
-  constexpr size_t kSlotBytes = size_t{2} << 20;
-  static_assert(kSlotBytes / 4 / kPackTile <= DirectIo::kSlotTiles, "a slot's tiles have marks");
   const size_t cell_bytes = wide ? 5 : 4;
   const size_t slot_cells = kSlotBytes / cell_bytes / kPackTile * kPackTile;
   const size_t launches = (count + slot_cells - 1) / slot_cells;
-  const size_t slots = std::min<size_t>(launches, DirectIo::kSlots);
   const size_t plane = launches == 1 ? (count + 255) / 256 * 256 : slot_cells;
   const size_t slot_bytes = plane * cell_bytes;
   DirectIo& io = ctx.io;
-  io.Reserve(slots * slot_bytes);
+  io.Reserve(std::min<size_t>(launches, DirectIo::kSlots) * slot_bytes);
   uint64_t marks[DirectIo::kSlots] = {};
   const auto cells_of = [&](size_t i) { return std::min(slot_cells, count - i * slot_cells); };
-  const auto launch = [&](size_t i) {
-    const size_t slot = i % slots;
+  ThroughRing(ctx, launches, [&](size_t i, size_t slot) {
     char* at = io.device() + slot * slot_bytes;
-    uint8_t* hi = reinterpret_cast<uint8_t*>(at + plane * 4);
     marks[slot] = io.NextMark();
     const uint32_t n = static_cast<uint32_t>(cells_of(i));
-    const uint32_t grid = std::min<uint32_t>(kPackWaves, (n + kPackTile - 1) / kPackTile);
-    hipLaunchKernelGGL((wide ? PackCells<true> : PackCells<false>), dim3(grid), dim3(kWave), 0, ctx.stream,
-                       d_cells + i * slot_cells, n, reinterpret_cast<uint32_t*>(at), hi, io.device_marks(slot),
-                       marks[slot]);
+    hipLaunchKernelGGL((wide ? PackCells<true> : PackCells<false>),
+                       dim3(std::min<uint32_t>(kPackWaves, (n + kPackTile - 1) / kPackTile)), dim3(kWave), 0, ctx.stream,
+                       d_cells + i * slot_cells, n, reinterpret_cast<uint32_t*>(at),
+                       reinterpret_cast<uint8_t*>(at + plane * 4), io.device_marks(slot), marks[slot]);
     CheckHip(hipGetLastError(), "PackCells launch");
-  };
-  try {
-    for (size_t i = 0; i < slots; ++i) launch(i);
-    for (size_t i = 0; i < launches; ++i) {
-      const size_t slot = i % slots;
-      const char* at = io.host() + slot * slot_bytes;
-      io.TakeCells(slot, marks[slot], ctx.stream, reinterpret_cast<const uint32_t*>(at),
-                   wide ? reinterpret_cast<const uint8_t*>(at + plane * 4) : nullptr, cells_of(i), kPackTile,
-                   cells + i * slot_cells);
-      if (i + slots < launches) launch(i + slots);
-    }
-  } catch (...) {
-    static_cast<void>(hipStreamSynchronize(ctx.stream));  // the ring is free again
-    throw;
-  }
+  }, [&](size_t i, size_t slot) {
+    const char* at = io.host() + slot * slot_bytes;
+    io.TakeCells(slot, marks[slot], ctx.stream, reinterpret_cast<const uint32_t*>(at),
+                 wide ? reinterpret_cast<const uint8_t*>(at + plane * 4) : nullptr, cells_of(i), kPackTile,
+                 cells + i * slot_cells);
+  });
+}
+
+void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes) {
+  if (bytes == 0) return;
+  if (dst == nullptr || src == nullptr) throw std::logic_error("download with a NULL buffer");
+  if (bytes % 4 != 0) throw std::logic_error("download of partial words");
+  constexpr size_t kSlotWords = kSlotBytes / 4;
+  const size_t count = bytes / 4, launches = (count + kSlotWords - 1) / kSlotWords;
+  const size_t slot_words = std::min(kSlotWords, count);
+  DirectIo& io = ctx.io;
+  io.Reserve(std::min<size_t>(launches, DirectIo::kSlots) * slot_words * 4);
+  uint64_t marks[DirectIo::kSlots] = {};
+  const auto words_of = [&](size_t i) { return std::min(kSlotWords, count - i * kSlotWords); };
+  ThroughRing(ctx, launches, [&](size_t i, size_t slot) {
+    marks[slot] = io.NextMark();
+    const uint32_t n = static_cast<uint32_t>(words_of(i));
+    hipLaunchKernelGGL(CopyWords, dim3(std::min<uint32_t>(kPackWaves, (n + kPackTile - 1) / kPackTile)), dim3(kWave),
+                       0, ctx.stream, static_cast<const uint32_t*>(src) + i * kSlotWords, n,
+                       reinterpret_cast<uint32_t*>(io.device()) + slot * slot_words, io.device_marks(slot),
+                       marks[slot]);
+    CheckHip(hipGetLastError(), "CopyWords launch");
+  }, [&](size_t i, size_t slot) {
+    const size_t n = words_of(i);
+    const uint32_t* from = reinterpret_cast<const uint32_t*>(io.host()) + slot * slot_words;
+    uint32_t* to = static_cast<uint32_t*>(dst) + i * kSlotWords;
+    // 64 KiB at a time, on host threads from 512 KiB up
+    io.TakeTiles(slot, marks[slot], ctx.stream, (n + kPackTile - 1) / kPackTile, 32, n < (size_t{1} << 17) ? 1 : 8,
+                 [&](size_t first, size_t last) {
+                   const size_t b = first * kPackTile, e = std::min(n, last * kPackTile);
+                   std::memcpy(to + b, from + b, (e - b) * 4);
+                 });
+  });
+}
+
+bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const KoptRowSegment* d_segments,
+                size_t segments, ee_kopt_task* d_rows) {
+  if (count == 0) return true;
+  constexpr size_t kHeader = 256;  // the refusal flag
+  constexpr size_t kSlotRows = (kSlotBytes - kHeader) / sizeof(ee_kopt_task) / kIngestRows * kIngestRows;
+  static_assert(kSlotRows / kIngestRows <= DirectIo::kSlotTiles, "a slot's groups have marks");
+  if (segments == 0 || segments > UINT32_MAX) throw std::logic_error("row segments");
+  const size_t launches = (count + kSlotRows - 1) / kSlotRows;
+  const size_t slot_bytes = kHeader + std::min(kSlotRows, (count + 63) / 64 * 64) * sizeof(ee_kopt_task);
+  DirectIo& io = ctx.io;
+  io.Reserve(std::min<size_t>(launches, DirectIo::kSlots) * slot_bytes);
+  uint64_t marks[DirectIo::kSlots] = {};
+  const auto rows_of = [&](size_t i) { return std::min(kSlotRows, count - i * kSlotRows); };
+  bool refused = false;
+  ThroughRing(ctx, launches, [&](size_t i, size_t slot) {
+    const size_t n = rows_of(i);
+    char* at = io.host() + slot * slot_bytes;
+    *reinterpret_cast<uint32_t*>(at) = 0;
+    // 64 KiB at a time, on host threads from 256 KiB up
+    const char* from = reinterpret_cast<const char*>(rows + i * kSlotRows);
+    const size_t bytes = n * sizeof(ee_kopt_task), piece = size_t{64} << 10;
+    ParallelFor((bytes + piece - 1) / piece, [&](size_t p) {
+      std::memcpy(at + kHeader + p * piece, from + p * piece, std::min(piece, bytes - p * piece));
+    }, bytes < (size_t{256} << 10) ? 1 : 8);
+    char* device = io.device() + slot * slot_bytes;
+    marks[slot] = io.NextMark();
+    hipLaunchKernelGGL(IngestRows, dim3(static_cast<uint32_t>((n + kIngestRows - 1) / kIngestRows)), dim3(kIngestRows), 0,
+                       ctx.stream, reinterpret_cast<const uint32_t*>(device + kHeader), static_cast<uint64_t>(i * kSlotRows),
+                       static_cast<uint32_t>(n), d_segments, static_cast<uint32_t>(segments),
+                       reinterpret_cast<uint32_t*>(d_rows), reinterpret_cast<uint32_t*>(device), io.device_marks(slot),
+                       marks[slot]);
+    CheckHip(hipGetLastError(), "IngestRows launch");
+  }, [&](size_t i, size_t slot) {
+    const size_t groups = (rows_of(i) + kIngestRows - 1) / kIngestRows;
+    for (size_t g = 0; g < groups; ++g) io.WaitTile(slot, g, marks[slot], ctx.stream);
+    refused = refused || *reinterpret_cast<const uint32_t*>(io.host() + slot * slot_bytes) != 0;
+  });
+  return !refused;
 }
 
 }  // namespace ee

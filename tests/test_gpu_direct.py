@@ -199,3 +199,42 @@ def test_hamilton_verdicts(ctx, degree):
     woff, wrep = O.ht_hamilton_replies(O.OGraph.from_snapshot(moved), target, centers,
                                        int((deg * (deg - 1) // 2).sum()))
     assert not usage.graph_hit and np.array_equal(off, woff) and np.array_equal(rep, wrep)
+
+
+@pytest.mark.parametrize("rows", [1, 255, 257, 43_520, 43_521, 90_001])
+def test_set_work_rows(ctx, rows):
+    """Rows checked by the device on their way in, at the edges of its groups
+    (256 rows) and slots (43,520): good rows give the oracle's masks, one bad
+    row anywhere is refused with the host's message and the batch keeps its
+    work."""
+    say(f"set_work rows={rows}")
+    a, b = graph(21, 400, EUC_2D, 1_000_000), graph(22, 300, CEIL_2D, 1 << 30)
+    k3 = rows // 2
+    tasks = np.concatenate([W.kopt_tasks(1, a, np.full(k3, 3, np.uint8)),
+                            W.kopt_tasks(2, b, np.full(rows - k3, 4, np.uint8))])
+    batch = KoptBatch(ctx)
+    ia, ib = batch.add_instance(a), batch.add_instance(b)
+    batch.set_output("masks")
+    segments = [(ia, 3, k3), (ib, 5, 0), (ib, 4, rows - k3)]
+    want = []
+    for g, k, part in ((a, 3, tasks[:k3]), (b, 4, tasks[k3:])):
+        cells, _, _ = O.kopt_costs(g.x, g.y, g.distance_type, k, part)
+        bits = cells.reshape(len(part), 4 if k == 3 else 25) < part["deleted_cost"][:, None]
+        want.append((bits << np.arange(bits.shape[1])).sum(axis=1).astype(np.uint32))
+    want = np.concatenate(want)
+    for at in sorted({0, k3 - 1, k3, rows - 1} & set(range(rows))):
+        batch.set_work(segments, tasks)
+        n = a.dimension if at < k3 else b.dimension
+        for port, value, cost in ((2, n, 0), (5, -1, 0), (4, None, 0), (0, None, -1)):
+            bad = tasks.copy()
+            if cost:
+                bad["deleted_cost"][at] = -5
+            elif value is None:
+                bad["port_nodes"][at, 4:6] = bad["port_nodes"][at, 1::-1]  # the first deleted edge again
+            else:
+                bad["port_nodes"][at, port] = value
+            with pytest.raises(_lib.InvalidArgument, match="negative deleted_cost" if cost else "deleted edge"):
+                batch.set_work(segments, bad)
+        batch.run()
+        assert np.array_equal(batch.download_masks()[:, 0], want)
+    batch.close()
