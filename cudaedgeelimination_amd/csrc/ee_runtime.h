@@ -176,7 +176,6 @@ struct JvCache {
   // exact static key (host copies)
   std::vector<int64_t> x, y, edge_weight;
   std::vector<int32_t> edge_u, edge_v;
-  std::vector<int32_t> host_active;
   // static: 8m + 8m + 16n bytes
   DeviceArray<int2> d_uv;
   DeviceArray<int64_t> d_weight;
@@ -224,7 +223,7 @@ class DirectIo {
   // The sizes the ring takes: the first when the context is made, which most
   // calls fit, the next for large results, and what a call asks for beyond.
   // Few steps, since fresh page-locked memory costs about 0.4 ms per MB.
-  static constexpr size_t kSizes[2] = {size_t{1} << 20, size_t{4} << 20};
+  static constexpr size_t kSizes[2] = {size_t{2} << 20, size_t{4} << 20};
   // At least `bytes`; growing discards the contents (no kernel may be using them).
   void Reserve(size_t bytes);
   char* host() { return mem_.get(); }
@@ -350,6 +349,21 @@ bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const Kopt
 // queued before on the context's stream, in transfer form through the
 // context's ring.  wide: some instance's coordinates are not near.
 void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide, int64_t* cells);
+
+// Where a snapshot's active flags (as words) and CSR go on the device, and
+// the bounds of its node ids and edge slots.
+struct JvDynamic {
+  int32_t *active, *row_offsets, *neighbors, *edge_ids;
+  uint32_t nodes, slots;
+};
+
+// Copies the snapshot's active flags and CSR (whose row offsets the caller
+// has checked) to the device through the context's ring; `then` runs once the
+// last part is queued, with the snapshot in place for work it queues on the
+// context's stream.  False if some neighbour or edge id is out of range; the
+// device then holds 0 in its place.
+bool UploadJvDynamic(Context& ctx, const ee_graph_view& g, size_t adjacency, const JvDynamic& to,
+                     const std::function<void()>& then);
 
 // Elements [offset, offset + count) of a device array into caller memory, as
 // DownloadToCaller.

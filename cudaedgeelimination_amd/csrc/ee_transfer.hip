@@ -3,8 +3,10 @@
 // the host's side of taking tiles out of it, the download of device-resident
 // cells and words, and the upload of task rows.
 #include <algorithm>
+#include <array>
 #include <cstring>
 #include <stdexcept>
+#include <vector>
 
 #include "ee_internal.h"
 #include "ee_jvhost.h"
@@ -113,6 +115,71 @@ __global__ __launch_bounds__(kIngestRows) void IngestRows(const uint32_t* __rest
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
     __hip_atomic_store(marks + blockIdx.x, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// One stretch of a snapshot's dynamic arrays in a slot: elements [first,
+// first + count) of `array`, from byte `at` of the slot (16-byte aligned).
+enum JvArray : uint32_t { kJvActive, kJvRowOffsets, kJvNeighbors, kJvEdgeIds };
+struct JvPiece {
+  uint32_t array, at;
+  uint64_t first;
+  uint32_t count, reserved;
+};
+constexpr uint32_t kJvPieces = 4;  // a slot holds at most one stretch of each array
+
+struct JvIngest {
+  JvDynamic to;
+  const char* staged;  // the slot: the refusal flag, then the pieces
+  uint32_t* refused;
+  uint64_t* marks;     // [gridDim.x]
+  uint64_t mark;
+  JvPiece pieces[kJvPieces];
+};
+
+// The slot's stretches to the device arrays, active flags widened to words,
+// ids checked (one out of range is stored as 0 and refuses the call).  PCIe
+// bounds it; the blocks read whole words in a row.
+constexpr uint32_t kJvBlocks = 256;
+__global__ __launch_bounds__(256) void IngestJv(JvIngest g) {
+  const uint32_t self = blockIdx.x * 256 + threadIdx.x, all = gridDim.x * 256;
+  bool bad = false;
+  for (uint32_t p = 0; p < kJvPieces; ++p) {  // uniform
+    const JvPiece piece = g.pieces[p];
+    if (piece.count == 0) continue;
+    const uint32_t* from = reinterpret_cast<const uint32_t*>(g.staged + piece.at);
+    if (piece.array == kJvActive) {
+      int32_t* to = g.to.active + piece.first;
+      for (uint32_t i = self; i < (piece.count + 3) / 4; i += all) {
+        const uint32_t flags = from[i];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          if (4 * i + u < piece.count) to[4 * i + u] = ((flags >> (8 * u)) & 0xffu) != 0 ? 1 : 0;
+        }
+      }
+      continue;
+    }
+    int32_t* to = (piece.array == kJvRowOffsets ? g.to.row_offsets
+                   : piece.array == kJvNeighbors ? g.to.neighbors
+                                                 : g.to.edge_ids) + piece.first;
+    const uint32_t limit = piece.array == kJvRowOffsets ? 0xffffffffu
+                           : piece.array == kJvNeighbors ? g.to.nodes
+                                                         : g.to.slots;
+#pragma unroll 4
+    for (uint32_t i = self; i < piece.count; i += all) {
+      const uint32_t v = from[i];
+      bad |= v >= limit;
+      to[i] = v >= limit ? 0 : static_cast<int32_t>(v);
+    }
+  }
+  if (bad) {
+    __hip_atomic_store(g.refused, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    __hip_atomic_store(g.marks + blockIdx.x, g.mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -300,6 +367,74 @@ bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const Kopt
   }, [&](size_t i, size_t slot) {
     const size_t groups = (rows_of(i) + kIngestRows - 1) / kIngestRows;
     for (size_t g = 0; g < groups; ++g) io.WaitTile(slot, g, marks[slot], ctx.stream);
+    refused = refused || *reinterpret_cast<const uint32_t*>(io.host() + slot * slot_bytes) != 0;
+  });
+  return !refused;
+}
+
+bool UploadJvDynamic(Context& ctx, const ee_graph_view& g, size_t adjacency, const JvDynamic& to,
+                     const std::function<void()>& then) {
+  // slots of 2 MiB: 1.4 MB through 512 KiB slots took 27 us more, the gaps
+  // between four launches
+  constexpr size_t kHeader = 256, room = kSlotBytes - kHeader;
+  const struct {
+    const char* from;
+    size_t count, element;
+  } arrays[kJvPieces] = {
+      {reinterpret_cast<const char*>(g.edge_active), static_cast<size_t>(g.edge_count), 1},
+      {reinterpret_cast<const char*>(g.row_offsets), static_cast<size_t>(g.dimension) + 1, 4},
+      {reinterpret_cast<const char*>(g.neighbors), adjacency, 4},
+      {reinterpret_cast<const char*>(g.csr_edge_ids), adjacency, 4}};
+  // slots filled one after the other with stretches of the arrays in turn
+  std::vector<std::array<JvPiece, kJvPieces>> plan;
+  size_t used = room, longest = 0;
+  for (uint32_t a = 0; a < kJvPieces; ++a) {
+    for (size_t first = 0; first < arrays[a].count;) {
+      if (room - used < 256) {
+        plan.emplace_back();
+        plan.back().fill(JvPiece{});
+        used = 0;
+      }
+      const size_t n = std::min(arrays[a].count - first, (room - used) / arrays[a].element);
+      plan.back()[a] = JvPiece{a, static_cast<uint32_t>(kHeader + used), first, static_cast<uint32_t>(n), 0};
+      used = std::min(room, (used + n * arrays[a].element + 15) / 16 * 16);
+      longest = std::max(longest, used);
+      first += n;
+    }
+  }
+  const size_t slot_bytes = (kHeader + longest + 255) / 256 * 256;
+  DirectIo& io = ctx.io;
+  io.Reserve(std::min<size_t>(plan.size(), DirectIo::kSlots) * slot_bytes);
+  uint64_t marks[DirectIo::kSlots] = {};
+  bool refused = false;
+  ThroughRing(ctx, plan.size(), [&](size_t i, size_t slot) {
+    char* at = io.host() + slot * slot_bytes;
+    *reinterpret_cast<uint32_t*>(at) = 0;
+    // 64 KiB at a time, on host threads where there is more of them
+    constexpr size_t kPart = size_t{64} << 10;
+    std::array<size_t, kJvPieces + 1> parts{};
+    for (uint32_t a = 0; a < kJvPieces; ++a) {
+      parts[a + 1] = parts[a] + (plan[i][a].count * arrays[a].element + kPart - 1) / kPart;
+    }
+    ParallelFor(parts[kJvPieces], [&](size_t part) {
+      uint32_t a = 0;
+      while (part >= parts[a + 1]) ++a;
+      const JvPiece& piece = plan[i][a];
+      const size_t b = (part - parts[a]) * kPart, bytes = piece.count * arrays[a].element;
+      std::memcpy(at + piece.at + b, arrays[a].from + piece.first * arrays[a].element + b, std::min(kPart, bytes - b));
+    }, parts[kJvPieces] < 6 ? 1 : 8);
+    JvIngest job{};
+    job.to = to;
+    job.staged = io.device() + slot * slot_bytes;
+    job.refused = reinterpret_cast<uint32_t*>(io.device() + slot * slot_bytes);
+    job.marks = io.device_marks(slot);
+    job.mark = marks[slot] = io.NextMark();
+    std::copy(plan[i].begin(), plan[i].end(), job.pieces);
+    hipLaunchKernelGGL(IngestJv, dim3(kJvBlocks), dim3(256), 0, ctx.stream, job);
+    CheckHip(hipGetLastError(), "IngestJv launch");
+    if (i + 1 == plan.size()) then();
+  }, [&](size_t, size_t slot) {
+    for (size_t b = 0; b < kJvBlocks; ++b) io.WaitTile(slot, b, marks[slot], ctx.stream);
     refused = refused || *reinterpret_cast<const uint32_t*>(io.host() + slot * slot_bytes) != 0;
   });
   return !refused;

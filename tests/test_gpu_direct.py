@@ -238,3 +238,35 @@ def test_set_work_rows(ctx, rows):
         batch.run()
         assert np.array_equal(batch.download_masks()[:, 0], want)
     batch.close()
+
+
+@pytest.mark.parametrize("n, neighbors", [(4, 3), (41, 6), (700, 10), (60_000, 8)])
+def test_jv_call_inputs(ctx, n, neighbors):
+    """The dynamic arrays on their way in (one slot and several; odd counts;
+    inactive edges), refused ids, and a snapshot that differs from the resident
+    one in one late weight or coordinate."""
+    say(f"jv call n={n}")
+    rng = np.random.default_rng(n)
+    g = W.knn_graph(rng.integers(0, 1_000_000, n), rng.integers(0, 1_000_000, n), EUC_2D, neighbors)
+    backend.clear_jv_cuda_cache(ctx)
+    for drop in (0, 1, 1 + g.edge_count // 7):
+        g.edge_active[rng.permutation(g.edge_count)[:drop]] = 0
+        g.rebuild_csr()
+        want = O.OGraph.from_snapshot(g).witnesses()
+        got, usage = backend.find_jv_witnesses(g, ctx)
+        assert np.array_equal(got, want) and usage.static_hit == (drop != 0)
+    a = g.adjacency_count
+    for name, value, text in (("neighbors", n, "neighbour"), ("neighbors", -1, "neighbour"),
+                              ("csr_edge_ids", g.edge_count, "edge id"), ("row_offsets", -2, "non-decreasing")):
+        bad = g.copy()
+        getattr(bad, name)[(a if name != "row_offsets" else n) - 1] = value
+        with pytest.raises(_lib.InvalidArgument, match=text):
+            backend.find_jv_witnesses(bad, ctx)
+    got, usage = backend.find_jv_witnesses(g, ctx)
+    assert np.array_equal(got, want) and usage.static_hit and usage.workspace_hit
+    moved = g.copy()
+    moved.x[n - 1] += 3000
+    moved = type(g).from_edges(moved.x, moved.y, EUC_2D, g.edge_u, g.edge_v, None, g.edge_active)
+    got, usage = backend.find_jv_witnesses(moved, ctx)
+    assert np.array_equal(got, O.OGraph.from_snapshot(moved).witnesses())
+    assert not usage.static_hit and usage.workspace_hit
