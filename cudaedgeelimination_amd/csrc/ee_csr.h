@@ -12,6 +12,8 @@
 // order, and the host rebuild the session keeps beside it is the same).
 #pragma once
 
+#include <vector>
+
 #include "ee_runtime.h"
 
 namespace ee {
@@ -21,9 +23,15 @@ class DeviceCsr {
   // n nodes, m edge slots, at most `adjacency` CSR entries, at most
   // `max_commits` slots per commit.
   void Allocate(size_t n, size_t m, size_t adjacency, size_t max_commits, int device);
-  // Uploads active flags (0/1 per slot) and a CSR into the current buffer.
-  void Upload(const int32_t* active, const int32_t* row_offsets, const int32_t* neighbors,
-              const int32_t* edge_ids, size_t adjacency, hipStream_t stream);
+  // Adds the upload of a snapshot to the current buffer: active flags (bytes)
+  // of m edge slots from slot `edge`, and the rows of n nodes from node
+  // `node`, whose entries start at entry `entry` and hold ids from 0 (union
+  // ids are formed on the way).  The last snapshot's end is set by AddEnd.
+  void AddUpload(std::vector<UploadItem>* items, size_t node, size_t n, size_t edge, size_t m, size_t entry,
+                 size_t entries, const uint8_t* active, const int32_t* row_offsets, const int32_t* neighbors,
+                 const int32_t* edge_ids);
+  // Adds the end of the last row; *end must live until the upload.
+  void AddEnd(std::vector<UploadItem>* items, const int32_t* end);
   // Pinned staging of a commit: word 0 the count, then the edge slots.
   int32_t* StageCommits() { return h_commits_.get(); }
   // Enqueues the upload of the staged commit (count + slots) on `stream`.

@@ -154,13 +154,20 @@ void DeviceCsr::Allocate(size_t n, size_t m, size_t adjacency, size_t max_commit
   h_commits_.get()[0] = 0;
 }
 
-void DeviceCsr::Upload(const int32_t* active, const int32_t* row_offsets, const int32_t* neighbors,
-                       const int32_t* edge_ids, size_t adjacency, hipStream_t stream) {
-  if (adjacency > adjacency_) throw std::logic_error("device CSR upload beyond its capacity");
-  active_.Upload(active, m_, stream);
-  ro_[cur_].Upload(row_offsets, n_ + 1, stream);
-  nb_[cur_].Upload(neighbors, adjacency, stream);
-  eid_[cur_].Upload(edge_ids, adjacency, stream);
+void DeviceCsr::AddUpload(std::vector<UploadItem>* items, size_t node, size_t n, size_t edge, size_t m, size_t entry,
+                          size_t entries, const uint8_t* active, const int32_t* row_offsets,
+                          const int32_t* neighbors, const int32_t* edge_ids) {
+  if (node + n > n_ || edge + m > m_ || entry + entries > adjacency_) {
+    throw std::logic_error("device CSR upload beyond its capacity");
+  }
+  items->push_back({kUploadFlags, active_.get() + edge, active, m});
+  items->push_back({kUploadWords, ro_[cur_].get() + node, row_offsets, n, 0, static_cast<uint32_t>(entry)});
+  items->push_back({kUploadWords, nb_[cur_].get() + entry, neighbors, entries, 0, static_cast<uint32_t>(node)});
+  items->push_back({kUploadWords, eid_[cur_].get() + entry, edge_ids, entries, 0, static_cast<uint32_t>(edge)});
+}
+
+void DeviceCsr::AddEnd(std::vector<UploadItem>* items, const int32_t* end) {
+  items->push_back({kUploadWords, ro_[cur_].get() + n_, end, 1});
 }
 
 void DeviceCsr::UploadCommits(hipStream_t stream) {

@@ -57,7 +57,7 @@ struct Fleet {
   DeviceArray<int32_t> d_witnesses;
   // device: active flags and CSR, updated by commits
   DeviceCsr csr;
-  Pinned<int32_t> h_active, h_row_offsets, h_neighbors, h_edge_ids, h_witnesses;
+  Pinned<int32_t> h_witnesses;
   // one captured epoch (commit, launch, download) per CSR buffer
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -135,47 +135,39 @@ struct Fleet {
     if (nodes >= (size_t{1} << 31) || slots >= (size_t{1} << 31) - 1 || adjacency >= (size_t{1} << 31)) {
       throw std::invalid_argument("JV fleet union exceeds int32 ids");
     }
-    std::vector<int2> uv(std::max<size_t>(slots, 1));
-    std::vector<int64_t> weight(std::max<size_t>(slots, 1));
-    std::vector<uint8_t> mode(std::max<size_t>(slots, 1));
-    std::vector<longlong2> xy(std::max<size_t>(nodes, 1));
-    ParallelFor(count, [&](size_t i) {
-      const JvHost& h = hosts[i];
-      const int32_t nb = static_cast<int32_t>(node_base[i]);
-      const uint8_t md = static_cast<uint8_t>((h.type & 1u) | (h.near ? 2u : 0u));
-      for (int32_t e = 0; e < h.m; ++e) {
-        const size_t s = edge_base[i] + static_cast<size_t>(e);
-        uv[s] = make_int2(nb + h.u[e], nb + h.v[e]);
-        weight[s] = h.weight[e];
-        mode[s] = md;
-      }
-      for (int32_t vtx = 0; vtx < h.n; ++vtx) xy[node_base[i] + vtx] = longlong2{h.x[vtx], h.y[vtx]};
-    });
+    std::vector<uint8_t> mode((std::max<size_t>(slots, 1) + 3) / 4 * 4);
     const int dev = ctx->device;
-    d_uv.Allocate(uv.size(), dev);
-    d_weight.Allocate(weight.size(), dev);
+    d_uv.Allocate(std::max<size_t>(slots, 1), dev);
+    d_weight.Allocate(std::max<size_t>(slots, 1), dev);
     d_mode.Allocate(mode.size(), dev);
-    d_xy.Allocate(xy.size(), dev);
-    d_witnesses.Allocate(uv.size(), dev);
+    d_xy.Allocate(std::max<size_t>(nodes, 1), dev);
+    d_witnesses.Allocate(std::max<size_t>(slots, 1), dev);
     // a commit deactivates each slot at most once
     csr.Allocate(nodes, slots, adjacency, slots, dev);
-    h_active.Reserve(uv.size());
-    h_witnesses.Reserve(uv.size());
-    h_row_offsets.Reserve(nodes + 1);
-    h_neighbors.Reserve(adjacency);
-    h_edge_ids.Reserve(adjacency);
-    d_uv.Upload(uv.data(), uv.size(), ctx->stream);
-    d_weight.Upload(weight.data(), weight.size(), ctx->stream);
-    d_mode.Upload(mode.data(), mode.size(), ctx->stream);
-    d_xy.Upload(xy.data(), xy.size(), ctx->stream);
-    ctx->Sync();
+    h_witnesses.Reserve(std::max<size_t>(slots, 1));
+    // the graphs' arrays go to the union as they are; endpoints become union
+    // node ids on the way
+    std::vector<UploadItem> items;
+    for (uint32_t i = 0; i < count; ++i) {
+      const JvHost& h = hosts[i];
+      const size_t m = static_cast<size_t>(h.m), n = static_cast<size_t>(h.n), eb = edge_base[i], nb = node_base[i];
+      std::memset(mode.data() + eb, (h.type & 1u) | (h.near ? 2u : 0u), m);
+      items.push_back({kUploadSpread32, d_uv.get() + eb, h.u.data(), m, 0, static_cast<uint32_t>(nb), 0});
+      items.push_back({kUploadSpread32, d_uv.get() + eb, h.v.data(), m, 0, static_cast<uint32_t>(nb), 1});
+      items.push_back({kUploadWords, d_weight.get() + eb, h.weight.data(), 2 * m});
+      items.push_back({kUploadSpread64, d_xy.get() + nb, h.x.data(), n, 0, 0, 0});
+      items.push_back({kUploadSpread64, d_xy.get() + nb, h.y.data(), n, 0, 0, 1});
+    }
+    items.push_back({kUploadWords, d_mode.get(), mode.data(), mode.size() / 4});
+    UploadItems(*ctx, items);
     // one hash segment per graph, each continuing from its own prefix
     std::vector<int32_t> node_offset(count);
-    for (uint32_t i = 0; i < count; ++i) node_offset[i] = static_cast<int32_t>(node_base[i]);
-    dhash.Allocate(edge_base, dev, ctx->stream, node_offset);
     std::vector<uint64_t> prefixes(count);
-    for (uint32_t i = 0; i < count; ++i) prefixes[i] = hosts[i].prefix_hash();
-    dhash.SetPrefixes(prefixes.data(), ctx->stream);
+    for (uint32_t i = 0; i < count; ++i) {
+      node_offset[i] = static_cast<int32_t>(node_base[i]);
+      prefixes[i] = hosts[i].prefix_hash();
+    }
+    dhash.Allocate(*ctx, edge_base, prefixes.data(), node_offset);
     CheckHip(hipStreamCreateWithFlags(&hash_stream, hipStreamNonBlocking), "hipStreamCreate");
     CheckHip(hipEventCreateWithFlags(&ev_flags, hipEventDisableTiming), "hipEventCreate");
     CheckHip(hipEventCreateWithFlags(&ev_hashed, hipEventDisableTiming), "hipEventCreate");
@@ -186,25 +178,18 @@ struct Fleet {
   }
 
   // The union's active flags and CSR from the host snapshots (first epoch).
-  size_t AssembleFull() {
-    std::vector<size_t> adj_base(hosts.size() + 1, 0);
-    for (size_t i = 0; i < hosts.size(); ++i) adj_base[i + 1] = adj_base[i] + hosts[i].neighbors.size();
-    const size_t adj = adj_base[hosts.size()];
-    if (adj > adjacency) throw std::logic_error("JV fleet adjacency grew");
-    ParallelFor(hosts.size(), [&](size_t i) {
+  void UploadFull() {
+    std::vector<UploadItem> items;
+    size_t adj = 0;
+    for (size_t i = 0; i < hosts.size(); ++i) {
       const JvHost& h = hosts[i];
-      const size_t eb = edge_base[i], nb = node_base[i], ab = adj_base[i];
-      for (int32_t e = 0; e < h.m; ++e) h_active.get()[eb + e] = h.active[e] ? 1 : 0;
-      for (int32_t vtx = 0; vtx < h.n; ++vtx) {
-        h_row_offsets.get()[nb + vtx] = static_cast<int32_t>(ab) + h.row_offsets[vtx];
-      }
-      for (size_t s = 0; s < h.neighbors.size(); ++s) {
-        h_neighbors.get()[ab + s] = static_cast<int32_t>(nb) + h.neighbors[s];
-        h_edge_ids.get()[ab + s] = static_cast<int32_t>(eb) + h.edge_ids[s];
-      }
-    });
-    h_row_offsets.get()[nodes] = static_cast<int32_t>(adj);
-    return adj;
+      csr.AddUpload(&items, node_base[i], static_cast<size_t>(h.n), edge_base[i], static_cast<size_t>(h.m), adj,
+                    h.neighbors.size(), h.active.data(), h.row_offsets.data(), h.neighbors.data(), h.edge_ids.data());
+      adj += h.neighbors.size();
+    }
+    const int32_t end = static_cast<int32_t>(adj);
+    csr.AddEnd(&items, &end);
+    UploadItems(*ctx, items);
   }
 
   // The union commit list of this epoch into the CSR's pinned staging: each
@@ -270,8 +255,7 @@ struct Fleet {
   // commit the staged list on the device.
   void EnqueueEpoch(bool first, bool use_graph, ee_jv_fleet_stats* st) {
     if (first) {
-      const size_t adj = AssembleFull();
-      csr.Upload(h_active.get(), h_row_offsets.get(), h_neighbors.get(), h_edge_ids.get(), adj, ctx->stream);
+      UploadFull();
       CheckHip(hipEventRecord(ctx->ev_begin, ctx->stream), "event record");
       EnqueueLaunch();
       return;

@@ -38,12 +38,11 @@ class DeviceContentHash {
   // Segment s owns edge slots [first[s], first[s + 1]); first is ascending,
   // with one more entry than there are segments.  node_offset[s] (or 0 for
   // every segment when empty) is subtracted from the stored endpoints before
-  // hashing: a union of graphs stores endpoints as union node ids.  Uploads
-  // the chunk, group and segment tables on `stream` and waits for them.
-  void Allocate(const std::vector<size_t>& first, int device, hipStream_t stream,
+  // hashing: a union of graphs stores endpoints as union node ids.
+  // prefixes: the segments' hashes so far (host values, one per segment).
+  // Uploads everything through the context's ring and waits.
+  void Allocate(Context& ctx, const std::vector<size_t>& first, const uint64_t* prefixes,
                 const std::vector<int32_t>& node_offset = {});
-  // The segments' prefixes (host values, one per segment), uploaded on stream.
-  void SetPrefixes(const uint64_t* prefixes, hipStream_t stream);
   // Enqueues on `stream` the hash of every segment's edge part (per slot u,
   // v, weight, active != 0) into out[s] (device memory, one per segment).
   void Enqueue(const int2* uv, const int64_t* weight, const int32_t* active, uint64_t* out, hipStream_t stream);

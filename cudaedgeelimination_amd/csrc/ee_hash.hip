@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kThreads) void ChunkSumKernel(const Chunk* __restri
 
 }  // namespace
 
-void DeviceContentHash::Allocate(const std::vector<size_t>& first, int device, hipStream_t stream,
+void DeviceContentHash::Allocate(Context& ctx, const std::vector<size_t>& first, const uint64_t* prefixes,
                                  const std::vector<int32_t>& node_offset) {
   if (first.size() < 2) throw std::invalid_argument("device content hash: no segments");
   if (!node_offset.empty() && node_offset.size() + 1 != first.size()) {
@@ -250,6 +250,7 @@ void DeviceContentHash::Allocate(const std::vector<size_t>& first, int device, h
   segments_ = sg.size();
   chunks_ = ch.size();
   groups_ = gr.size();
+  const int device = ctx.device;
   chunk_desc_.Allocate(std::max<size_t>(chunks_, 1), device);
   group_desc_.Allocate(std::max<size_t>(groups_, 1), device);
   segment_desc_.Allocate(segments_, device);
@@ -258,16 +259,10 @@ void DeviceContentHash::Allocate(const std::vector<size_t>& first, int device, h
   group_perm_.Allocate(std::max<size_t>(groups_, 1) * kStates, device);
   chunk_start_.Allocate(std::max<size_t>(chunks_, 1), device);
   group_start_.Allocate(std::max<size_t>(groups_, 1), device);
-  if (chunks_ > 0) chunk_desc_.Upload(ch.data(), chunks_, stream);
-  if (groups_ > 0) group_desc_.Upload(gr.data(), groups_, stream);
-  segment_desc_.Upload(sg.data(), segments_, stream);
-  CheckHip(hipStreamSynchronize(stream), "hipStreamSynchronize");
-}
-
-void DeviceContentHash::SetPrefixes(const uint64_t* prefixes, hipStream_t stream) {
-  if (segments_ == 0) throw std::logic_error("device content hash not allocated");
-  prefixes_.Upload(prefixes, segments_, stream);
-  CheckHip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  UploadItems(ctx, {{kUploadWords, chunk_desc_.get(), ch.data(), chunks_ * (sizeof(Chunk) / 4)},
+                    {kUploadWords, group_desc_.get(), gr.data(), groups_ * (sizeof(Group) / 4)},
+                    {kUploadWords, segment_desc_.get(), sg.data(), segments_ * (sizeof(Segment) / 4)},
+                    {kUploadWords, prefixes_.get(), prefixes, segments_ * 2}});
 }
 
 void DeviceContentHash::Enqueue(const int2* uv, const int64_t* weight, const int32_t* active, uint64_t* out,
@@ -331,8 +326,7 @@ ee_status ee_graph_content_hash_hip(ee_ctx* handle, int32_t n, uint8_t distance_
     d_weight.Upload(edge_weight, count, ctx->stream);
     d_active.Upload(active.data(), count, ctx->stream);
     ee::DeviceContentHash h;
-    h.Allocate({0, count}, ctx->device, ctx->stream);
-    h.SetPrefixes(&prefix, ctx->stream);
+    h.Allocate(*ctx, {0, count}, &prefix);
     h.Enqueue(d_uv.get(), d_weight.get(), d_active.get(), d_out.get(), ctx->stream);
     d_out.Download(hash, 1, ctx->stream);
     ctx->Sync();

@@ -473,15 +473,13 @@ void UploadHtGraph(Context& ctx, const ee_graph_view& g) {
   const size_t a = static_cast<size_t>(g.row_offsets[g.dimension]);
   c.valid = false;
   c.last_kind = 0;  // verdict bits go with their snapshot
-  std::vector<longlong2> xy(n);
-  for (size_t i = 0; i < n; ++i) xy[i] = make_longlong2(g.x[i], g.y[i]);
   c.d_xy.Allocate(n, ctx.device);
   c.d_row_offsets.Allocate(n + 1, ctx.device);
   c.d_neighbors.Allocate(std::max<size_t>(a, 1), ctx.device);
-  c.d_xy.Upload(xy.data(), n, ctx.stream);
-  c.d_row_offsets.Upload(g.row_offsets, n + 1, ctx.stream);
-  c.d_neighbors.Upload(g.neighbors, a, ctx.stream);
-  ctx.Sync();
+  UploadItems(ctx, {{kUploadSpread64, c.d_xy.get(), g.x, n, 0, 0, 0},
+                    {kUploadSpread64, c.d_xy.get(), g.y, n, 0, 0, 1},
+                    {kUploadWords, c.d_row_offsets.get(), g.row_offsets, n + 1},
+                    {kUploadWords, c.d_neighbors.get(), g.neighbors, a}});
   c.x.assign(g.x, g.x + n);
   c.y.assign(g.y, g.y + n);
   c.row_offsets.assign(g.row_offsets, g.row_offsets + n + 1);

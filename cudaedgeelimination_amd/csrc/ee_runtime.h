@@ -350,20 +350,27 @@ bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const Kopt
 // context's ring.  wide: some instance's coordinates are not near.
 void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide, int64_t* cells);
 
-// Where a snapshot's active flags (as words) and CSR go on the device, and
-// the bounds of its node ids and edge slots.
-struct JvDynamic {
-  int32_t *active, *row_offsets, *neighbors, *edge_ids;
-  uint32_t nodes, slots;
+// An array on its way to the device: `count` elements of `from`, caller or
+// host memory, to the device address `to`.
+enum UploadKind : uint32_t {
+  kUploadWords,     // 32-bit words plus `add`; with a limit, words below it
+  kUploadFlags,     // bytes to 32-bit 0 or 1
+  kUploadSpread32,  // 32-bit words plus `add` to component `lane` of pairs
+  kUploadSpread64,  // 64-bit words to component `lane` of pairs
 };
-
-// Copies the snapshot's active flags and CSR (whose row offsets the caller
-// has checked) to the device through the context's ring; `then` runs once the
-// last part is queued, with the snapshot in place for work it queues on the
-// context's stream.  False if some neighbour or edge id is out of range; the
-// device then holds 0 in its place.
-bool UploadJvDynamic(Context& ctx, const ee_graph_view& g, size_t adjacency, const JvDynamic& to,
-                     const std::function<void()>& then);
+struct UploadItem {
+  UploadKind kind;
+  void* to;
+  const void* from;
+  size_t count;
+  uint32_t limit = 0, add = 0, lane = 0;
+};
+// Copies the items to the device through the context's ring, in few launches
+// and no copy command; `then` runs once the last part is queued, with the
+// arrays in place for work it queues on the context's stream.  Returns once
+// the arrays are in place; false if some word reached its limit (the device
+// then holds `add` alone in its place).
+bool UploadItems(Context& ctx, const std::vector<UploadItem>& items, const std::function<void()>& then = [] {});
 
 // Elements [offset, offset + count) of a device array into caller memory, as
 // DownloadToCaller.

@@ -46,15 +46,6 @@ KoptInstance MakeKoptInstance(uint64_t coord_base, const int64_t* x, const int64
   return inst;
 }
 
-std::vector<longlong2> Interleave(const int64_t* x, const int64_t* y, int32_t n) {
-  std::vector<longlong2> xy(static_cast<size_t>(n));
-  for (int32_t i = 0; i < n; ++i) {
-    xy[static_cast<size_t>(i)].x = x[i];
-    xy[static_cast<size_t>(i)].y = y[i];
-  }
-  return xy;
-}
-
 // ------------------------------------------------------------------ device
 int CountDevices() {
   int count = 0;
@@ -194,16 +185,14 @@ bool PrepareJvStatic(Context& ctx, const ee_graph_view& g) {
   if (StaticMatches(c, g)) return true;
   ValidateStaticJv(g);
   const size_t n = static_cast<size_t>(g.dimension), m = static_cast<size_t>(g.edge_count);
-  std::vector<int2> uv(m);
-  for (size_t e = 0; e < m; ++e) uv[e] = make_int2(g.edge_u[e], g.edge_v[e]);
-  const std::vector<longlong2> xy = Interleave(g.x, g.y, g.dimension);
   DeviceArray<int2> d_uv(m, ctx.device);
   DeviceArray<int64_t> d_weight(m, ctx.device);
   DeviceArray<longlong2> d_xy(n, ctx.device);
-  d_uv.Upload(uv.data(), m, ctx.stream);
-  d_weight.Upload(g.edge_weight, m, ctx.stream);
-  d_xy.Upload(xy.data(), n, ctx.stream);
-  ctx.Sync();
+  UploadItems(ctx, {{kUploadSpread32, d_uv.get(), g.edge_u, m, 0, 0, 0},
+                    {kUploadSpread32, d_uv.get(), g.edge_v, m, 0, 0, 1},
+                    {kUploadWords, d_weight.get(), g.edge_weight, 2 * m},
+                    {kUploadSpread64, d_xy.get(), g.x, n, 0, 0, 0},
+                    {kUploadSpread64, d_xy.get(), g.y, n, 0, 0, 1}});
   c.d_uv = std::move(d_uv);
   c.d_weight = std::move(d_weight);
   c.d_xy = std::move(d_xy);
@@ -306,12 +295,13 @@ void FindJvCandidates(Context& ctx, const ee_graph_view& g, int32_t* witnesses, 
     workspace_hit =
         PrepareJvWorkspace(ctx, static_cast<size_t>(g.dimension), static_cast<size_t>(m), adjacency) && workspace_hit;
     auto t0 = std::chrono::steady_clock::now();
-    const JvDynamic to{c.d_active.get(),  c.d_row_offsets.get(),
-                       c.d_neighbors.get(), c.d_edge_ids.get(),
-                       static_cast<uint32_t>(g.dimension), static_cast<uint32_t>(m)};
-    const bool accepted = UploadJvDynamic(ctx, g, adjacency, to, [&] {
-      LaunchJv(JvArgs(ctx, m, g.distance_type), ctx.jv_grid, ctx.stream);
-    });
+    const bool accepted = UploadItems(
+        ctx,
+        {{kUploadFlags, c.d_active.get(), g.edge_active, static_cast<size_t>(m)},
+         {kUploadWords, c.d_row_offsets.get(), g.row_offsets, static_cast<size_t>(g.dimension) + 1},
+         {kUploadWords, c.d_neighbors.get(), g.neighbors, adjacency, static_cast<uint32_t>(g.dimension)},
+         {kUploadWords, c.d_edge_ids.get(), g.csr_edge_ids, adjacency, static_cast<uint32_t>(m)}},
+        [&] { LaunchJv(JvArgs(ctx, m, g.distance_type), ctx.jv_grid, ctx.stream); });
     u.h2d_ms = MsSince(t0);
     t0 = std::chrono::steady_clock::now();
     if (!accepted) {
@@ -392,10 +382,8 @@ KoptHits PrepareKoptCaches(Context& ctx, const int64_t* x, const int64_t* y, int
       throw std::invalid_argument("k-opt cost needs distance-safe integer coordinates");
     }
     const size_t nn = static_cast<size_t>(n);
-    const std::vector<longlong2> xy = Interleave(x, y, n);
     DeviceArray<longlong2> d_xy(nn, ctx.device);
-    d_xy.Upload(xy.data(), nn, ctx.stream);
-    ctx.Sync();
+    UploadItems(ctx, {{kUploadSpread64, d_xy.get(), x, nn, 0, 0, 0}, {kUploadSpread64, d_xy.get(), y, nn, 0, 0, 1}});
     c.d_xy = std::move(d_xy);
     c.x.assign(x, x + nn);
     c.y.assign(y, y + nn);

@@ -46,7 +46,6 @@ struct Session {
 
   Context* ctx;
   JvHost host;
-  std::vector<int32_t> active32;
   Pinned<int32_t> witnesses;
   hipEvent_t ev_compact = nullptr;
   // snapshot hashes on the device: one slot per generation of a run
@@ -71,12 +70,11 @@ struct Session {
 
   void UploadFull(double* h2d_ms) {
     const auto t0 = std::chrono::steady_clock::now();
-    const int32_t m = host.m;
-    active32.resize(static_cast<size_t>(m));
-    for (int32_t e = 0; e < m; ++e) active32[e] = host.active[e] ? 1 : 0;
-    csr.Upload(active32.data(), host.row_offsets.data(), host.neighbors.data(), host.edge_ids.data(),
-               host.neighbors.size(), ctx->stream);
-    ctx->Sync();
+    std::vector<UploadItem> items;
+    csr.AddUpload(&items, 0, static_cast<size_t>(host.n), 0, static_cast<size_t>(host.m), 0, host.neighbors.size(),
+                  host.active.data(), host.row_offsets.data(), host.neighbors.data(), host.edge_ids.data());
+    csr.AddEnd(&items, &host.row_offsets[static_cast<size_t>(host.n)]);
+    UploadItems(*ctx, items);
     *h2d_ms += MsSince(t0);
   }
 
@@ -241,10 +239,6 @@ ee_status ee_jv_session_create(ee_ctx* handle, const ee_graph_view* g, ee_jv_ses
     s->host.Load(g);
     const ee::JvHost& h = s->host;
     const size_t n = static_cast<size_t>(h.n), m = static_cast<size_t>(h.m);
-    std::vector<int2> uv(m);
-    std::vector<longlong2> xy(n);
-    for (size_t e = 0; e < m; ++e) uv[e] = make_int2(h.u[e], h.v[e]);
-    for (size_t i = 0; i < n; ++i) xy[i] = longlong2{h.x[i], h.y[i]};
     s->d_uv.Allocate(std::max<size_t>(m, 1), ctx->device);
     s->d_weight.Allocate(std::max<size_t>(m, 1), ctx->device);
     s->d_xy.Allocate(n, ctx->device);
@@ -253,20 +247,20 @@ ee_status ee_jv_session_create(ee_ctx* handle, const ee_graph_view* g, ee_jv_ses
     // at most every slot active (2 CSR entries each), at most every slot per commit
     s->csr.Allocate(n, m, 2 * m, m, ctx->device);
     ee::CheckHip(hipEventCreate(&s->ev_compact), "hipEventCreate");
-    s->d_uv.Upload(uv.data(), m, ctx->stream);
-    s->d_weight.Upload(h.weight.data(), m, ctx->stream);
-    s->d_xy.Upload(xy.data(), n, ctx->stream);
+    ee::UploadItems(*ctx, {{ee::kUploadSpread32, s->d_uv.get(), h.u.data(), m, 0, 0, 0},
+                           {ee::kUploadSpread32, s->d_uv.get(), h.v.data(), m, 0, 0, 1},
+                           {ee::kUploadWords, s->d_weight.get(), h.weight.data(), 2 * m},
+                           {ee::kUploadSpread64, s->d_xy.get(), h.x.data(), n, 0, 0, 0},
+                           {ee::kUploadSpread64, s->d_xy.get(), h.y.data(), n, 0, 0, 1}});
     if (m > 0) {
-      s->dhash.Allocate({0, m}, ctx->device, ctx->stream);
       const uint64_t prefix = s->host.prefix_hash();
-      s->dhash.SetPrefixes(&prefix, ctx->stream);
+      s->dhash.Allocate(*ctx, {0, m}, &prefix);
       ee::CheckHip(hipStreamCreateWithFlags(&s->hash_stream, hipStreamNonBlocking), "hipStreamCreate");
       ee::CheckHip(hipEventCreateWithFlags(&s->ev_flags, hipEventDisableTiming), "hipEventCreate");
       ee::CheckHip(hipEventCreateWithFlags(&s->ev_hashed, hipEventDisableTiming), "hipEventCreate");
       ee::Session* raw = s.get();
       s->host.hash_source = [raw](std::shared_future<uint64_t>* job) { return raw->HashOfNewGeneration(job); };
     }
-    ctx->Sync();
     *out = reinterpret_cast<ee_jv_session*>(s.release());
   });
 }

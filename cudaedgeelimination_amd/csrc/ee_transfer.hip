@@ -118,68 +118,83 @@ __global__ __launch_bounds__(kIngestRows) void IngestRows(const uint32_t* __rest
   }
 }
 
-// One stretch of a snapshot's dynamic arrays in a slot: elements [first,
-// first + count) of `array`, from byte `at` of the slot (16-byte aligned).
-enum JvArray : uint32_t { kJvActive, kJvRowOffsets, kJvNeighbors, kJvEdgeIds };
-struct JvPiece {
-  uint32_t array, at;
-  uint64_t first;
-  uint32_t count, reserved;
-};
-constexpr uint32_t kJvPieces = 4;  // a slot holds at most one stretch of each array
+constexpr uint32_t kPartThreads = 256;
+constexpr uint32_t kPartBytes = 8192;  // of a part in a slot, at most; 4096 and 2048 measured slower
 
-struct JvIngest {
-  JvDynamic to;
-  const char* staged;  // the slot: the refusal flag, then the pieces
-  uint32_t* refused;
-  uint64_t* marks;     // [gridDim.x]
-  uint64_t mark;
-  JvPiece pieces[kJvPieces];
+// A part of an upload item in a slot: `count` elements from byte `at` of the
+// slot (16-byte aligned) to `to`.
+struct UploadPart {
+  uint64_t to;
+  uint32_t at, count, kind, limit, add, lane;
 };
+static_assert(sizeof(UploadPart) == 32, "parts are read as whole 32-byte records");
 
-// The slot's stretches to the device arrays, active flags widened to words,
-// ids checked (one out of range is stored as 0 and refuses the call).  PCIe
-// bounds it; the blocks read whole words in a row.
-constexpr uint32_t kJvBlocks = 256;
-__global__ __launch_bounds__(256) void IngestJv(JvIngest g) {
-  const uint32_t self = blockIdx.x * 256 + threadIdx.x, all = gridDim.x * 256;
+// The parts of a slot to their arrays, in the forms of UploadKind.  A value
+// at or above its limit is stored as `add` alone and refuses the upload.
+// PCIe bounds it: a block holds a whole part in registers before it stores,
+// and many blocks keep the link busy (1.44 MB of a JV call, host copy
+// included, 67 us; parts of 2 KiB 95 us).  marks[b] once block b is done.
+// Against copy commands from caller memory, one per array: 64 graphs with
+// 435,000 edge slots built and uploaded in 2.5 ms, 5.1 ms before.
+__global__ __launch_bounds__(kPartThreads) void StoreParts(const UploadPart* __restrict__ parts, uint32_t count,
+                                                  const char* __restrict__ slot, uint32_t* __restrict__ refused,
+                                                  uint64_t* __restrict__ marks, uint64_t mark) {
+  constexpr uint32_t kHeld = kPartBytes / 4 / kPartThreads;  // a thread's words of a part, all in flight at once
+  const uint32_t t = threadIdx.x;
   bool bad = false;
-  for (uint32_t p = 0; p < kJvPieces; ++p) {  // uniform
-    const JvPiece piece = g.pieces[p];
-    if (piece.count == 0) continue;
-    const uint32_t* from = reinterpret_cast<const uint32_t*>(g.staged + piece.at);
-    if (piece.array == kJvActive) {
-      int32_t* to = g.to.active + piece.first;
-      for (uint32_t i = self; i < (piece.count + 3) / 4; i += all) {
-        const uint32_t flags = from[i];
+  for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {  // uniform
+    const UploadPart part = parts[i];
+    const uint32_t* from = reinterpret_cast<const uint32_t*>(slot + part.at);
+    int32_t* to = reinterpret_cast<int32_t*>(part.to);
+    if (part.kind == kUploadSpread64) {
+      const int64_t* from64 = reinterpret_cast<const int64_t*>(from);
+      int64_t* to64 = reinterpret_cast<int64_t*>(part.to);
+      int64_t v[kHeld / 2];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-          if (4 * i + u < piece.count) to[4 * i + u] = ((flags >> (8 * u)) & 0xffu) != 0 ? 1 : 0;
-        }
+      for (uint32_t j = 0; j < kHeld / 2; ++j) {
+        const uint32_t q = j * kPartThreads + t;
+        v[j] = q < part.count ? from64[q] : 0;
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < kHeld / 2; ++j) {
+        const uint32_t q = j * kPartThreads + t;
+        if (q < part.count) to64[2 * q + part.lane] = v[j];
       }
       continue;
     }
-    int32_t* to = (piece.array == kJvRowOffsets ? g.to.row_offsets
-                   : piece.array == kJvNeighbors ? g.to.neighbors
-                                                 : g.to.edge_ids) + piece.first;
-    const uint32_t limit = piece.array == kJvRowOffsets ? 0xffffffffu
-                           : piece.array == kJvNeighbors ? g.to.nodes
-                                                         : g.to.slots;
-#pragma unroll 4
-    for (uint32_t i = self; i < piece.count; i += all) {
-      const uint32_t v = from[i];
-      bad |= v >= limit;
-      to[i] = v >= limit ? 0 : static_cast<int32_t>(v);
+    const uint32_t words = part.kind == kUploadFlags ? (part.count + 3) / 4 : part.count;
+    uint32_t v[kHeld];
+#pragma unroll
+    for (uint32_t j = 0; j < kHeld; ++j) {
+      const uint32_t q = j * kPartThreads + t;
+      v[j] = q < words ? from[q] : 0;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kHeld; ++j) {
+      const uint32_t q = j * kPartThreads + t;
+      if (q >= words) break;
+      if (part.kind == kUploadWords) {
+        const bool out = v[j] >= part.limit && part.limit != 0;
+        bad |= out;
+        to[q] = static_cast<int32_t>((out ? 0u : v[j]) + part.add);
+      } else if (part.kind == kUploadSpread32) {
+        to[2 * q + part.lane] = static_cast<int32_t>(v[j] + part.add);
+      } else {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          if (4 * q + u < part.count) to[4 * q + u] = ((v[j] >> (8 * u)) & 0xffu) != 0 ? 1 : 0;
+        }
+      }
     }
   }
   if (bad) {
-    __hip_atomic_store(g.refused, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(refused, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-    __hip_atomic_store(g.marks + blockIdx.x, g.mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(marks + blockIdx.x, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -372,69 +387,69 @@ bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const Kopt
   return !refused;
 }
 
-bool UploadJvDynamic(Context& ctx, const ee_graph_view& g, size_t adjacency, const JvDynamic& to,
-                     const std::function<void()>& then) {
-  // slots of 2 MiB: 1.4 MB through 512 KiB slots took 27 us more, the gaps
-  // between four launches
-  constexpr size_t kHeader = 256, room = kSlotBytes - kHeader;
-  const struct {
-    const char* from;
-    size_t count, element;
-  } arrays[kJvPieces] = {
-      {reinterpret_cast<const char*>(g.edge_active), static_cast<size_t>(g.edge_count), 1},
-      {reinterpret_cast<const char*>(g.row_offsets), static_cast<size_t>(g.dimension) + 1, 4},
-      {reinterpret_cast<const char*>(g.neighbors), adjacency, 4},
-      {reinterpret_cast<const char*>(g.csr_edge_ids), adjacency, 4}};
-  // slots filled one after the other with stretches of the arrays in turn
-  std::vector<std::array<JvPiece, kJvPieces>> plan;
-  size_t used = room, longest = 0;
-  for (uint32_t a = 0; a < kJvPieces; ++a) {
-    for (size_t first = 0; first < arrays[a].count;) {
-      if (room - used < 256) {
-        plan.emplace_back();
-        plan.back().fill(JvPiece{});
-        used = 0;
-      }
-      const size_t n = std::min(arrays[a].count - first, (room - used) / arrays[a].element);
-      plan.back()[a] = JvPiece{a, static_cast<uint32_t>(kHeader + used), first, static_cast<uint32_t>(n), 0};
-      used = std::min(room, (used + n * arrays[a].element + 15) / 16 * 16);
-      longest = std::max(longest, used);
+bool UploadItems(Context& ctx, const std::vector<UploadItem>& items, const std::function<void()>& then) {
+  constexpr size_t kHeader = 256, kMaxParts = 2048, kMaxBlocks = 1024;
+  constexpr size_t kTable = kMaxParts * sizeof(UploadPart), kData = kHeader + kTable;
+  // slots of 2 MiB, filled one after the other: 1.4 MB through four slots of
+  // 512 KiB took 27 us more, the gaps between the launches
+  constexpr size_t room = kSlotBytes - kData;
+  struct Slot {
+    std::vector<UploadPart> parts;
+    std::vector<const char*> from;
+    size_t used = 0;
+  };
+  std::vector<Slot> plan;
+  for (const UploadItem& item : items) {
+    const size_t element = item.kind == kUploadFlags ? 1 : item.kind == kUploadSpread64 ? 8 : 4;
+    const size_t out = item.kind == kUploadFlags ? 4 : item.kind == kUploadWords ? 4 : item.kind == kUploadSpread32 ? 8 : 16;
+    for (size_t first = 0; first < item.count;) {
+      // flags grow fourfold: a part of them holds a quarter
+      const size_t most = (item.kind == kUploadFlags ? kPartBytes / 4 : kPartBytes) / element;
+      const size_t n = std::min(item.count - first, most), bytes = (n * element + 15) / 16 * 16;
+      if (plan.empty() || plan.back().parts.size() == kMaxParts || room - plan.back().used < bytes) plan.emplace_back();
+      Slot& s = plan.back();
+      s.parts.push_back({reinterpret_cast<uint64_t>(item.to) + first * out, static_cast<uint32_t>(kData + s.used),
+                         static_cast<uint32_t>(n), static_cast<uint32_t>(item.kind), item.limit, item.add, item.lane});
+      s.from.push_back(static_cast<const char*>(item.from) + first * element);
+      s.used += bytes;
       first += n;
     }
   }
-  const size_t slot_bytes = (kHeader + longest + 255) / 256 * 256;
+  if (plan.empty()) {
+    then();
+    return true;
+  }
+  size_t longest = 0;
+  for (const Slot& s : plan) longest = std::max(longest, s.used);
+  const size_t slot_bytes = (kData + longest + 255) / 256 * 256;
   DirectIo& io = ctx.io;
   io.Reserve(std::min<size_t>(plan.size(), DirectIo::kSlots) * slot_bytes);
   uint64_t marks[DirectIo::kSlots] = {};
   bool refused = false;
+  const auto blocks_of = [&](size_t i) { return std::min(plan[i].parts.size(), kMaxBlocks); };
   ThroughRing(ctx, plan.size(), [&](size_t i, size_t slot) {
+    const Slot& s = plan[i];
     char* at = io.host() + slot * slot_bytes;
     *reinterpret_cast<uint32_t*>(at) = 0;
-    // 64 KiB at a time, on host threads where there is more of them
-    constexpr size_t kPart = size_t{64} << 10;
-    std::array<size_t, kJvPieces + 1> parts{};
-    for (uint32_t a = 0; a < kJvPieces; ++a) {
-      parts[a + 1] = parts[a] + (plan[i][a].count * arrays[a].element + kPart - 1) / kPart;
-    }
-    ParallelFor(parts[kJvPieces], [&](size_t part) {
-      uint32_t a = 0;
-      while (part >= parts[a + 1]) ++a;
-      const JvPiece& piece = plan[i][a];
-      const size_t b = (part - parts[a]) * kPart, bytes = piece.count * arrays[a].element;
-      std::memcpy(at + piece.at + b, arrays[a].from + piece.first * arrays[a].element + b, std::min(kPart, bytes - b));
-    }, parts[kJvPieces] < 6 ? 1 : 8);
-    JvIngest job{};
-    job.to = to;
-    job.staged = io.device() + slot * slot_bytes;
-    job.refused = reinterpret_cast<uint32_t*>(io.device() + slot * slot_bytes);
-    job.marks = io.device_marks(slot);
-    job.mark = marks[slot] = io.NextMark();
-    std::copy(plan[i].begin(), plan[i].end(), job.pieces);
-    hipLaunchKernelGGL(IngestJv, dim3(kJvBlocks), dim3(256), 0, ctx.stream, job);
-    CheckHip(hipGetLastError(), "IngestJv launch");
+    std::memcpy(at + kHeader, s.parts.data(), s.parts.size() * sizeof(UploadPart));
+    // sixteen parts at a time, on host threads where there are many
+    constexpr size_t kGroup = 16;
+    const size_t groups = (s.parts.size() + kGroup - 1) / kGroup;
+    ParallelFor(groups, [&](size_t g) {
+      for (size_t p = g * kGroup, e = std::min(s.parts.size(), p + kGroup); p < e; ++p) {
+        const size_t element = s.parts[p].kind == kUploadFlags ? 1 : s.parts[p].kind == kUploadSpread64 ? 8 : 4;
+        std::memcpy(at + s.parts[p].at, s.from[p], s.parts[p].count * element);
+      }
+    }, groups < 6 ? 1 : 8);
+    char* device = io.device() + slot * slot_bytes;
+    marks[slot] = io.NextMark();
+    hipLaunchKernelGGL(StoreParts, dim3(static_cast<uint32_t>(blocks_of(i))), dim3(kPartThreads), 0, ctx.stream,
+                       reinterpret_cast<const UploadPart*>(device + kHeader), static_cast<uint32_t>(s.parts.size()),
+                       device, reinterpret_cast<uint32_t*>(device), io.device_marks(slot), marks[slot]);
+    CheckHip(hipGetLastError(), "StoreParts launch");
     if (i + 1 == plan.size()) then();
-  }, [&](size_t, size_t slot) {
-    for (size_t b = 0; b < kJvBlocks; ++b) io.WaitTile(slot, b, marks[slot], ctx.stream);
+  }, [&](size_t i, size_t slot) {
+    for (size_t b = 0; b < blocks_of(i); ++b) io.WaitTile(slot, b, marks[slot], ctx.stream);
     refused = refused || *reinterpret_cast<const uint32_t*>(io.host() + slot * slot_bytes) != 0;
   });
   return !refused;

@@ -13,8 +13,8 @@ import pytest
 import _oracle as O
 from cudaedgeelimination_amd import _lib, backend
 from cudaedgeelimination_amd import workloads as W
-from cudaedgeelimination_amd.graph import CEIL_2D, EUC_2D
-from cudaedgeelimination_amd.resident import KoptBatch
+from cudaedgeelimination_amd.graph import CEIL_2D, EUC_2D, GraphSnapshot
+from cudaedgeelimination_amd.resident import JvFleet, JvSession, KoptBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -270,3 +270,39 @@ def test_jv_call_inputs(ctx, n, neighbors):
     got, usage = backend.find_jv_witnesses(moved, ctx)
     assert np.array_equal(got, O.OGraph.from_snapshot(moved).witnesses())
     assert not usage.static_hit and usage.workspace_hit
+
+
+@pytest.mark.parametrize("n, neighbors", [(3, 2), (682, 3), (1_023, 3), (1_024, 4), (1_025, 4), (2_049, 5),
+                                          (8_193, 6), (50_001, 8)])
+def test_session_snapshot_upload(ctx, n, neighbors):
+    """Sessions and fleets put their arrays in place in parts of at most 8 KiB: at
+    the edges of a part and over several slots, the device's snapshot is the
+    graph's, and the hashes (which read the endpoints, weights and flags) and
+    witnesses are the host's and the oracle's."""
+    say(f"session upload n={n}")
+    rng = np.random.default_rng(n)
+    graphs = []
+    for part in (n, 5, n // 2 + 3):
+        g = W.knn_graph(rng.integers(0, 1_000_000, part), rng.integers(0, 1_000_000, part), EUC_2D,
+                        min(neighbors, part - 1))
+        active = g.edge_active.copy()
+        active[:: 7] = 0
+        graphs.append(GraphSnapshot.from_edges(g.x, g.y, EUC_2D, g.edge_u, g.edge_v, g.edge_weight, active))
+    singles = []
+    for g in graphs:
+        s = JvSession(ctx, g)
+        run = s.run(1)
+        assert run.initial_hash == g.content_hash()
+        got = s.device_snapshot()
+        for name in ("edge_active", "row_offsets", "neighbors", "csr_edge_ids"):
+            assert np.array_equal(got[name], getattr(g, name)), name
+        s.close()
+        s = JvSession(ctx, g)
+        singles.append(O.canonical_proof(s.run(100).proof))
+        s.close()
+    for use_graph in (False, True):
+        f = JvFleet(ctx, graphs)
+        f.run(100, use_graph)
+        for i, proof in enumerate(singles):
+            assert O.canonical_proof(f.proof(i)) == proof, i
+        f.close()
