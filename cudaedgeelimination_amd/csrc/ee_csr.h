@@ -22,7 +22,7 @@ class DeviceCsr {
  public:
   // n nodes, m edge slots, at most `adjacency` CSR entries, at most
   // `max_commits` slots per commit.
-  void Allocate(size_t n, size_t m, size_t adjacency, size_t max_commits, int device);
+  void Allocate(size_t n, size_t m, size_t adjacency, size_t max_commits, int device, MemoryPool* pool);
   // Adds the upload of a snapshot to the current buffer: active flags (bytes)
   // of m edge slots from slot `edge`, and the rows of n nodes from node
   // `node`, whose entries start at entry `entry` and hold ids from 0 (union

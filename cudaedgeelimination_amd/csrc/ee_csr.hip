@@ -129,7 +129,8 @@ __global__ __launch_bounds__(kThreads) void CompactKernel(
 
 }  // namespace
 
-void DeviceCsr::Allocate(size_t n, size_t m, size_t adjacency, size_t max_commits, int device) {
+void DeviceCsr::Allocate(size_t n, size_t m, size_t adjacency, size_t max_commits, int device,
+                         MemoryPool* pool) {
   if (n >= (size_t{1} << 31) || m >= (size_t{1} << 31) || adjacency >= (size_t{1} << 31) ||
       max_commits >= (size_t{1} << 31) - 1) {
     throw std::invalid_argument("device CSR exceeds int32 ids");
@@ -139,18 +140,18 @@ void DeviceCsr::Allocate(size_t n, size_t m, size_t adjacency, size_t max_commit
   adjacency_ = std::max<size_t>(adjacency, 1);
   max_commits_ = max_commits;
   cur_ = 0;
-  active_.Allocate(std::max<size_t>(m, 1), device);
+  active_.Allocate(std::max<size_t>(m, 1), device, pool);
   for (int b = 0; b < 2; ++b) {
-    ro_[b].Allocate(n + 1, device);
-    nb_[b].Allocate(adjacency_, device);
-    eid_[b].Allocate(adjacency_, device);
+    ro_[b].Allocate(n + 1, device, pool);
+    nb_[b].Allocate(adjacency_, device, pool);
+    eid_[b].Allocate(adjacency_, device, pool);
   }
   const size_t blocks = (adjacency_ + kThreads - 1) / kThreads;
-  masks_.Allocate(blocks * kWavesPerBlock, device);
-  block_counts_.Allocate(blocks, device);
-  block_offsets_.Allocate(blocks + 1, device);
-  commits_.Allocate(max_commits + 1, device);
-  h_commits_.Reserve(max_commits + 1);
+  masks_.Allocate(blocks * kWavesPerBlock, device, pool);
+  block_counts_.Allocate(blocks, device, pool);
+  block_offsets_.Allocate(blocks + 1, device, pool);
+  commits_.Allocate(max_commits + 1, device, pool);
+  h_commits_.Reserve(max_commits + 1, pool);
   h_commits_.get()[0] = 0;
 }
 

@@ -42,7 +42,6 @@ struct Fleet {
     if (hash_stream != nullptr) static_cast<void>(hipStreamSynchronize(hash_stream));
     if (ev_flags != nullptr) static_cast<void>(hipEventDestroy(ev_flags));
     if (ev_hashed != nullptr) static_cast<void>(hipEventDestroy(ev_hashed));
-    if (hash_stream != nullptr) static_cast<void>(hipStreamDestroy(hash_stream));
   }
 
   Context* ctx;
@@ -67,7 +66,7 @@ struct Fleet {
   DeviceContentHash dhash;
   DeviceArray<uint64_t> d_hashes;
   std::vector<uint64_t> h_hashes;
-  hipStream_t hash_stream = nullptr;
+  hipStream_t hash_stream = nullptr;  // the context's
   hipEvent_t ev_flags = nullptr, ev_hashed = nullptr;
   size_t hash_slots = 0;      // enqueued this run
   bool hash_pending = false;  // new generations of this step take the newest slot
@@ -137,14 +136,15 @@ struct Fleet {
     }
     std::vector<uint8_t> mode((std::max<size_t>(slots, 1) + 3) / 4 * 4);
     const int dev = ctx->device;
-    d_uv.Allocate(std::max<size_t>(slots, 1), dev);
-    d_weight.Allocate(std::max<size_t>(slots, 1), dev);
-    d_mode.Allocate(mode.size(), dev);
-    d_xy.Allocate(std::max<size_t>(nodes, 1), dev);
-    d_witnesses.Allocate(std::max<size_t>(slots, 1), dev);
+    MemoryPool* const pool = &ctx->pool;
+    d_uv.Allocate(std::max<size_t>(slots, 1), dev, pool);
+    d_weight.Allocate(std::max<size_t>(slots, 1), dev, pool);
+    d_mode.Allocate(mode.size(), dev, pool);
+    d_xy.Allocate(std::max<size_t>(nodes, 1), dev, pool);
+    d_witnesses.Allocate(std::max<size_t>(slots, 1), dev, pool);
     // a commit deactivates each slot at most once
-    csr.Allocate(nodes, slots, adjacency, slots, dev);
-    h_witnesses.Reserve(std::max<size_t>(slots, 1));
+    csr.Allocate(nodes, slots, adjacency, slots, dev, pool);
+    h_witnesses.Reserve(std::max<size_t>(slots, 1), pool);
     // the graphs' arrays go to the union as they are; endpoints become union
     // node ids on the way
     std::vector<UploadItem> items;
@@ -168,7 +168,7 @@ struct Fleet {
       prefixes[i] = hosts[i].prefix_hash();
     }
     dhash.Allocate(*ctx, edge_base, prefixes.data(), node_offset);
-    CheckHip(hipStreamCreateWithFlags(&hash_stream, hipStreamNonBlocking), "hipStreamCreate");
+    hash_stream = ctx->HashStream();
     CheckHip(hipEventCreateWithFlags(&ev_flags, hipEventDisableTiming), "hipEventCreate");
     CheckHip(hipEventCreateWithFlags(&ev_hashed, hipEventDisableTiming), "hipEventCreate");
     for (uint32_t i = 0; i < count; ++i) {
@@ -302,7 +302,7 @@ struct Fleet {
     size_t max_m = 0;
     for (const JvHost& h : hosts) max_m = std::max(max_m, static_cast<size_t>(h.m));
     const size_t hash_capacity = (std::min<size_t>(max_rounds, max_m) + 1) * hosts.size();
-    if (d_hashes.count() < hash_capacity) d_hashes.Allocate(hash_capacity, ctx->device);
+    if (d_hashes.count() < hash_capacity) d_hashes.Allocate(hash_capacity, ctx->device, &ctx->pool);
     std::vector<const std::vector<int32_t>*> commits(hosts.size(), nullptr);
     auto t0 = std::chrono::steady_clock::now();
     EnqueueEpoch(true, use_graph, &st);

@@ -251,14 +251,15 @@ void DeviceContentHash::Allocate(Context& ctx, const std::vector<size_t>& first,
   chunks_ = ch.size();
   groups_ = gr.size();
   const int device = ctx.device;
-  chunk_desc_.Allocate(std::max<size_t>(chunks_, 1), device);
-  group_desc_.Allocate(std::max<size_t>(groups_, 1), device);
-  segment_desc_.Allocate(segments_, device);
-  prefixes_.Allocate(segments_, device);
-  perm_.Allocate(std::max<size_t>(chunks_, 1) * kStates, device);
-  group_perm_.Allocate(std::max<size_t>(groups_, 1) * kStates, device);
-  chunk_start_.Allocate(std::max<size_t>(chunks_, 1), device);
-  group_start_.Allocate(std::max<size_t>(groups_, 1), device);
+  MemoryPool* const pool = &ctx.pool;
+  chunk_desc_.Allocate(std::max<size_t>(chunks_, 1), device, pool);
+  group_desc_.Allocate(std::max<size_t>(groups_, 1), device, pool);
+  segment_desc_.Allocate(segments_, device, pool);
+  prefixes_.Allocate(segments_, device, pool);
+  perm_.Allocate(std::max<size_t>(chunks_, 1) * kStates, device, pool);
+  group_perm_.Allocate(std::max<size_t>(groups_, 1) * kStates, device, pool);
+  chunk_start_.Allocate(std::max<size_t>(chunks_, 1), device, pool);
+  group_start_.Allocate(std::max<size_t>(groups_, 1), device, pool);
   UploadItems(ctx, {{kUploadWords, chunk_desc_.get(), ch.data(), chunks_ * (sizeof(Chunk) / 4)},
                     {kUploadWords, group_desc_.get(), gr.data(), groups_ * (sizeof(Group) / 4)},
                     {kUploadWords, segment_desc_.get(), sg.data(), segments_ * (sizeof(Segment) / 4)},

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <charconv>
 #include <chrono>
 #include <condition_variable>
 #include <exception>
@@ -12,6 +13,7 @@
 #include <thread>
 #include <vector>
 #include <cstdio>
+#include <cstring>
 #include <sstream>
 #include <stdexcept>
 #include <tuple>
@@ -469,10 +471,32 @@ void JvHost::EndRun(double total_ms) {
   // V1 proof text (src/cpu/jv_elimination.cpp:324-368)
   std::ostringstream out;
   out << "CUDAEE_PROOF_V1\nbackend hip\ninitial_hash " << Hex(stats.initial_hash) << '\n';
+  // records by the thousand: numbers written in place, a snapshot's hash once
+  std::vector<std::string> hashes(snaps_.size());
+  std::string lines;
+  lines.reserve(records_.size() * 56);
   for (const Record& r : records_) {
-    out << "record " << r.epoch << ' ' << Hex(snaps_[r.snap].Get()) << ' ' << r.edge << ' ' << r.a << ' '
-        << r.b << " JV " << r.witness << '\n';
+    std::string& hash = hashes[r.snap];
+    if (hash.empty()) hash = Hex(snaps_[r.snap].Get());
+    char line[128] = "record ";
+    char* at = line + 7;
+    const auto number = [&](auto v) { at = std::to_chars(at, line + sizeof(line), v).ptr; };
+    const auto text = [&](const char* t, size_t count) { at = static_cast<char*>(std::memcpy(at, t, count)) + count; };
+    number(r.epoch);
+    text(" ", 1);
+    text(hash.data(), hash.size());
+    text(" ", 1);
+    number(r.edge);
+    text(" ", 1);
+    number(r.a);
+    text(" ", 1);
+    number(r.b);
+    text(" JV ", 4);
+    number(r.witness);
+    text("\n", 1);
+    lines.append(line, static_cast<size_t>(at - line));
   }
+  out << lines;
   for (const Metrics& mt : metrics_) {
     out << "metrics " << mt.epoch << ' ' << mt.before << ' ' << mt.proposed << ' ' << mt.verified
         << ' ' << mt.rejected << ' ' << mt.committed << ' ' << mt.propose_ms << ' ' << mt.verify_ms

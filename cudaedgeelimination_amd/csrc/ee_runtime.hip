@@ -97,7 +97,18 @@ Context::~Context() {
   kopt = KoptCache{};
   static_cast<void>(hipEventDestroy(ev_begin));
   static_cast<void>(hipEventDestroy(ev_end));
+  if (hash_stream != nullptr) {
+    static_cast<void>(hipStreamSynchronize(hash_stream));
+    static_cast<void>(hipStreamDestroy(hash_stream));
+  }
   static_cast<void>(hipStreamDestroy(stream));
+}
+
+hipStream_t Context::HashStream() {
+  if (hash_stream == nullptr) {
+    CheckHip(hipStreamCreateWithFlags(&hash_stream, hipStreamNonBlocking), "hipStreamCreate");
+  }
+  return hash_stream;
 }
 
 void Context::Activate() const { CheckHip(hipSetDevice(device), "hipSetDevice"); }

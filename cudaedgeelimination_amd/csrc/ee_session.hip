@@ -41,7 +41,6 @@ struct Session {
     if (ev_compact != nullptr) static_cast<void>(hipEventDestroy(ev_compact));
     if (ev_flags != nullptr) static_cast<void>(hipEventDestroy(ev_flags));
     if (ev_hashed != nullptr) static_cast<void>(hipEventDestroy(ev_hashed));
-    if (hash_stream != nullptr) static_cast<void>(hipStreamDestroy(hash_stream));
   }
 
   Context* ctx;
@@ -52,7 +51,7 @@ struct Session {
   DeviceContentHash dhash;
   DeviceArray<uint64_t> d_hashes;
   std::vector<uint64_t> h_hashes;
-  hipStream_t hash_stream = nullptr;
+  hipStream_t hash_stream = nullptr;  // the context's
   hipEvent_t ev_flags = nullptr, ev_hashed = nullptr;
   // a fault for tests of the fail-closed path: one witness of the next
   // epoch's host copy replaced before re-verification
@@ -171,7 +170,7 @@ struct Session {
     } else {
       // one hash per generation: the first, and one after each commit
       const size_t slots = static_cast<size_t>(std::min<uint64_t>(max_rounds, static_cast<uint64_t>(host.m))) + 1;
-      if (d_hashes.count() < slots) d_hashes.Allocate(slots, ctx->device);
+      if (d_hashes.count() < slots) d_hashes.Allocate(slots, ctx->device, &ctx->pool);
       // the first epoch uploads the host's snapshot (a run may follow another)
       UploadFull(&host.stats.h2d_ms);
       EnqueueHash();
@@ -239,13 +238,14 @@ ee_status ee_jv_session_create(ee_ctx* handle, const ee_graph_view* g, ee_jv_ses
     s->host.Load(g);
     const ee::JvHost& h = s->host;
     const size_t n = static_cast<size_t>(h.n), m = static_cast<size_t>(h.m);
-    s->d_uv.Allocate(std::max<size_t>(m, 1), ctx->device);
-    s->d_weight.Allocate(std::max<size_t>(m, 1), ctx->device);
-    s->d_xy.Allocate(n, ctx->device);
-    s->d_witnesses.Allocate(std::max<size_t>(m, 1), ctx->device);
-    s->witnesses.Reserve(std::max<size_t>(m, 1));
+    ee::MemoryPool* const pool = &ctx->pool;
+    s->d_uv.Allocate(std::max<size_t>(m, 1), ctx->device, pool);
+    s->d_weight.Allocate(std::max<size_t>(m, 1), ctx->device, pool);
+    s->d_xy.Allocate(n, ctx->device, pool);
+    s->d_witnesses.Allocate(std::max<size_t>(m, 1), ctx->device, pool);
+    s->witnesses.Reserve(std::max<size_t>(m, 1), pool);
     // at most every slot active (2 CSR entries each), at most every slot per commit
-    s->csr.Allocate(n, m, 2 * m, m, ctx->device);
+    s->csr.Allocate(n, m, 2 * m, m, ctx->device, pool);
     ee::CheckHip(hipEventCreate(&s->ev_compact), "hipEventCreate");
     ee::UploadItems(*ctx, {{ee::kUploadSpread32, s->d_uv.get(), h.u.data(), m, 0, 0, 0},
                            {ee::kUploadSpread32, s->d_uv.get(), h.v.data(), m, 0, 0, 1},
@@ -255,7 +255,7 @@ ee_status ee_jv_session_create(ee_ctx* handle, const ee_graph_view* g, ee_jv_ses
     if (m > 0) {
       const uint64_t prefix = s->host.prefix_hash();
       s->dhash.Allocate(*ctx, {0, m}, &prefix);
-      ee::CheckHip(hipStreamCreateWithFlags(&s->hash_stream, hipStreamNonBlocking), "hipStreamCreate");
+      s->hash_stream = ctx->HashStream();
       ee::CheckHip(hipEventCreateWithFlags(&s->ev_flags, hipEventDisableTiming), "hipEventCreate");
       ee::CheckHip(hipEventCreateWithFlags(&s->ev_hashed, hipEventDisableTiming), "hipEventCreate");
       ee::Session* raw = s.get();

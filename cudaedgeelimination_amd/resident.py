@@ -18,6 +18,15 @@ from .graph import GraphSnapshot
 TEMPLATES_PER_K = {3: 4, 4: 25, 5: 208}
 
 
+def _proof_text(read, *args) -> str:
+    """The text of a proof call: its length, then one copy and one decode."""
+    length = C.c_size_t()
+    _lib.check(read(*args, None, 0, C.byref(length)))
+    buf = np.empty(length.value + 1, np.uint8)
+    _lib.check(read(*args, C.cast(_lib.ptr(buf), C.c_char_p), len(buf), C.byref(length)))
+    return str(memoryview(buf)[:length.value], "utf-8")
+
+
 class KoptBatch:
     """Instances (coordinates) plus (instance, k, rows) segments evaluated in
     one launch; the cost output stays on the device until downloaded."""
@@ -208,13 +217,10 @@ class JvSession:
     def run(self, max_rounds: int = 100) -> JvRun:
         st = _lib.JvRunStats()
         _lib.check(_lib.lib().ee_jv_session_run(self._h, max_rounds, C.byref(st)))
-        length = C.c_size_t()
-        _lib.check(_lib.lib().ee_jv_session_proof(self._h, None, 0, C.byref(length)))
-        buf = C.create_string_buffer(length.value + 1)
-        _lib.check(_lib.lib().ee_jv_session_proof(self._h, buf, len(buf), C.byref(length)))
+        proof = _proof_text(_lib.lib().ee_jv_session_proof, self._h)
         return JvRun(st.epochs, st.edges_scanned, st.proposed, st.committed, st.initial_hash,
                      st.final_hash, st.device_ms, st.h2d_ms, st.d2h_ms, st.propose_ms,
-                     st.verify_ms, st.commit_ms, st.total_ms, buf.value.decode(), st.compact_ms,
+                     st.verify_ms, st.commit_ms, st.total_ms, proof, st.compact_ms,
                      st.hash_wait_ms)
 
     def inject_witness(self, edge: int, witness: int) -> None:
@@ -274,11 +280,7 @@ class JvFleet:
         return st.as_dict()
 
     def proof(self, index: int) -> str:
-        length = C.c_size_t()
-        _lib.check(_lib.lib().ee_jv_fleet_proof(self._h, index, None, 0, C.byref(length)))
-        buf = C.create_string_buffer(length.value + 1)
-        _lib.check(_lib.lib().ee_jv_fleet_proof(self._h, index, buf, len(buf), C.byref(length)))
-        return buf.value.decode()
+        return _proof_text(_lib.lib().ee_jv_fleet_proof, self._h, index)
 
     def instance_stats(self, index: int) -> dict:
         st = _lib.JvRunStats()

@@ -306,3 +306,34 @@ def test_session_snapshot_upload(ctx, n, neighbors):
         for i, proof in enumerate(singles):
             assert O.canonical_proof(f.proof(i)) == proof, i
         f.close()
+
+
+@pytest.mark.parametrize("order", [(40, 3_000, 40, 900, 3_000), (3_000, 2_900, 1_500, 3_000, 5)])
+def test_sessions_one_after_the_other(ctx, order):
+    """A context keeps the memory of closed sessions and fleets for the next:
+    whatever it held, and whatever is open beside it, the next run's proof is
+    a fresh context's."""
+    say(f"reused memory {order}")
+    graphs = [W.knn_graph(*np.random.default_rng(n).integers(0, 1_000_000, (2, n)), EUC_2D, 4) for n in order]
+
+    def alone(g):
+        own = backend.Context(0)
+        s = JvSession(own, g)
+        proof = O.canonical_proof(s.run(100).proof)
+        s.close()
+        own.close()
+        return proof
+
+    want = [alone(g) for g in graphs]
+    beside = JvSession(ctx, graphs[0])
+    for _ in range(2):
+        for g, proof in zip(graphs, want):
+            s = JvSession(ctx, g)
+            assert O.canonical_proof(s.run(100).proof) == proof
+            s.close()
+        f = JvFleet(ctx, graphs)
+        f.run(100)
+        assert [O.canonical_proof(f.proof(i)) for i in range(len(order))] == want
+        f.close()
+    assert O.canonical_proof(beside.run(100).proof) == want[0]
+    beside.close()
