@@ -143,7 +143,8 @@ struct KoptLaunch {
   // packed_lo non-null: instead of int64 cells, write each cell's transfer
   // form (ExpandCells): its low word to packed_lo[cell] and, on instances
   // that are not near, its high byte to packed_hi[cell], both in host memory;
-  // once tile i's cells are there, `mark` goes to marks[i].  Task rows are
+  // once tile i's cells are there, `mark` goes to marks[i] (marks null: the
+  // host waits for the launch instead).  Task rows are
   // then read as another agent's: node ids at or above bound_nodes read node 0.
   uint32_t* packed_lo;
   uint8_t* packed_hi;

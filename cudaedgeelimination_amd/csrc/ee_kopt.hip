@@ -658,9 +658,11 @@ __device__ void TileLoop(const KoptLaunch& a, const KoptPointers& bufs, char* sm
     if constexpr (kOut == kOutPacked || kMade) {
       // the tile's output, then its mark: the host takes a tile's output once
       // it sees the mark, while later tiles are still on their way
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-      if (lane == 0) {
-        __hip_atomic_store(a.marks + (tile - a.k_tile_begin[ki]), a.mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (a.marks != nullptr) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+        if (lane == 0) {
+          __hip_atomic_store(a.marks + (tile - a.k_tile_begin[ki]), a.mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
       }
     }
   }

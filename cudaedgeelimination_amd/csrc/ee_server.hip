@@ -5,10 +5,11 @@
 // rows, output buffer) and JV rechecks (JV graph, edge slots, witness
 // buffer).  One worker thread forms batches from the queue in arrival order
 // under a cell limit, a request limit and an HBM budget, and issues each
-// batch on one of `pipeline_depth` slots (own stream, device buffers and
-// pinned staging): upload tasks, tiles and edge lists, one launch of the
-// tiled k-opt kernel over all the batch's (graph, k) segments and one JV
-// launch over all its listed edge slots, download the results.  While a batch
+// batch on one of `pipeline_depth` slots (own stream and page-locked
+// buffers): one launch of the tiled k-opt kernel over all the batch's
+// (graph, k) segments and one JV launch over all its listed edge slots, which
+// read rows, tiles and edge lists from the slot's page-locked memory and write
+// cells (in transfer form) and witnesses there.  While a batch
 // is in flight the worker keeps admitting and issuing into a free slot, so
 // requests that arrive meanwhile overlap on the device.  A second thread
 // blocks on the oldest batch in flight, copies each request's results into
@@ -17,6 +18,11 @@
 // it until it finishes or another request arrives.  With one slot there is no
 // second thread: the worker issues, waits and completes each batch in turn
 // (the plain per-query path).
+//
+// Against copies in and out of device buffers on the slot's stream: a burst
+// of 60 mixed requests 475 -> 394 us, one request of 4,096 k = 5 rows 430 ->
+// 206 us (half the bytes cross PCIe), rechecks of 16,384 edge slots 74 -> 60
+// us, 75,000 slots and single rows the same.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -70,17 +76,16 @@ struct Request {
 struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t ev_begin = nullptr, ev_end = nullptr, ev_done = nullptr;
-  DeviceArray<ee_kopt_task> d_tasks;
-  DeviceArray<int64_t> d_costs;
-  DeviceArray<KoptTile> d_tiles;
+  // page-locked memory the kernels read and write in place
   Pinned<ee_kopt_task> h_tasks;
-  Pinned<int64_t> h_costs;
+  Pinned<uint8_t> h_cells;  // in transfer form: `plane` low words, then `plane` high bytes
   Pinned<KoptTile> h_tiles;
   std::vector<KoptSegment> segments;
-  DeviceArray<int32_t> d_jv_list, d_jv_out;
   Pinned<int32_t> h_jv_list, h_jv_out;
   std::vector<std::shared_ptr<Request>> requests;
   std::vector<uint64_t> offsets;
+  std::vector<uint8_t> wide;  // per request: some cell may need its high byte
+  uint64_t plane = 0;
   uint64_t bytes = 0;
   uint64_t batch_id = 0;
   bool busy = false;
@@ -235,7 +240,9 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
     size_t kopt_requests = 0;
     bool present[3] = {false, false, false};
     slot.offsets.clear();
+    slot.wide.clear();
     for (const auto& r : batch) {
+      slot.wide.push_back(!r->jv && worker_instances[r->graph].near == 0);
       if (r->jv) {
         slot.offsets.push_back(items);
         items += r->edges.size();
@@ -253,12 +260,10 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
     CheckHip(hipEventRecord(slot.ev_begin, slot.stream), "event record");
     if (kopt_requests > 0) {
       slot.h_tasks.Reserve(rows);
-      slot.h_costs.Reserve(cells);
+      slot.plane = (cells + kSegmentAlignCells - 1) / kSegmentAlignCells * kSegmentAlignCells;
+      slot.h_cells.Reserve(slot.plane * 5);
       slot.segments.resize(kopt_requests);
       slot.h_tiles.Reserve(tiles);
-      if (slot.d_tasks.count() < rows) slot.d_tasks.Allocate(Grow(slot.d_tasks.count(), rows), ctx->device);
-      if (slot.d_costs.count() < cells) slot.d_costs.Allocate(Grow(slot.d_costs.count(), cells), ctx->device);
-      if (slot.d_tiles.count() < tiles) slot.d_tiles.Allocate(Grow(slot.d_tiles.count(), tiles), ctx->device);
       uint64_t row = 0;
       size_t seg = 0;
       for (size_t i = 0; i < batch.size(); ++i) {
@@ -272,13 +277,13 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
       KoptAssignTiles(slot.segments.data(), kopt_requests, worker_instances.data(), plans.data(), tuning,
                       slot.h_tiles.get(), &a);
       if (a.tile_count != tiles) throw std::logic_error("server tile count mismatch");
-      slot.d_tasks.Upload(slot.h_tasks.get(), rows, slot.stream);
-      if (a.inline_count == 0) slot.d_tiles.Upload(slot.h_tiles.get(), tiles, slot.stream);
       a.xy = d_xy.get();
-      a.tiles = slot.d_tiles.get();
-      a.tasks = slot.d_tasks.get();
+      a.tiles = slot.h_tiles.device();
+      a.tasks = slot.h_tasks.device();
+      a.bound_nodes = UINT32_MAX;  // the rows are the slot's own, checked when submitted
       a.plans = d_plans.get();
-      a.costs = slot.d_costs.get();
+      a.packed_lo = reinterpret_cast<uint32_t*>(slot.h_cells.device());
+      a.packed_hi = slot.h_cells.device() + slot.plane * 4;
       bool near_only = true;
       for (const KoptSegment& sg : slot.segments) near_only = near_only && worker_instances[sg.instance].near != 0;
       const size_t shared = KoptPrepareLayout(&a, plans.data(), present, tuning, near_only);
@@ -287,8 +292,6 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
     if (items > 0) {
       slot.h_jv_list.Reserve(items);
       slot.h_jv_out.Reserve(items);
-      if (slot.d_jv_list.count() < items) slot.d_jv_list.Allocate(Grow(slot.d_jv_list.count(), items), ctx->device);
-      if (slot.d_jv_out.count() < items) slot.d_jv_out.Allocate(Grow(slot.d_jv_out.count(), items), ctx->device);
       for (size_t i = 0; i < batch.size(); ++i) {
         const Request& r = *batch[i];
         if (!r.jv) continue;
@@ -297,7 +300,6 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
         }
         std::memcpy(slot.h_jv_list.get() + slot.offsets[i], r.edges.data(), r.edges.size() * sizeof(int32_t));
       }
-      slot.d_jv_list.Upload(slot.h_jv_list.get(), items, slot.stream);
       JvLaunch j{};
       j.edge_count = static_cast<int32_t>(items);
       j.edge_uv = d_jv_uv.get();
@@ -307,14 +309,12 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
       j.neighbors = d_jv_neighbors.get();
       j.csr_edge_ids = d_jv_edge_ids.get();
       j.xy = d_jv_xy.get();
-      j.witnesses = slot.d_jv_out.get();
+      j.witnesses = slot.h_jv_out.device();
       j.edge_mode = d_jv_mode.get();
-      j.edge_list = slot.d_jv_list.get();
+      j.edge_list = slot.h_jv_list.device();
       LaunchJv(j, 0, slot.stream);
     }
     CheckHip(hipEventRecord(slot.ev_end, slot.stream), "event record");
-    if (kopt_requests > 0) slot.d_costs.Download(slot.h_costs.get(), cells, slot.stream);
-    if (items > 0) slot.d_jv_out.Download(slot.h_jv_out.get(), items, slot.stream);
     CheckHip(hipEventRecord(slot.ev_done, slot.stream), "event record");
     {
       std::lock_guard<std::mutex> lk(mu);
@@ -337,6 +337,7 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
     }
     return true;
   } catch (const std::exception& e) {
+    static_cast<void>(hipStreamSynchronize(slot.stream));  // a launch may still use the slot's memory
     Fail(batch, e.what());
     return false;
   }
@@ -345,16 +346,36 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
 void Server::Complete(Slot& slot) {
   float ms = 0.0f;
   static_cast<void>(hipEventElapsedTime(&ms, slot.ev_begin, slot.ev_end));
+  // the results in pieces, on host threads from 64 Ki cells up (below, waking
+  // them costs more than it saves: 75,000 witnesses alone took 170 us on eight
+  // threads, 158 on one; 852,000 cells 236 us on one, 206 on eight)
+  struct Piece {
+    size_t request;
+    uint64_t first, count;
+  };
+  constexpr uint64_t kPieceCells = 16384, kSerialCells = 65536;
+  std::vector<Piece> pieces;
+  uint64_t cells = 0;
   for (size_t i = 0; i < slot.requests.size(); ++i) {
-    Request& r = *slot.requests[i];
+    const uint64_t count = slot.requests[i]->cells;
+    if (!slot.requests[i]->jv) cells += count;
+    for (uint64_t f = 0; f < count; f += kPieceCells) pieces.push_back({i, f, std::min(kPieceCells, count - f)});
+  }
+  ParallelFor(pieces.size(), [&](size_t p) {
+    const Piece& piece = pieces[p];
+    const Request& r = *slot.requests[piece.request];
+    const uint64_t at = slot.offsets[piece.request] + piece.first;
     if (r.jv) {
       // union node ids back to the graph's own ids
-      const int32_t* w = slot.h_jv_out.get() + slot.offsets[i];
-      for (size_t j = 0; j < r.edges.size(); ++j) r.witnesses[j] = w[j] >= 0 ? w[j] - r.node_base : -1;
+      const int32_t* w = slot.h_jv_out.get() + at;
+      for (uint64_t j = 0; j < piece.count; ++j) r.witnesses[piece.first + j] = w[j] >= 0 ? w[j] - r.node_base : -1;
     } else {
-      std::memcpy(r.out, slot.h_costs.get() + slot.offsets[i], r.cells * sizeof(int64_t));
+      const uint8_t* packed = slot.h_cells.get();
+      ExpandCells(reinterpret_cast<const uint32_t*>(packed) + at,
+                  slot.wide[piece.request] != 0 ? packed + slot.plane * 4 + at : nullptr, piece.count,
+                  r.out + piece.first);
     }
-  }
+  }, cells < kSerialCells ? 1 : 8);
   std::lock_guard<std::mutex> lk(mu);
   const auto now = Clock::now();
   for (auto& r : slot.requests) {
@@ -646,13 +667,8 @@ ee_status ee_server_create(ee_ctx* handle, const ee_server_config* config, ee_se
     // plus the alignment padding between the requests of a batch
     const uint64_t max_pool = max_cells + ee::kSegmentAlignCells * config->max_batch_requests;
     for (ee::Slot& slot : s->slots) {
-      slot.d_tasks.Allocate(max_rows, ctx->device);
-      slot.d_costs.Allocate(max_pool, ctx->device);
-      slot.d_tiles.Allocate(max_rows, ctx->device);
-      slot.d_jv_list.Allocate(max_cells, ctx->device);
-      slot.d_jv_out.Allocate(max_cells, ctx->device);
       slot.h_tasks.Reserve(max_rows);
-      slot.h_costs.Reserve(max_pool);
+      slot.h_cells.Reserve(max_pool * 5);
       slot.h_tiles.Reserve(max_rows);
       slot.h_jv_list.Reserve(max_cells);
       slot.h_jv_out.Reserve(max_cells);

@@ -624,12 +624,12 @@ ee_status ee_jv_fleet_active(const ee_jv_fleet* fleet, uint32_t index, uint8_t* 
  * and JV rechecks (ee_server_submit_jv) from any thread; a worker thread packs whatever has arrived into the next
  * batched launch (continuous batching) as long as the batch stays within the
  * cell and HBM budgets, runs up to `pipeline_depth` batches concurrently on
- * separate streams (upload, kernel and download of one batch overlap with the
- * next), copies each request's cells to the caller's buffer and marks it
+ * separate streams (a batch's rows, kernels and results overlap with the
+ * next; kernels read and write page-locked memory in place), writes each request's cells to the caller's buffer and marks it
  * complete.  Cells are bit-identical to ee_kopt_eval_costs with the canonical
  * templates.  With max_batch_requests = 1 and pipeline_depth = 1 the server
- * is the plain per-query path: one synchronous upload, launch and download
- * per request, in arrival order. */
+ * is the plain per-query path: one launch per request, waited for, in
+ * arrival order. */
 typedef struct ee_server ee_server;
 
 typedef struct {

@@ -14,7 +14,7 @@ import _oracle as O
 from cudaedgeelimination_amd import _lib, backend
 from cudaedgeelimination_amd import workloads as W
 from cudaedgeelimination_amd.graph import CEIL_2D, EUC_2D, GraphSnapshot
-from cudaedgeelimination_amd.resident import JvFleet, JvSession, KoptBatch
+from cudaedgeelimination_amd.resident import JvFleet, JvSession, KoptBatch, KoptServer
 
 pytestmark = pytest.mark.gpu
 
@@ -337,3 +337,33 @@ def test_sessions_one_after_the_other(ctx, order):
         f.close()
     assert O.canonical_proof(beside.run(100).proof) == want[0]
     beside.close()
+
+
+@pytest.mark.parametrize("batching", [True, False])
+@pytest.mark.parametrize("rows, slots", [(1, 1), (9, 2), (300, 255), (6_000, 4_097)])
+def test_server_in_place(ctx, rows, slots, batching):
+    """Served batches read rows, tiles and edge lists from page-locked memory
+    and leave cells and witnesses there: near and wide instances in one batch
+    (with and without high bytes), several k, a request beyond the batch
+    limit, and JV rechecks beside them."""
+    say(f"server rows={rows} slots={slots} batching={batching}")
+    graphs = [graph(5, 400, EUC_2D, 1_000_000), graph(6, 700, CEIL_2D, 1 << 30)]
+    server = KoptServer(ctx, max_batch_cells=20_000, batching=batching)
+    ids = [server.add_graph(g) for g in graphs]
+    gj = W.knn_graph(*np.random.default_rng(9).integers(0, 1_000_000, (2, 1_000)), EUC_2D, 8)
+    jid = server.add_jv_graph(gj)
+    edges = np.arange(slots, dtype=np.int32)[::-1] % gj.edge_count
+    whole, _ = backend.find_jv_witnesses(gj, ctx)
+    requests, want = [], []
+    for i, g in enumerate(graphs):
+        for k in (3, 4, 5):
+            count = rows if k == 5 and i == 1 else min(rows, 40)
+            tasks = W.kopt_tasks(rows + k, g, np.full(count, k, np.uint8))
+            requests.append((ids[i], k, tasks))
+            want.append(O.kopt_costs(g.x, g.y, g.distance_type, k, tasks)[0])
+        requests.append((jid, 0, edges))
+        want.append(whole[edges])
+    for _ in range(3):
+        for (got, _), exact in zip(server.wait_many(server.submit_many(requests), 60_000), want):
+            assert np.array_equal(got, exact)
+    server.close()
