@@ -278,12 +278,13 @@ class DirectIo {
  public:
   static constexpr size_t kSlots = 2;
   static constexpr size_t kSlotTiles = 4096;
-  // The sizes the ring takes: the first when the context is made, which most
-  // calls fit, the next for large results, and what a call asks for beyond.
-  // Few steps, since fresh page-locked memory costs about 0.4 ms per MB.
-  static constexpr size_t kSizes[2] = {size_t{2} << 20, size_t{4} << 20};
-  // At least `bytes`; growing discards the contents (no kernel may be using them).
-  void Reserve(size_t bytes);
+  // The ring is made with the context and keeps its size: fresh page-locked
+  // memory costs about 0.4 ms per MB, which a first large call would pay (a
+  // ring of 2 MiB that grew to 4 made that of 4,096 k = 5 rows 1.5 ms, it is
+  // 0.5 ms now).  Half of it per slot; slots of 1 MiB in 2 took a third longer
+  // on large results (batch cells 400 -> 520 us).
+  static constexpr size_t kBytes = size_t{4} << 20, kSlotBytes = kBytes / kSlots;
+  void Create();
   char* host() { return mem_.get(); }
   char* device() { return device_; }
   uint64_t* device_marks(size_t slot) { return device_marks_ + slot * kSlotTiles; }

@@ -83,7 +83,7 @@ Context::Context(int requested) {
   CheckHip(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
   CheckHip(hipEventCreate(&ev_begin), "hipEventCreate");
   CheckHip(hipEventCreate(&ev_end), "hipEventCreate");
-  io.Reserve(0);  // the first calls find their ring
+  io.Create();
   hipDeviceProp_t prop{};
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
     compute_units = prop.multiProcessorCount;
@@ -425,12 +425,19 @@ KoptHits PrepareKoptCaches(Context& ctx, const int64_t* x, const int64_t* y, int
 // its output: mask words, or cells in transfer form (low words, then high
 // bytes on instances that are not near).
 struct KoptChunks {
-  static constexpr size_t kSlotBytes = size_t{4} << 20;
+  // One launch where everything fits the ring, slots of half of it otherwise:
+  // 16,384 k = 4 rows (2.4 MB) take 108 us in one launch and 138 in two.  A
+  // tile is 0.3 MB at most.  kPads: the parts of a slot start on 256 bytes.
+  static constexpr size_t kPads = 5 * 256;
 
   KoptChunks(size_t rows, uint32_t tile_rows, size_t position_bytes, size_t low_bytes, size_t high_bytes)
       : rows_(rows) {
     const size_t per_row = sizeof(ee_kopt_task) + position_bytes + low_bytes + high_bytes;
-    const size_t fit = std::min<size_t>(std::max<size_t>(kSlotBytes / per_row / tile_rows, 1), DirectIo::kSlotTiles);
+    const size_t tiles = (rows + tile_rows - 1) / tile_rows, tile_bytes = tile_rows * per_row;
+    const bool whole = tiles <= DirectIo::kSlotTiles && tiles * tile_bytes + kPads <= DirectIo::kBytes;
+    const size_t room = whole ? DirectIo::kBytes : DirectIo::kSlotBytes;
+    const size_t fit = std::min<size_t>((room - kPads) / tile_bytes, DirectIo::kSlotTiles);
+    if (fit == 0) throw std::logic_error("a k-opt tile exceeds the ring");
     count = (rows + fit * tile_rows - 1) / (fit * tile_rows);
     // launches of equal size, whole tiles each
     const size_t even = (rows + count - 1) / count;
@@ -517,7 +524,6 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
   const KoptChunks chunks(task_count, tile_rows, made ? 4 * k : 0, 4 * (masks ? mask_words : template_count),
                           wide ? template_count : 0);
   DirectIo& io = ctx.io;
-  io.Reserve(chunks.slots * chunks.slot_bytes);
 
   KoptInstance inst{};
   inst.n = static_cast<uint32_t>(n);

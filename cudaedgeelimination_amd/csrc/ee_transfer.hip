@@ -216,32 +216,16 @@ void ThroughRing(Context& ctx, size_t launches, Start&& start, Finish&& finish) 
   }
 }
 
-// A launch's share of the ring's second size.
-constexpr size_t kSlotBytes = size_t{2} << 20;
+constexpr size_t kSlotBytes = DirectIo::kSlotBytes;
 static_assert(kSlotBytes / 4 / kPackTile <= DirectIo::kSlotTiles, "a slot's tiles have marks");
-static_assert(kSlotBytes * DirectIo::kSlots <= DirectIo::kSizes[1], "the slots fit");
 
 }  // namespace
 
-void DirectIo::Reserve(size_t bytes) {
-  const auto device_of = [](void* host) {
-    void* d = nullptr;
-    CheckHip(hipHostGetDevicePointer(&d, host, 0), "hipHostGetDevicePointer");
-    return d;
-  };
-  if (marks_.count() == 0) {
-    marks_.Reserve(kSlots * kSlotTiles);
-    device_marks_ = static_cast<uint64_t*>(device_of(marks_.get()));
-  }
-  for (const size_t size : kSizes) {
-    if (bytes <= size) {
-      bytes = size;
-      break;
-    }
-  }
-  if (bytes <= mem_.count()) return;
-  mem_.Reserve(bytes);
-  device_ = static_cast<char*>(device_of(mem_.get()));
+void DirectIo::Create() {
+  marks_.Reserve(kSlots * kSlotTiles);
+  device_marks_ = marks_.device();
+  mem_.Reserve(kBytes);
+  device_ = mem_.device();
 }
 
 void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t stream) const {
@@ -284,7 +268,7 @@ void DirectIo::TakeCells(size_t slot, uint64_t mark, hipStream_t stream, const u
 // and no copy command.  21.8 MB of near cells (10.9 MB, 195 us of PCIe) take
 // 265 us, 26.8 MB in three downloads 365 us instead of 736.  Slots of 4 MiB
 // would save 30 us of gaps between launches, for 1.5 ms more of page-locked
-// memory in a context's first large download; launches alternating on two
+// memory when a context is made; launches alternating on two
 // streams, with slots of 1 or 2 MiB, measured slower (290-360 us).
 void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide, int64_t* cells) {
   if (count == 0) return;
@@ -295,7 +279,6 @@ void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide
   const size_t plane = launches == 1 ? (count + 255) / 256 * 256 : slot_cells;
   const size_t slot_bytes = plane * cell_bytes;
   DirectIo& io = ctx.io;
-  io.Reserve(std::min<size_t>(launches, DirectIo::kSlots) * slot_bytes);
   uint64_t marks[DirectIo::kSlots] = {};
   const auto cells_of = [&](size_t i) { return std::min(slot_cells, count - i * slot_cells); };
   ThroughRing(ctx, launches, [&](size_t i, size_t slot) {
@@ -323,7 +306,6 @@ void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes) {
   const size_t count = bytes / 4, launches = (count + kSlotWords - 1) / kSlotWords;
   const size_t slot_words = std::min(kSlotWords, count);
   DirectIo& io = ctx.io;
-  io.Reserve(std::min<size_t>(launches, DirectIo::kSlots) * slot_words * 4);
   uint64_t marks[DirectIo::kSlots] = {};
   const auto words_of = [&](size_t i) { return std::min(kSlotWords, count - i * kSlotWords); };
   ThroughRing(ctx, launches, [&](size_t i, size_t slot) {
@@ -357,7 +339,6 @@ bool UploadRows(Context& ctx, const ee_kopt_task* rows, size_t count, const Kopt
   const size_t launches = (count + kSlotRows - 1) / kSlotRows;
   const size_t slot_bytes = kHeader + std::min(kSlotRows, (count + 63) / 64 * 64) * sizeof(ee_kopt_task);
   DirectIo& io = ctx.io;
-  io.Reserve(std::min<size_t>(launches, DirectIo::kSlots) * slot_bytes);
   uint64_t marks[DirectIo::kSlots] = {};
   const auto rows_of = [&](size_t i) { return std::min(kSlotRows, count - i * kSlotRows); };
   bool refused = false;
@@ -423,7 +404,6 @@ bool UploadItems(Context& ctx, const std::vector<UploadItem>& items, const std::
   for (const Slot& s : plan) longest = std::max(longest, s.used);
   const size_t slot_bytes = (kData + longest + 255) / 256 * 256;
   DirectIo& io = ctx.io;
-  io.Reserve(std::min<size_t>(plan.size(), DirectIo::kSlots) * slot_bytes);
   uint64_t marks[DirectIo::kSlots] = {};
   bool refused = false;
   const auto blocks_of = [&](size_t i) { return std::min(plan[i].parts.size(), kMaxBlocks); };

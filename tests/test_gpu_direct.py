@@ -31,7 +31,9 @@ def graph(seed, n, dtype, box):
 
 @pytest.mark.parametrize("box", [1_000_000, 1 << 30])
 @pytest.mark.parametrize("k, rows", [(3, 1), (3, 63), (3, 65), (3, 70_000), (4, 15), (4, 17), (4, 2_731),
-                                     (5, 1), (5, 3), (5, 5), (5, 315), (5, 316), (5, 4_799), (5, 20_011)])
+                                     (5, 1), (5, 3), (5, 5), (5, 315), (5, 316), (5, 4_799), (5, 20_011),
+                                     # the whole ring in one launch, and two slots: near, then wide
+                                     (5, 4_760), (5, 4_764), (5, 3_848), (5, 3_852)])
 def test_rows_match_oracle(ctx, k, rows, box):
     say(f"direct k={k} rows={rows} box={box}")
     dtype = CEIL_2D if rows % 2 else EUC_2D
