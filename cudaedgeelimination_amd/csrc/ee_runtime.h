@@ -38,7 +38,7 @@ int CountDevices();
 // kept for the next: bounded, released with the context, one lock around it.
 // A block comes back only after the streams that used it were synchronised.
 // Allocating and freeing it anew took 110 us of a session's 270 us to create
-// and 95 us to close (7,200 edge slots), and 1.1 ms for 64 graphs.
+// and 95 us to close (15,836 edge slots), and 1.1 ms for 64 graphs.
 class MemoryPool {
  public:
   static constexpr size_t kMaxBlocks = 64, kMaxDevice = size_t{64} << 20, kMaxHost = size_t{8} << 20;
