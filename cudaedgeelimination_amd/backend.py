@@ -253,8 +253,8 @@ def evaluate_ht_hamilton_replies_cuda(graph: GraphSnapshot, target, centers,
     offsets = np.empty(len(centers) + 1, dtype=np.uint64)
     total, usage = C.c_uint64(), _lib.HtUsage()
     view = graph.view()
-    # the reply count is known after the device's count pass: size the
-    # buffer from it and copy the replies left on the device
+    # the reply count is known once the pairs are tested: size the buffer
+    # from it and have the replies written there
     _lib.check(_lib.lib().ee_ht_hamilton_replies(
         ctx.handle, C.byref(view), int(target[0]), int(target[1]),
         _lib.ptr(centers) if len(centers) else None, len(centers), _lib.ptr(offsets),

@@ -15,10 +15,10 @@
 // pair (pairs numbered in the reference's first-major order), and a ballot
 // plus a popcount prefix place the surviving pairs in order.
 //
-// Two forms of the output.  Where every row is short (kBitsDegree), one pass
-// writes each pair's verdict as a bit into host memory, and the host writes
-// the replies from the bits into the caller's buffer: a reply is its center
-// and two neighbours, 12 bytes that the host has, against one bit.
+// Two forms of the output.  Where the centers' rows are short (PlanVerdicts),
+// one pass writes each pair's verdict as a bit into host memory, and the host
+// writes the replies from the bits into the caller's buffer: a reply is its
+// center and two neighbours, 12 bytes that the host has, against one bit.
 // Otherwise a count pass, an offset scan and a write pass leave the replies
 // on the device, which then never holds more than the replies themselves.
 #include <algorithm>
@@ -157,11 +157,8 @@ __global__ __launch_bounds__(kHtBlock) void HtHamiltonKernel(
   if (!kWrite && lane == 0) counts[item] = found;
 }
 
-// Rows of up to this many neighbours (2,016 pairs in LDS, then up to 130,816
-// recomputed per pair) take the verdict bits, if all centers' words fit
-// kBitsBytes of host memory.
-constexpr uint32_t kBitsDegree = 512;
-constexpr size_t kBitsBytes = size_t{32} << 20;
+// Words of verdict bits of a row of d neighbours.
+__host__ __device__ inline uint32_t VerdictWords(uint32_t d) { return d < 2 ? 0 : (d * (d - 1) / 2 + 63) / 64; }
 
 // A neighbour of the center under test: what the pair test needs of it.  x
 // and y are the low words on near snapshots (differences stay exact).
@@ -181,31 +178,35 @@ __device__ inline int64_t RowDist(const HtRow<kNear>& a, const HtRow<kNear>& b, 
   }
 }
 
-// Neighbours per center in a wavefront's first phase, and its centers.
+// Neighbours per center in a wavefront's first phase.
 constexpr uint32_t kVerdictGroup = 16;
-constexpr uint32_t kVerdictCenters = 64 / kVerdictGroup;
 
-// Verdict bits of each center's pairs, `stride` words per center (zero past
-// its pairs), and their counts.  A wavefront takes 4 consecutive centers, so
-// its reads of centers and writes of words and counts are whole stretches of
-// host memory.  The centers gather their neighbours on 16 lanes each (rows
-// of up to 16, the usual case; otherwise they take the wavefront one by one),
-// then each center's pairs take the 64 lanes, out of LDS.  Bound by those
-// gathers and the pair arithmetic: 41 us for the 30,000-node graph's 1.56
-// million pairs.  One center per wavefront, reading its id and writing its
-// words over PCIe by itself, took 64 us; 8 and 16 centers 41 and 50 us, and
-// 7 and 19 us more where few centers leave the chip to single wavefronts.
-template <bool kNear>
+// Verdict bits of each center's pairs, in words of their own, and their
+// counts.  With a stride every center has that many words (zero past its
+// pairs); otherwise VerdictWords of its row, and first_words[w] is the first
+// of wavefront w's.  A wavefront takes kCenters consecutive centers, so its
+// reads of centers and writes of words and counts are whole stretches of
+// host memory.  Of 4, the centers gather their neighbours on 16 lanes each
+// (rows of up to 16, the usual case; otherwise they take the wavefront one by
+// one), then each center's pairs take the 64 lanes, out of LDS.  Bound by
+// those gathers and the pair arithmetic: 41 us for the 30,000-node graph's
+// 1.56 million pairs.  One center per wavefront, reading its id and writing
+// its words over PCIe by itself, took 64 us there; 8 and 16 centers 41 and 50
+// us, and 7 and 19 us more where few centers leave the chip to single
+// wavefronts.  Rows beyond the LDS cache recompute both neighbours per pair
+// and end the launch, so wherever there is one a wavefront takes one center.
+template <bool kNear, uint32_t kCenters>
 __global__ __launch_bounds__(kHtBlock) void HtVerdictKernel(
     const longlong2* __restrict__ xy, const int32_t* __restrict__ row_offsets,
     const int32_t* __restrict__ neighbors, int32_t nodes, int type, int32_t tu, int32_t tv,
-    const int32_t* __restrict__ centers, uint32_t center_count, uint32_t stride, uint64_t* __restrict__ bits,
-    uint32_t* __restrict__ counts) {
+    const int32_t* __restrict__ centers, uint32_t center_count, uint32_t stride,
+    const uint32_t* __restrict__ first_words, uint64_t* __restrict__ bits, uint32_t* __restrict__ counts) {
   __shared__ HtRow<kNear> rows[kHtWaves][kHtLdsNeighbors];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t first = (blockIdx.x * kHtWaves + wave) * kVerdictCenters;
+  const uint32_t number = blockIdx.x * kHtWaves + wave;
+  const uint32_t first = number * kCenters;
   if (first >= center_count) return;  // whole wavefronts leave together
-  const uint32_t here = min(kVerdictCenters, center_count - first);
+  const uint32_t here = min(kCenters, center_count - first);
   HtRow<kNear>* const mine = rows[wave];
   const int64_t target_cost = Dist<kNear>(xy, tu, tv, type);
   // lane i < here: center i of the wavefront, its row (empty for an id out of
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(kHtBlock) void HtVerdictKernel(
   uint64_t word = 0;       // lane l: word l of the stretch being filled
   uint32_t at = 0;         // words of the wavefront so far
   uint32_t my_count = 0;   // lane i: surviving pairs of center i
-  uint64_t* const out = bits + static_cast<uint64_t>(first) * stride;
+  uint64_t* const out = bits + (stride != 0 ? static_cast<uint64_t>(first) * stride : first_words[number]);
   const uint32_t q = lane / kVerdictGroup;
   const int32_t q_degree = __shfl(my_degree, static_cast<int>(q));
   const bool together = __ballot(q_degree > static_cast<int32_t>(kVerdictGroup)) == 0;
@@ -262,7 +263,8 @@ __global__ __launch_bounds__(kHtBlock) void HtVerdictKernel(
     }
     const uint32_t pairs = d < 2 ? 0 : d * (d - 1) / 2;
     uint32_t found = 0;
-    for (uint32_t w = 0; w < stride; ++w) {
+    const uint32_t words = stride != 0 ? stride : VerdictWords(d);
+    for (uint32_t w = 0; w < words; ++w) {
       const uint32_t p = w * 64 + lane;
       bool keep = false;
       if (p < pairs) {
@@ -508,39 +510,57 @@ uint64_t HtResidentBytes(const HtCache& c) {
          c.d_counts.bytes() + c.d_offsets.bytes() + c.d_chunk_sums.bytes() + c.d_replies.bytes();
 }
 
-// Replies of centers [b, e) from their verdict bits, in order, to `out`.
-int32_t* WriteReplies(const HtCache& c, const HtCache::Verdicts& v, size_t b, size_t e, int32_t* out) {
+// Replies of centers [b, e), whose verdict bits begin at `bits`, in order, to
+// `out`.
+void WriteReplies(const HtCache& c, const HtCache::Verdicts& v, const uint64_t* bits, size_t b, size_t e,
+                  int32_t* out) {
   for (size_t item = b; item < e; ++item) {
     const int32_t center = v.centers.get()[item];
     const int32_t* row = c.neighbors.data() + c.row_offsets[static_cast<size_t>(center)];
     const uint32_t d = static_cast<uint32_t>(c.row_offsets[static_cast<size_t>(center) + 1] -
                                              c.row_offsets[static_cast<size_t>(center)]);
-    if (d < 2) continue;
-    const uint64_t* bits = v.bits.get() + item * v.stride;
-    const uint32_t pairs = d * (d - 1) / 2;
+    const uint32_t pairs = d < 2 ? 0 : d * (d - 1) / 2;
+    const uint32_t words = VerdictWords(d);
     bool all = true;  // the usual case: every pair survives
-    for (uint32_t w = 0; w * 64 < pairs; ++w) {
+    for (uint32_t w = 0; w < words; ++w) {
       const uint32_t left = pairs - w * 64;
       all = all && bits[w] == (left >= 64 ? ~uint64_t{0} : (uint64_t{1} << left) - 1);
     }
-    uint32_t p = 0;
-    for (uint32_t i = 0; i + 1 < d; ++i) {
-      for (uint32_t j = i + 1; j < d; ++j, ++p) {
-        if (!all && ((bits[p / 64] >> (p % 64)) & 1u) == 0) continue;
-        out[0] = center;
-        out[1] = row[i];
-        out[2] = row[j];
-        out += 3;
+    if (all) {
+      for (uint32_t i = 0; i + 1 < d; ++i) {
+        const int32_t first = row[i];
+        for (uint32_t j = i + 1; j < d; ++j) {
+          out[0] = center;
+          out[1] = first;
+          out[2] = row[j];
+          out += 3;
+        }
+      }
+    } else {
+      uint32_t i = 0, begin = 0, end = d - 1;  // pairs [begin, end) are those of neighbour i
+      for (uint32_t w = 0; w < words; ++w) {
+        for (uint64_t left = bits[w]; left != 0; left &= left - 1) {
+          const uint32_t p = w * 64 + static_cast<uint32_t>(__builtin_ctzll(left));
+          while (p >= end) {
+            ++i;
+            begin = end;
+            end += d - 1 - i;
+          }
+          out[0] = center;
+          out[1] = row[i];
+          out[2] = row[p - begin + i + 1];
+          out += 3;
+        }
       }
     }
+    bits += v.stride != 0 ? v.stride : words;
   }
-  return out;
 }
 
-// Centers per group of the reply counts and of the host's work.
-constexpr size_t kGroupCenters = 256;
-// Host threads: writing 19 MB of replies takes 12 about 0.15 ms.
+// Host threads: writing 19 MB of replies takes 12 about 0.15 ms.  Below
+// kSerialReplies waking them costs more than it saves.
 constexpr unsigned kReplyThreads = 12;
+constexpr uint64_t kSerialReplies = 100000;
 
 // Replies [first, first + count) of the last verdicts.
 void CopyVerdictReplies(const HtCache& c, uint64_t first, uint64_t count, int32_t* out) {
@@ -552,17 +572,18 @@ void CopyVerdictReplies(const HtCache& c, uint64_t first, uint64_t count, int32_
   const size_t g0 = group_of(first), g1 = group_of(first + count - 1) + 1;
   ParallelFor(g1 - g0, [&](size_t i) {
     const size_t g = g0 + i;
-    const size_t b = g * kGroupCenters, e = std::min(v.count, b + kGroupCenters);
+    const size_t b = g * v.group, e = std::min(v.count, b + v.group);
+    const uint64_t* bits = v.bits.get() + (v.stride != 0 ? b * v.stride : v.first_words()[b / v.per_wave]);
     const uint64_t from = v.group_first[g], to = v.group_first[g + 1];
     if (from >= first && to <= first + count) {
-      WriteReplies(c, v, b, e, out + 3 * (from - first));
+      WriteReplies(c, v, bits, b, e, out + 3 * (from - first));
       return;
     }
     std::vector<int32_t> whole(3 * (to - from));  // a group the range cuts
-    WriteReplies(c, v, b, e, whole.data());
+    WriteReplies(c, v, bits, b, e, whole.data());
     const uint64_t lo = std::max(from, first), hi = std::min(to, first + count);
     std::copy(whole.begin() + 3 * (lo - from), whole.begin() + 3 * (hi - from), out + 3 * (lo - first));
-  }, g1 - g0 < 8 ? 1 : kReplyThreads);
+  }, count < kSerialReplies ? 1 : kReplyThreads);
 }
 
 void CheckHamilton(const ee_graph_view& g, int32_t tu, int32_t tv, const int32_t* centers, size_t count) {
@@ -577,34 +598,93 @@ void CheckHamilton(const ee_graph_view& g, int32_t tu, int32_t tv, const int32_t
   if (bad) throw std::invalid_argument("HT Hamilton replies: invalid center");
 }
 
-// Whether the call's verdict bits fit host memory, on the resident snapshot.
-size_t VerdictStride(const HtCache& c) {
-  const size_t d = c.max_degree;
-  return std::max<size_t>(1, (d * (d - std::min<size_t>(d, 1)) / 2 + 63) / 64);
-}
-bool TakesVerdicts(const HtCache& c, size_t count) {
-  return c.max_degree <= kBitsDegree && count <= UINT32_MAX && count * VerdictStride(c) * 8 <= kBitsBytes;
+// How a call's verdict bits lie in host memory, or that it does not take them.
+struct VerdictPlan {
+  bool take = false;
+  uint32_t stride = 0;    // words of every center, or 0: as many as its row needs
+  uint32_t per_wave = 4;  // centers of a wavefront
+  size_t words = 0;
+};
+
+// The rule goes by the rows of the given centers on the resident snapshot, not
+// by its longest row: a hub among short rows costs its own words only.
+//  - kUniformDegree: up to here (4 words) all centers get the longest row's
+//    words and the host need not look at the rows; 32 bytes a center are less
+//    than its replies.
+//  - kMeanWords: the form is faster as far as both were measured, from the
+//    smallest calls (one launch and one wait for four and three): whole calls
+//    on k-NN graphs, 300 to 30,000 centers with 3 to 52 words each, 154-5,260
+//    us by three passes and 73-2,020 by bits; complete graphs of 40 to 90
+//    nodes (12 to 62 words) 91-455 and 60-189.  Beyond, replies are hundreds
+//    of MB, which PCIe carries about as fast as host threads write them.
+//  - kBitsDegree: pair numbers stay exact in the kernel's float root.
+//  - kBitsBytes and kBitsCenters bound what a context keeps page-locked.
+constexpr uint32_t kUniformDegree = 23;
+constexpr size_t kMeanWords = 64;
+constexpr uint32_t kBitsDegree = 512;
+constexpr size_t kBitsBytes = size_t{32} << 20;
+constexpr size_t kBitsCenters = kBitsBytes / sizeof(uint64_t);
+
+VerdictPlan PlanVerdicts(const HtCache& c, const int32_t* centers, size_t count) {
+  VerdictPlan p;
+  if (count == 0 || count > kBitsCenters) return p;
+  uint32_t longest = c.max_degree;
+  if (c.max_degree <= kUniformDegree) {
+    p.stride = std::max<uint32_t>(1, VerdictWords(c.max_degree));
+    p.words = count * p.stride;
+  } else {
+    longest = 0;
+    for (size_t i = 0; i < count; ++i) {
+      const size_t v = static_cast<uint32_t>(centers[i]);
+      if (v >= static_cast<size_t>(c.dimension)) continue;  // refused later
+      const uint32_t d = static_cast<uint32_t>(c.row_offsets[v + 1] - c.row_offsets[v]);
+      longest = std::max(longest, d);
+      if (longest > kBitsDegree) return p;
+      p.words += VerdictWords(d);
+    }
+  }
+  p.per_wave = longest <= kHtLdsNeighbors ? 4 : 1;
+  p.take = p.words <= kMeanWords * count && p.words * sizeof(uint64_t) <= kBitsBytes;
+  return p;
 }
 
 // Starts the verdict pass on the resident snapshot into the buffer that does
 // not hold the last call's; returns whether the buffers had room.
-bool LaunchVerdicts(Context& ctx, int type, int32_t tu, int32_t tv, const int32_t* centers, size_t count) {
+bool LaunchVerdicts(Context& ctx, int type, int32_t tu, int32_t tv, const int32_t* centers, size_t count,
+                    const VerdictPlan& plan) {
   HtCache& c = ctx.ht;
   HtCache::Verdicts& v = c.verdicts[c.current ^ 1];
-  v.stride = VerdictStride(c);
+  v.stride = plan.stride;
+  v.per_wave = plan.per_wave;
   v.count = count;
-  const bool room = v.centers.count() >= 2 * count && v.bits.count() >= count * v.stride;
+  // groups of the host's work: some 512 words, whole wavefronts
+  v.group = std::max<size_t>(4, std::min<size_t>(256, 512 * count / std::max<size_t>(plan.words, 1)) / 4 * 4);
+  const size_t waves = (count + plan.per_wave - 1) / plan.per_wave;
+  const size_t ints = 2 * count + (plan.stride != 0 ? 0 : waves), words = std::max<size_t>(plan.words, 1);
+  const bool room = v.centers.count() >= ints && v.bits.count() >= words;
   for (HtCache::Verdicts& b : c.verdicts) {
     if (&b != &v && c.last_kind == 1 && c.last_bits) continue;  // growing would drop the last call's replies
-    b.centers.Reserve(Grow(b.centers.count(), 2 * count));
-    b.bits.Reserve(Grow(b.bits.count(), count * v.stride));
+    // both, so that the next call of this size finds room as this one's does
+    b.centers.Reserve(std::min(Grow(b.centers.count(), ints), 3 * kBitsCenters));
+    b.bits.Reserve(std::min(Grow(b.bits.count(), words), kBitsBytes / sizeof(uint64_t)));
   }
   std::memcpy(v.centers.get(), centers, count * sizeof(int32_t));
-  const auto kernel = c.near ? HtVerdictKernel<true> : HtVerdictKernel<false>;
-  const size_t per_block = kHtWaves * kVerdictCenters;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((count + per_block - 1) / per_block)), dim3(kHtBlock), 0,
+  if (plan.stride == 0) {
+    uint32_t* const first_words = reinterpret_cast<uint32_t*>(v.centers.get()) + 2 * count;
+    uint32_t run = 0;
+    for (size_t i = 0; i < count; ++i) {
+      if (i % plan.per_wave == 0) first_words[i / plan.per_wave] = run;
+      const size_t node = static_cast<uint32_t>(centers[i]);
+      if (node >= static_cast<size_t>(c.dimension)) continue;
+      run += VerdictWords(static_cast<uint32_t>(c.row_offsets[node + 1] - c.row_offsets[node]));
+    }
+  }
+  const auto kernel = plan.per_wave == 1 ? (c.near ? HtVerdictKernel<true, 1> : HtVerdictKernel<false, 1>)
+                                         : (c.near ? HtVerdictKernel<true, 4> : HtVerdictKernel<false, 4>);
+  const uint32_t* const device = reinterpret_cast<const uint32_t*>(v.centers.device());
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((waves + kHtWaves - 1) / kHtWaves)), dim3(kHtBlock), 0,
                      ctx.stream, c.d_xy.get(), c.d_row_offsets.get(), c.d_neighbors.get(), c.dimension, type, tu, tv,
-                     v.centers.device(), static_cast<uint32_t>(count), static_cast<uint32_t>(v.stride),
+                     v.centers.device(), static_cast<uint32_t>(count), plan.stride, device + 2 * count,
                      v.bits.device(), reinterpret_cast<uint32_t*>(v.centers.device() + count));
   CheckHip(hipGetLastError(), "HtVerdictKernel launch");
   return room;
@@ -614,11 +694,11 @@ bool LaunchVerdicts(Context& ctx, int type, int32_t tu, int32_t tv, const int32_
 uint64_t CountVerdicts(HtCache& c, uint64_t* offsets) {
   HtCache::Verdicts& v = c.verdicts[c.current ^ 1];
   const uint32_t* counts = reinterpret_cast<const uint32_t*>(v.centers.get() + v.count);
-  const size_t groups = (v.count + kGroupCenters - 1) / kGroupCenters;
+  const size_t groups = (v.count + v.group - 1) / v.group;
   v.group_first.assign(groups + 1, 0);
   uint64_t run = 0;
   for (size_t g = 0; g < groups; ++g) {
-    for (size_t i = g * kGroupCenters, e = std::min(v.count, i + kGroupCenters); i < e; ++i) {
+    for (size_t i = g * v.group, e = std::min(v.count, i + v.group); i < e; ++i) {
       run += counts[i];
       offsets[i + 1] = run;
     }
@@ -629,11 +709,11 @@ uint64_t CountVerdicts(HtCache& c, uint64_t* offsets) {
 
 // As HamiltonReplies below, by verdict bits.  started: the pass is under way.
 void VerdictReplies(Context& ctx, const ee_graph_view& g, int32_t tu, int32_t tv, const int32_t* centers,
-                    size_t count, bool started, uint64_t* offsets, ee_ht_neighbor_pair* replies, uint64_t capacity,
+                    size_t count, const VerdictPlan& plan, bool started, uint64_t* offsets, ee_ht_neighbor_pair* replies, uint64_t capacity,
                     uint64_t* total, ee_ht_usage* u) {
   HtCache& c = ctx.ht;
   auto t0 = std::chrono::steady_clock::now();
-  if (!started) u->workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count) ? 1 : 0;
+  if (!started) u->workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count, plan) ? 1 : 0;
   ctx.Sync();
   *total = CountVerdicts(c, offsets);
   u->kernel_ms = MsSince(t0);
@@ -668,13 +748,11 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
   const bool likely = count > 0 && tu >= 0 && tu != tv && tv < g.dimension && ctx.ht.valid &&
                       ctx.ht.dimension == g.dimension && ctx.ht.distance_type == g.distance_type &&
                       ctx.ht.active.size() == static_cast<size_t>(g.edge_count) &&
-                      std::memcmp(ctx.ht.x.data(), g.x, std::min<size_t>(ctx.ht.x.size(), 64) * 8) == 0 &&
-                      TakesVerdicts(ctx.ht, count);
-  bool started = false;
-  if (likely) {
-    u.workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count) ? 1 : 0;
-    started = true;
-  }
+                      std::memcmp(ctx.ht.x.data(), g.x, std::min<size_t>(ctx.ht.x.size(), 64) * 8) == 0;
+  VerdictPlan plan;
+  if (likely) plan = PlanVerdicts(ctx.ht, centers, count);
+  bool started = plan.take;
+  if (started) u.workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count, plan) ? 1 : 0;
   try {
     u.graph_hit = HtGraphMatches(ctx.ht, g) ? 1 : 0;
     if (!u.graph_hit) ValidateHtGraph(g);
@@ -697,9 +775,10 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
     if (usage) *usage = u;
     return;
   }
-  if (started || TakesVerdicts(c, count)) {
+  if (!started) plan = PlanVerdicts(c, centers, count);
+  if (plan.take) {
     u.h2d_ms = MsSince(t0);
-    VerdictReplies(ctx, g, tu, tv, centers, count, started, offsets, replies, capacity, total, &u);
+    VerdictReplies(ctx, g, tu, tv, centers, count, plan, started, offsets, replies, capacity, total, &u);
     if (usage) *usage = u;
     return;
   }

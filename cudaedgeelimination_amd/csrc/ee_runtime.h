@@ -347,13 +347,18 @@ struct HtCache {
   int last_kind = 0;                 // last completed call: 1 Hamilton, 2 end replies
   uint64_t last_total = 0;           // its reply count
   // Hamilton replies as verdict bits: per center `stride` words in host
-  // memory, bit p set where pair p survives.  The call under way uses the
-  // other buffer, so that a refused one leaves the last one's replies.
+  // memory, or with stride 0 as many as its row needs, bit p set where pair p
+  // survives.  The call under way uses the other buffer, so that a refused
+  // one leaves the last one's replies.
   struct Verdicts {
-    Pinned<int32_t> centers;  // the centers, then their reply counts
+    // the centers, then their reply counts, then (stride 0) the first word of
+    // each wavefront's centers
+    Pinned<int32_t> centers;
     Pinned<uint64_t> bits;
-    size_t count = 0, stride = 0;
+    size_t count = 0, stride = 0, per_wave = 4;
+    size_t group = 256;                 // centers of a group of the host's work
     std::vector<uint64_t> group_first;  // replies before each group of centers, and in all
+    const uint32_t* first_words() const { return reinterpret_cast<const uint32_t*>(centers.get()) + 2 * count; }
   };
   Verdicts verdicts[2];
   int current = 0;

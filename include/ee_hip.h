@@ -247,11 +247,17 @@ typedef struct {
  * order.  offsets receives center_count + 1 entries (center i's replies are
  * [offsets[i], offsets[i+1])), replies the first min(*total, capacity)
  * replies (ee_ht_copy_replies copies the rest), *total their count.  What is
- * kept for ee_ht_copy_replies is one bit per neighbour pair where every row
- * is short (at most 512 entries, 32 MiB of bits in all), else, after a count
- * pass, exactly *total replies on the device.  The snapshot must pass the reference's HT graph checks
+ * kept for ee_ht_copy_replies is one bit per neighbour pair where the
+ * centers' rows are short (at most 4,096 pairs a center on average and 512
+ * neighbours each, 32 MiB of bits and 2^22 centers in all), else, after a
+ * count pass, exactly *total replies on the device.  The bits and up to 12
+ * bytes a center lie in page-locked memory, twice (a refused call leaves the
+ * last one's), which grows to at most twice what a call needed and 80 MiB
+ * each.  The snapshot must pass the reference's HT graph checks
  * (ht_replies.cu:521-553): a symmetric CSR of exactly the active edges,
- * rows strictly ascending. */
+ * rows strictly ascending.  usage->h2d_ms covers the checks, beside which the
+ * pass over a resident snapshot already runs, usage->kernel_ms the wait for
+ * the rest of it, and usage->d2h_ms the writing of the replies. */
 ee_status ee_ht_hamilton_replies(ee_ctx* ctx, const ee_graph_view* graph, int32_t target_u,
                                  int32_t target_v, const int32_t* centers, size_t center_count,
                                  uint64_t* offsets, ee_ht_neighbor_pair* replies, uint64_t capacity,

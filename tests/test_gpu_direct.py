@@ -1,10 +1,12 @@
-"""Leaf-cost calls whose kernel reads rows from and writes cells to host
-memory, at the sizes where their tiles and launches end: one row, one row
-either side of a tile, several launches through the ring's slots, and more
-launches than slots; near and wide coordinates (one and two planes of the
-transfer form).  Whole numbers, so every comparison is exact."""
+"""Calls whose kernels read inputs from and write results to host memory, at
+the sizes where their tiles and launches end: one row, one row either side of
+a tile, several launches through the ring's slots, and more launches than
+slots; near and wide coordinates (one and two planes of the transfer form);
+and at every line of a rule that chooses a form.  Whole numbers, so every
+comparison is exact."""
 from __future__ import annotations
 
+import itertools
 import sys
 
 import numpy as np
@@ -201,6 +203,114 @@ def test_hamilton_verdicts(ctx, degree):
     woff, wrep = O.ht_hamilton_replies(O.OGraph.from_snapshot(moved), target, centers,
                                        int((deg * (deg - 1) // 2).sum()))
     assert not usage.graph_hit and np.array_equal(off, woff) and np.array_equal(rep, wrep)
+
+
+def edges_graph(pairs, n, dtype=EUC_2D, box=1_000_000, seed=5):
+    """A snapshot on random points with exactly these edges."""
+    rng = np.random.default_rng(seed)
+    u, v = (np.array(c, np.int32) for c in zip(*sorted(set(map(tuple, map(sorted, pairs))))))
+    return GraphSnapshot.from_edges(rng.integers(0, box, n), rng.integers(0, box, n), dtype, u, v)
+
+
+def hamilton_oracle(g, target, centers):
+    deg = np.diff(g.row_offsets).astype(np.int64)[centers]
+    return O.ht_hamilton_replies(O.OGraph.from_snapshot(g), target, centers, int((deg * (deg - 1) // 2).sum()))
+
+
+@pytest.mark.parametrize("form", ["near", "wide", "ceil"])
+@pytest.mark.parametrize("degree", [0, 1, 15, 16, 17, 22, 23, 24, 63, 64, 65, 91, 92])
+def test_hamilton_rows_either_side(ctx, degree, form):
+    """Complete graphs (rows of one length) around every line of the verdict
+    form: 16 neighbours gathered together, one stride for all up to 23, 64
+    cached in LDS, 64 words a center on average (92 neighbours take three
+    passes); near, 64-bit and CEIL_2D distances; beside them centers without
+    edges, in lists that end inside a wavefront."""
+    say(f"ht rows degree {degree} {form}")
+    n = max(degree + 1, 2)
+    pairs = list(itertools.combinations(range(n), 2)) + [(n, n + 1)]  # the target apart
+    g = edges_graph(pairs if degree else [(n, n + 1)], n + 7, CEIL_2D if form == "ceil" else EUC_2D,
+                    1 << 30 if form == "wide" else 1_000_000, degree + 1)
+    alone = np.arange(n + 2, n + 7, dtype=np.int32)  # no edges
+    for target in ((n, n + 1), (0, 1)) if degree else ((n, n + 1),):
+        rest = np.setdiff1d(np.arange(n + 2, dtype=np.int32), np.array(target, np.int32))
+        lists = [rest, np.concatenate([alone[:2], rest, alone[2:3], rest[:3]]), np.tile(rest, 3)[:-1]]
+        for centers in lists + ([alone] if degree < 24 else []):
+            want = hamilton_oracle(g, target, centers)
+            for _ in range(2):
+                off, rep, _ = backend.evaluate_ht_hamilton_replies_cuda(g, target, centers, ctx)
+                assert np.array_equal(off, want[0]) and np.array_equal(rep, want[1])
+
+
+@pytest.mark.parametrize("hub", [30, 512, 513])
+def test_hamilton_hub_costs_its_own_words(hub):
+    """A hub among short rows: what the context keeps follows the centers'
+    own rows (all 2,044 words of a row of 512 for each of 3,000 centers would
+    be 49 MB, twice), whether the hub is a center, several times, or not."""
+    say(f"ht hub {hub}")
+    n = 3_000
+    g = edges_graph([(i, i + 1) for i in range(1, n - 1)] + [(0, 5 * i + 1) for i in range(hub)], n)
+    own = backend.Context(0)
+    target = (n - 2, n - 1)
+    plain = np.arange(1, n - 2, dtype=np.int32)
+    for centers, hubs in ((plain, 0), (np.concatenate([plain[:1_001], [0], plain[1_001:]]).astype(np.int32), 1),
+                          (np.tile(np.concatenate([[0], plain[:40]]), 31).astype(np.int32), 31)):
+        want = hamilton_oracle(g, target, centers)
+        for _ in range(2):
+            off, rep, usage = backend.evaluate_ht_hamilton_replies_cuda(g, target, centers, own)
+            assert np.array_equal(off, want[0]) and np.array_equal(rep, want[1])
+        # the snapshot; centers, counts, bits and offsets, twice and grown at
+        # most twofold; or the replies, their counts and offsets
+        pairs = hubs * hub * (hub - 1) // 2 + 2 * len(centers)
+        words = pairs // 64 + 2 * len(centers)
+        assert usage.resident_bytes < 200_000 + 4 * (8 * words + 9 * len(centers)) + (24 * pairs if hub > 512 else 0)
+    own.close()
+
+
+@pytest.mark.parametrize("form", ["near", "wide", "ceil"])
+def test_hamilton_three_passes(ctx, form):
+    """The count, scan and write passes over more centers than one scan chunk
+    holds (1,024), repeated ones among them: a hub beyond 512 neighbours sends
+    the call there; 64-bit and CEIL_2D distances, rows beyond the LDS cache."""
+    say(f"ht three passes {form}")
+    n = 700
+    pairs = [(0, i) for i in range(1, 600)] + list(itertools.combinations(range(1, 80), 2))
+    pairs += [(i, i + 1) for i in range(1, n - 1)] + [(i, i + 7) for i in range(80, n - 7, 2)]
+    g = edges_graph(pairs, n, CEIL_2D if form == "ceil" else EUC_2D, 1 << 30 if form == "wide" else 1_000_000)
+    rest = np.arange(1, n, dtype=np.int32)
+    for target, centers in (((n - 2, n - 1), np.concatenate([rest[:-2], [0], np.tile(rest[::-1][2:], 3)])),
+                            ((1, 2), np.concatenate([np.tile(rest[2:], 2), [0, 0], rest[5:40]]))):
+        centers = np.ascontiguousarray(centers, np.int32)
+        want = hamilton_oracle(g, target, centers)
+        for _ in range(2):
+            off, rep, usage = backend.evaluate_ht_hamilton_replies_cuda(g, target, centers, ctx)
+            assert np.array_equal(off, want[0]) and np.array_equal(rep, want[1])
+        assert usage.resident_bytes > 12 * len(rep) and len(centers) > 1_024
+        total = len(rep)
+        part = np.empty((total // 2, 3), np.int32)
+        _lib.check(_lib.lib().ee_ht_copy_replies(ctx.handle, total // 3, total // 2, _lib.ptr(part)))
+        assert np.array_equal(part, rep[total // 3:total // 3 + total // 2])
+
+
+@pytest.mark.parametrize("hub, centers, takes", [(2, 1 << 22, True), (2, (1 << 22) + 1, False),
+                                                 (22, 1 << 20, True), (22, (1 << 20) + 1, False)])
+def test_hamilton_bits_limit(hub, centers, takes):
+    """32 MiB of verdict bits, at one word and at four words a center, and one
+    center more: both forms give the oracle's replies."""
+    say(f"ht bits limit hub {hub} centers {centers}")
+    n = 1_000
+    g = edges_graph([(i, i + 1) for i in range(1, n - 1)] + [(0, 40 * i + 1) for i in range(hub)], n)
+    target, base = (n - 2, n - 1), np.arange(2, n - 3, dtype=np.int32)
+    off, rep = hamilton_oracle(g, target, base)
+    times, left = divmod(centers, len(base))
+    own = backend.Context(0)
+    got_off, got, usage = backend.evaluate_ht_hamilton_replies_cuda(g, target, np.resize(base, centers), own)
+    assert np.array_equal(got, np.concatenate([np.tile(rep, (times, 1)), rep[:off[left]]]))
+    per = np.diff(off)
+    assert np.array_equal(np.diff(got_off), np.resize(per, centers)) and got_off[0] == 0
+    # bits, centers and counts, twice; or centers, counts and offsets (20
+    # bytes a center) and the replies
+    assert (usage.resident_bytes >= 2 * ((32 << 20) + 8 * centers)) == takes
+    own.close()
 
 
 @pytest.mark.parametrize("rows", [1, 255, 257, 43_520, 43_521, 90_001])
