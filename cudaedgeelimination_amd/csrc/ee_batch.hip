@@ -259,6 +259,16 @@ struct Batch {
     return static_cast<double>(ms) / launches;
   }
 
+  // No work: nothing to launch or read until the next set_work.
+  void DropWork() {
+    DropGraph();
+    ClearWritten();
+    segments.clear();
+    task_count = cell_count = tile_count = 0;
+    for (bool& present : k_present) present = false;
+    layout_dirty = true;
+  }
+
   // Forgets which extra pools hold results (new work or output mode).
   void ClearWritten() {
     for (PipeLane& l : lanes) l.written = false;
@@ -620,24 +630,45 @@ ee_status ee_kopt_batch_set_work(ee_kopt_batch* batch, const ee_kopt_segment_des
     const auto room = [&](auto& array, uint64_t count) {
       if (array.count() < std::max<uint64_t>(count, 1)) array.Allocate(std::max<uint64_t>(count, 1), b.ctx->device);
     };
-    room(b.d_next_tasks, rows);
+    try {
+      room(b.d_next_tasks, rows);
+    } catch (const std::runtime_error&) {
+      // no room for both works' rows: the new ones in place of the old, which
+      // a refusal would have kept, so the host checks them first
+      refuse_rows();
+      b.DropWork();
+      b.d_tasks = {};
+      room(b.d_next_tasks, rows);
+    }
     room(b.d_row_segments, checks.size());
     b.d_row_segments.Upload(checks.data(), checks.size(), b.ctx->stream);
     if (!ee::UploadRows(*b.ctx, tasks, rows, b.d_row_segments.get(), checks.size() - 1, b.d_next_tasks.get())) {
       refuse_rows();
       throw std::logic_error("the device refused task rows that the host accepts");
     }
-    b.DropGraph();
-    b.ClearWritten();
+    // the old work ends here: should the pools below find no room, no launch
+    // pairs its tiles with the new rows or with a freed pool
+    b.DropWork();
     std::swap(b.d_tasks, b.d_next_tasks);
-    room(b.d_costs, cells);
+    const auto pool_room = [&](auto& array, uint64_t count) {
+      try {
+        room(array, count);
+      } catch (const std::runtime_error&) {
+        b.d_next_tasks = {};  // the old work's rows
+        room(array, count);
+      }
+    };
+    uint32_t words = 1;  // MaskWords() of the new work
+    for (int i = 0; i < 3; ++i) {
+      if (present[i]) words = std::max(words, (b.plans[i].templates + 31u) / 32u);
+    }
+    pool_room(b.d_costs, cells);
+    if (b.mask_output) pool_room(b.d_masks, rows * words);
     b.segments = std::move(segs);
     b.task_count = rows;
     b.cell_count = cells;
     for (int i = 0; i < 3; ++i) b.k_present[i] = present[i];
-    if (b.mask_output) room(b.d_masks, rows * b.MaskWords());
     b.ctx->Sync();
-    b.layout_dirty = true;
   });
 }
 
@@ -772,12 +803,12 @@ ee_status ee_kopt_batch_set_output(ee_kopt_batch* batch, uint32_t mode) {
     ee::Batch& b = ee::AsBatch(batch);
     if (mode > 1) throw std::invalid_argument("output mode must be 0 (costs) or 1 (improving masks)");
     b.ctx->Activate();
-    b.mask_output = mode == 1;
-    b.ClearWritten();
-    if (b.mask_output) {
+    if (mode == 1) {  // room first: a batch without it keeps its mode
       const uint64_t words = std::max<uint64_t>(b.task_count * b.MaskWords(), 1);
       if (b.d_masks.count() < words) b.d_masks.Allocate(words, b.ctx->device);
     }
+    b.mask_output = mode == 1;
+    b.ClearWritten();
     b.DropGraph();  // the launch arguments change
   });
 }

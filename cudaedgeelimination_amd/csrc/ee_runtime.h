@@ -164,6 +164,7 @@ template <typename T> class DeviceArray {
         status = hipMalloc(&p, bytes);
       }
       if (status != hipSuccess) {
+        static_cast<void>(hipGetLastError());  // a later launch's check is not to find it
         throw std::runtime_error(std::string("hipMalloc(") + std::to_string(bytes) +
                                  " bytes): " + hipGetErrorString(status));
       }

@@ -6,6 +6,7 @@ and at every line of a rule that chooses a form.  Whole numbers, so every
 comparison is exact."""
 from __future__ import annotations
 
+import ctypes as C
 import itertools
 import sys
 
@@ -349,6 +350,42 @@ def test_set_work_rows(ctx, rows):
                 batch.set_work(segments, bad)
         batch.run()
         assert np.array_equal(batch.download_masks()[:, 0], want)
+    batch.close()
+
+
+@pytest.mark.parametrize("output", ["costs", "masks"])
+def test_set_work_without_room(ctx, output):
+    """Rows that fit the device with cells that do not (as many as would fill
+    it whole): the call fails and the batch has no work, neither the old one's
+    tiles with the new rows nor a freed pool; the next work runs."""
+    say(f"set_work without room, {output}")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert _lib.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    count = total.value // (208 * 8) + 1
+    g = graph(23, 400, EUC_2D, 1_000_000)
+    tasks = W.kopt_tasks(3, g, np.full(500, 5, np.uint8))
+    want, _, _ = O.kopt_costs(g.x, g.y, EUC_2D, 5, tasks)
+    batch = KoptBatch(ctx)
+    instance = batch.add_instance(g)
+    batch.set_output(output)
+    batch.set_work([(instance, 5, 500)], tasks)
+    batch.run()
+    rows = np.empty(count, tasks.dtype)
+    rows[:] = tasks[7]
+    with pytest.raises(_lib.EeError, match="hipMalloc"):
+        batch.set_work([(instance, 5, count)], rows)
+    del rows
+    assert batch.run(3) == 0.0
+    if output == "costs":
+        with pytest.raises(_lib.InvalidArgument):
+            batch.download(0, 1)
+    else:
+        with pytest.raises(_lib.InvalidArgument):
+            batch.download_masks(0, 1)
+    batch.set_work([(instance, 5, 500)], tasks)
+    batch.set_output("costs")
+    batch.run()
+    assert np.array_equal(batch.segment_costs(0), want)
     batch.close()
 
 
