@@ -9,11 +9,11 @@
 #include <cstdint>
 #include <cstring>
 #include <functional>
-#include <mutex>
 #include <string>
 #include <vector>
 
 #include "ee_internal.h"
+#include "ee_pool.h"
 
 namespace ee {
 
@@ -34,34 +34,12 @@ KoptInstance MakeKoptInstance(uint64_t coord_base, const int64_t* x, const int64
                               uint8_t distance_type);
 int CountDevices();
 
-// Freed device and page-locked memory of a context's sessions and fleets,
-// kept for the next: bounded, released with the context, one lock around it.
-// A block comes back only after the streams that used it were synchronised.
-// Allocating and freeing it anew took 110 us of a session's 270 us to create
-// and 95 us to close (15,836 edge slots), and 1.1 ms for 64 graphs.
-class MemoryPool {
- public:
-  static constexpr size_t kMaxBlocks = 64, kMaxDevice = size_t{64} << 20, kMaxHost = size_t{8} << 20;
-  MemoryPool() = default;
-  ~MemoryPool() { Release(); }
-  MemoryPool(const MemoryPool&) = delete;
-  MemoryPool& operator=(const MemoryPool&) = delete;
-  // A kept block of at least `bytes` (its size in *got), or null.
-  void* Take(bool host, size_t bytes, size_t* got);
-  // Whether the pool keeps the block; the caller frees it otherwise.
-  bool Give(bool host, void* ptr, size_t bytes);
-  void Release();  // frees what is kept
-
- private:
-  struct Block {
-    void* ptr;
-    size_t bytes;
-    bool host;
-  };
-  std::mutex mu_;
-  std::vector<Block> blocks_;
-  size_t held_[2] = {0, 0};
-};
+// `bytes` of device memory on the current device or of page-locked host
+// memory.  Where there is none, the memory that contexts keep for their next
+// sessions and fleets is freed first.
+void* NewDeviceMemory(size_t bytes);
+void* NewHostMemory(size_t bytes);
+void FreeMemory(bool host, void* ptr);
 
 // Page-locked host staging of at least `count` elements (hipHostMalloc);
 // growing discards the contents.  The pages are written once when allocated:
@@ -91,7 +69,7 @@ template <typename T> class Pinned {
     size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
     void* p = pool != nullptr ? pool->Take(true, bytes, &bytes) : nullptr;
     if (p == nullptr) {
-      CheckHip(hipHostMalloc(&p, bytes, hipHostMallocDefault), "hipHostMalloc");
+      p = NewHostMemory(bytes);
       std::memset(p, 0, bytes);
     }
     ptr_ = static_cast<T*>(p);
@@ -157,18 +135,7 @@ template <typename T> class DeviceArray {
     CheckHip(hipSetDevice(device), "hipSetDevice");
     size_t bytes = count * sizeof(T);
     void* p = pool != nullptr ? pool->Take(false, bytes, &bytes) : nullptr;
-    if (p == nullptr) {
-      hipError_t status = hipMalloc(&p, bytes);
-      if (status == hipErrorOutOfMemory && pool != nullptr) {
-        pool->Release();
-        status = hipMalloc(&p, bytes);
-      }
-      if (status != hipSuccess) {
-        static_cast<void>(hipGetLastError());  // a later launch's check is not to find it
-        throw std::runtime_error(std::string("hipMalloc(") + std::to_string(bytes) +
-                                 " bytes): " + hipGetErrorString(status));
-      }
-    }
+    if (p == nullptr) p = NewDeviceMemory(bytes);
     ptr_ = static_cast<T*>(p);
     count_ = count;
     held_ = bytes;
@@ -367,7 +334,7 @@ struct HtCache {
 };
 
 struct Context {
-  MemoryPool pool;  // released last
+  MemoryPool pool{FreeMemory};  // released last
   explicit Context(int requested_device);
   ~Context();
   Context(const Context&) = delete;

@@ -36,6 +36,34 @@ void CheckHip(hipError_t status, const char* what) {
   }
 }
 
+namespace {
+
+// `allocate` until it succeeds or has failed without the contexts' kept memory.
+template <typename F> void* NewMemory(size_t bytes, const char* what, F&& allocate) {
+  void* p = nullptr;
+  hipError_t status = allocate(&p);
+  if (status == hipErrorOutOfMemory) {
+    MemoryPool::ReleaseAll();
+    static_cast<void>(hipGetLastError());  // a later launch's check is not to find the failure
+    status = allocate(&p);
+  }
+  if (status == hipSuccess) return p;
+  static_cast<void>(hipGetLastError());
+  throw std::runtime_error(std::string(what) + "(" + std::to_string(bytes) + " bytes): " + hipGetErrorString(status));
+}
+
+}  // namespace
+
+void* NewDeviceMemory(size_t bytes) {
+  return NewMemory(bytes, "hipMalloc", [&](void** p) { return hipMalloc(p, bytes); });
+}
+
+void* NewHostMemory(size_t bytes) {
+  return NewMemory(bytes, "hipHostMalloc", [&](void** p) { return hipHostMalloc(p, bytes, hipHostMallocDefault); });
+}
+
+void FreeMemory(bool host, void* ptr) { static_cast<void>(host ? hipHostFree(ptr) : hipFree(ptr)); }
+
 KoptInstance MakeKoptInstance(uint64_t coord_base, const int64_t* x, const int64_t* y, int32_t n,
                               uint8_t distance_type) {
   KoptInstance inst{};

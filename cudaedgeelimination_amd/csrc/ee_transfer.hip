@@ -435,36 +435,4 @@ bool UploadItems(Context& ctx, const std::vector<UploadItem>& items, const std::
   return !refused;
 }
 
-void* MemoryPool::Take(bool host, size_t bytes, size_t* got) {
-  std::lock_guard<std::mutex> lk(mu_);
-  // the smallest block that fits, at most twice the size asked for
-  size_t best = blocks_.size();
-  for (size_t i = 0; i < blocks_.size(); ++i) {
-    const Block& b = blocks_[i];
-    if (b.host != host || b.bytes < bytes || b.bytes / 2 > std::max<size_t>(bytes, size_t{64} << 10)) continue;
-    if (best == blocks_.size() || b.bytes < blocks_[best].bytes) best = i;
-  }
-  if (best == blocks_.size()) return nullptr;
-  const Block b = blocks_[best];
-  blocks_.erase(blocks_.begin() + static_cast<std::ptrdiff_t>(best));
-  held_[host] -= b.bytes;
-  *got = b.bytes;
-  return b.ptr;
-}
-
-bool MemoryPool::Give(bool host, void* ptr, size_t bytes) {
-  std::lock_guard<std::mutex> lk(mu_);
-  if (blocks_.size() >= kMaxBlocks || held_[host] + bytes > (host ? kMaxHost : kMaxDevice)) return false;
-  blocks_.push_back({ptr, bytes, host});
-  held_[host] += bytes;
-  return true;
-}
-
-void MemoryPool::Release() {
-  std::lock_guard<std::mutex> lk(mu_);
-  for (const Block& b : blocks_) static_cast<void>(b.host ? hipHostFree(b.ptr) : hipFree(b.ptr));
-  blocks_.clear();
-  held_[0] = held_[1] = 0;
-}
-
 }  // namespace ee

@@ -1,5 +1,5 @@
 // Test harness, not part of the product: the backend's host-only units
-// (ee_host.cpp, ee_gen.cpp, ee_jvhost.cpp, ee_certify.cpp) and the oracle,
+// (ee_host.cpp, ee_gen.cpp, ee_jvhost.cpp, ee_certify.cpp, ee_pool.cpp) and the oracle,
 // built with AddressSanitizer and UndefinedBehaviorSanitizer by plain g++
 // (oracle/Makefile, target sanitize; run by tests/test_host.py), as the
 // reference builds its host code with sanitizers (CMakeLists.txt:100-106).
@@ -18,11 +18,16 @@
 //    use) against the oracle's restoring square root;
 //  - the certification pool: every iteration exactly once and the first
 //    exception rethrown after all of them, for pools of 1 to 16 threads,
-//    two of them driven at once.
+//    two of them driven at once;
+//  - the pool of freed blocks: its bounds, that blocks of sizes no longer
+//    asked for make room, and that one allocation's need empties every pool.
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <iostream>
+#include <map>
+#include <mutex>
 #include <random>
 #include <sstream>
 #include <stdexcept>
@@ -36,6 +41,7 @@
 #include "ee_hip.h"
 #include "ee_jvhost.h"
 #include "ee_oracle.h"
+#include "ee_pool.h"
 
 namespace {
 
@@ -283,6 +289,96 @@ void PoolChecks() {
   Expect(bad.load() == 0, "certification pool runs every iteration once and rethrows");
 }
 
+
+// Blocks handed out by malloc and not yet freed, for CheckMemoryPool.
+std::mutex g_blocks_mu;
+std::map<void*, size_t> g_blocks;
+
+void* NewBlock(size_t bytes) {
+  void* p = std::malloc(1);
+  std::lock_guard<std::mutex> lk(g_blocks_mu);
+  g_blocks[p] = bytes;
+  return p;
+}
+
+void FreeBlock(bool, void* p) {
+  std::lock_guard<std::mutex> lk(g_blocks_mu);
+  Expect(g_blocks.erase(p) == 1, "a block is freed once");
+  std::free(p);
+}
+
+size_t Held() {
+  std::lock_guard<std::mutex> lk(g_blocks_mu);
+  size_t bytes = 0;
+  for (const auto& b : g_blocks) bytes += b.second;
+  return bytes;
+}
+
+void CheckMemoryPool() {
+  using Pool = ee::MemoryPool;
+  constexpr size_t kMiB = size_t{1} << 20;
+  const auto give = [](Pool& pool, bool host, size_t bytes) {
+    void* p = NewBlock(bytes);
+    if (!pool.Give(host, p, bytes)) FreeBlock(host, p);
+  };
+  const auto take = [](Pool& pool, bool host, size_t bytes) {
+    size_t got = 0;
+    void* p = pool.Take(host, bytes, &got);
+    Expect(p == nullptr || got >= bytes, "a block holds what was asked for");
+    if (p != nullptr) FreeBlock(host, p);
+    return p != nullptr ? got : 0;
+  };
+  Pool pool(FreeBlock);
+  Expect(take(pool, false, 1) == 0, "an empty pool");
+  // the smallest that fits, of the right kind, at most twice the size or 128 KiB
+  for (size_t mib : {6, 3, 4, 1}) give(pool, false, mib * kMiB);
+  give(pool, true, 2 * kMiB);
+  Expect(take(pool, true, 3 * kMiB) == 0 && take(pool, false, 2 * kMiB) == 3 * kMiB, "the smallest that fits");
+  Expect(take(pool, false, 2 * kMiB) == 4 * kMiB && take(pool, false, 2 * kMiB) == 0, "at most twice the size");
+  give(pool, false, 128 << 10);
+  Expect(take(pool, false, 100) == 128 << 10 && take(pool, false, 100) == 0, "small sizes take up to 128 KiB");
+  pool.Release();
+  Expect(Held() == 0, "a released pool holds nothing");
+  // sessions of many sizes, one after the other: each closes with 26 blocks,
+  // and the next of the same size finds them, whatever came before
+  for (size_t size = 1; size <= 40; ++size) {
+    const size_t bytes = (size << 12) * (size % 7 + 1) + (200 << 10);
+    for (int session = 0; session < 2; ++session) {
+      size_t found = 0;
+      for (int b = 0; b < 26; ++b) found += take(pool, b % 13 == 0, bytes) != 0;
+      Expect(session == 0 || found == 26, "the next session of a size finds its blocks");
+      for (int b = 0; b < 26; ++b) give(pool, b % 13 == 0, bytes);
+    }
+    Expect(Held() <= Pool::kMaxDevice + Pool::kMaxHost, "the pool's bytes are bounded");
+    Expect(g_blocks.size() <= Pool::kMaxBlocks, "the pool's blocks are bounded");
+  }
+  // one block of the whole bound replaces all others of its kind; one beyond it is not kept
+  give(pool, false, Pool::kMaxDevice);
+  give(pool, true, Pool::kMaxHost);
+  Expect(Held() == Pool::kMaxDevice + Pool::kMaxHost, "a block as large as the bound");
+  give(pool, false, Pool::kMaxDevice + 1);
+  Expect(Held() == Pool::kMaxDevice + Pool::kMaxHost && take(pool, false, Pool::kMaxDevice) != 0, "one beyond it");
+  // several pools used on their own threads while another empties them all
+  {
+    Pool second(FreeBlock);
+    const auto work = [&](Pool& mine) {
+      for (int i = 0; i < 2000; ++i) {
+        if (take(mine, i % 2 == 0, 4096) == 0) give(mine, i % 2 == 0, 4096 + 512 * static_cast<size_t>(i % 9));
+      }
+    };
+    std::thread a([&] { work(pool); }), b([&] { work(second); });
+    for (int i = 0; i < 200; ++i) Pool::ReleaseAll();
+    a.join();
+    b.join();
+    give(second, false, kMiB);
+    give(pool, false, kMiB);
+    Pool::ReleaseAll();
+    Expect(Held() == 0, "every pool is emptied");
+    give(second, false, kMiB);
+  }
+  Expect(Held() == 0, "a pool frees its blocks at its end");
+}
+
 }  // namespace
 
 int main() {
@@ -317,6 +413,7 @@ int main() {
     CheckSnapshot(g, "lattice");
     JvRun(g, "lattice");
   }
+  CheckMemoryPool();
   std::cout << (g_failures == 0 ? "sanitized host checks passed" : "sanitized host checks failed") << '\n';
   return g_failures == 0 ? 0 : 1;
 }
