@@ -56,37 +56,6 @@ constexpr unsigned kPublishCopyThreads = 8;
 
 double Ms(Clock::time_point a, Clock::time_point b) { return std::chrono::duration<double, std::milli>(b - a).count(); }
 
-// Coherent, device-mapped host memory: the device reads and writes it over
-// the bus, and the host sees the device's stores without a copy.
-template <typename T> class CoherentHost {
- public:
-  CoherentHost() = default;
-  ~CoherentHost() {
-    if (host_ != nullptr) static_cast<void>(hipHostFree(host_));
-  }
-  CoherentHost(const CoherentHost&) = delete;
-  CoherentHost& operator=(const CoherentHost&) = delete;
-  void Allocate(size_t count) {
-    void* p = nullptr;
-    CheckHip(hipHostMalloc(&p, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent),
-             "hipHostMalloc (coherent)");
-    host_ = static_cast<T*>(p);
-    count_ = count;
-    std::memset(p, 0, std::max<size_t>(count, 1) * sizeof(T));
-    void* d = nullptr;
-    CheckHip(hipHostGetDevicePointer(&d, p, 0), "hipHostGetDevicePointer");
-    device_ = static_cast<T*>(d);
-  }
-  T* host() { return host_; }
-  T* device() { return device_; }
-  size_t count() const { return count_; }
-
- private:
-  T* host_ = nullptr;
-  T* device_ = nullptr;
-  size_t count_ = 0;
-};
-
 // First-fit allocation in arrival order over a circular range; blocks may be
 // freed in any order and their space returns once every older block is free.
 class RingArena {

@@ -38,7 +38,7 @@ int CountDevices();
 // memory.  Where there is none, the memory that contexts keep for their next
 // sessions and fleets is freed first.
 void* NewDeviceMemory(size_t bytes);
-void* NewHostMemory(size_t bytes);
+void* NewHostMemory(size_t bytes, unsigned flags = hipHostMallocDefault);
 void FreeMemory(bool host, void* ptr);
 
 // Page-locked host staging of at least `count` elements (hipHostMalloc);
@@ -108,6 +108,37 @@ template <typename T> class Pinned {
   T* ptr_ = nullptr;
   size_t count_ = 0, bytes_ = 0;
   MemoryPool* pool_ = nullptr;
+};
+
+// Coherent, device-mapped host memory, cleared: kernels read and write it over
+// the bus, and the host sees their stores while they run, as they see its.
+// What one side polls while the other writes lies here.
+template <typename T> class CoherentHost {
+ public:
+  CoherentHost() = default;
+  ~CoherentHost() {
+    if (host_ != nullptr) static_cast<void>(hipHostFree(host_));
+  }
+  CoherentHost(const CoherentHost&) = delete;
+  CoherentHost& operator=(const CoherentHost&) = delete;
+  void Allocate(size_t count) {
+    const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+    host_ = static_cast<T*>(NewHostMemory(bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    count_ = count;
+    std::memset(static_cast<void*>(host_), 0, bytes);
+    void* d = nullptr;
+    CheckHip(hipHostGetDevicePointer(&d, host_, 0), "hipHostGetDevicePointer");
+    device_ = static_cast<T*>(d);
+  }
+  T* host() { return host_; }
+  const T* host() const { return host_; }
+  T* device() { return device_; }
+  size_t count() const { return count_; }
+
+ private:
+  T* host_ = nullptr;
+  T* device_ = nullptr;
+  size_t count_ = 0;
 };
 
 // Owning device allocation of `count` elements of T on one device.
@@ -240,8 +271,10 @@ struct KoptCache {
 // another.  One per context, used by its thread between synchronisations.
 //
 // A kernel marks each tile's output with the launch's mark, a number no
-// earlier launch used, once the output is in host memory.  The marks have an
-// area of their own, so that a word there is never anything but a mark.
+// earlier launch used, once the output is in host memory; the host polls the
+// marks and takes the output while the kernel runs, so both lie in coherent
+// memory.  The marks have an area of their own, so that a word there is never
+// anything but a mark.
 class DirectIo {
  public:
   static constexpr size_t kSlots = 2;
@@ -253,9 +286,9 @@ class DirectIo {
   // on large results (batch cells 400 -> 520 us).
   static constexpr size_t kBytes = size_t{4} << 20, kSlotBytes = kBytes / kSlots;
   void Create();
-  char* host() { return mem_.get(); }
-  char* device() { return device_; }
-  uint64_t* device_marks(size_t slot) { return device_marks_ + slot * kSlotTiles; }
+  char* host() { return mem_.host(); }
+  char* device() { return mem_.device(); }
+  uint64_t* device_marks(size_t slot) { return marks_.device() + slot * kSlotTiles; }
   uint64_t bytes() const { return mem_.count() + marks_.count() * sizeof(uint64_t); }
   uint64_t NextMark() { return ++mark_; }
   // Returns once tile `tile` of the slot's launch, on `stream`, carries
@@ -271,10 +304,8 @@ class DirectIo {
                  const std::function<void(size_t, size_t)>& take) const;
 
  private:
-  Pinned<char> mem_;
-  Pinned<uint64_t> marks_;
-  char* device_ = nullptr;
-  uint64_t* device_marks_ = nullptr;
+  CoherentHost<char> mem_;
+  CoherentHost<uint64_t> marks_;
   uint64_t mark_ = 0;
 };
 

@@ -58,8 +58,8 @@ void* NewDeviceMemory(size_t bytes) {
   return NewMemory(bytes, "hipMalloc", [&](void** p) { return hipMalloc(p, bytes); });
 }
 
-void* NewHostMemory(size_t bytes) {
-  return NewMemory(bytes, "hipHostMalloc", [&](void** p) { return hipHostMalloc(p, bytes, hipHostMallocDefault); });
+void* NewHostMemory(size_t bytes, unsigned flags) {
+  return NewMemory(bytes, "hipHostMalloc", [&](void** p) { return hipHostMalloc(p, bytes, flags); });
 }
 
 void FreeMemory(bool host, void* ptr) { static_cast<void>(host ? hipHostFree(ptr) : hipFree(ptr)); }

@@ -222,14 +222,12 @@ static_assert(kSlotBytes / 4 / kPackTile <= DirectIo::kSlotTiles, "a slot's tile
 }  // namespace
 
 void DirectIo::Create() {
-  marks_.Reserve(kSlots * kSlotTiles);
-  device_marks_ = marks_.device();
-  mem_.Reserve(kBytes);
-  device_ = mem_.device();
+  marks_.Allocate(kSlots * kSlotTiles);
+  mem_.Allocate(kBytes);
 }
 
 void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t stream) const {
-  const uint64_t* at = marks_.get() + slot * kSlotTiles + tile;
+  const uint64_t* at = marks_.host() + slot * kSlotTiles + tile;
   const auto seen = [&] { return __atomic_load_n(at, __ATOMIC_ACQUIRE) == mark; };
   for (uint64_t polls = 1; !seen(); ++polls) {
     // a kernel that ended, or failed, without the mark: look now and then
