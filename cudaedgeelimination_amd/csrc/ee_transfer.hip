@@ -230,8 +230,9 @@ void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t str
   const uint64_t* at = marks_.host() + slot * kSlotTiles + tile;
   const auto seen = [&] { return __atomic_load_n(at, __ATOMIC_ACQUIRE) == mark; };
   for (uint64_t polls = 1; !seen(); ++polls) {
+    __builtin_ia32_pause();
     // a kernel that ended, or failed, without the mark: look now and then
-    if (polls % (uint64_t{1} << 20) != 0) continue;
+    if (polls % (uint64_t{1} << 16) != 0) continue;
     const hipError_t status = hipStreamQuery(stream);
     if (status == hipErrorNotReady || seen()) continue;
     CheckHip(status, "kernel writing to host memory");
@@ -241,6 +242,9 @@ void DirectIo::WaitTile(size_t slot, size_t tile, uint64_t mark, hipStream_t str
 
 void DirectIo::TakeTiles(size_t slot, uint64_t mark, hipStream_t stream, size_t tiles, size_t group,
                          unsigned threads, const std::function<void(size_t, size_t)>& take) const {
+  // the work queued before the launch is waited for here, not on the process's
+  // host threads, which run one caller's job at a time
+  if (tiles > 0) WaitTile(slot, 0, mark, stream);
   ParallelFor((tiles + group - 1) / group, [&](size_t g) {
     const size_t first = g * group, last = std::min(tiles, first + group);
     for (size_t t = first; t < last; ++t) WaitTile(slot, t, mark, stream);

@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes as C
 import itertools
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -516,3 +517,53 @@ def test_server_in_place(ctx, rows, slots, batching):
         for (got, _), exact in zip(server.wait_many(server.submit_many(requests), 60_000), want):
             assert np.array_equal(got, exact)
     server.close()
+
+
+def test_two_contexts_on_two_threads():
+    """Contexts used side by side, each by its own thread: one reads large
+    results (the process's host threads take its tiles), the other runs JV
+    calls, sessions and small leaf blocks, whose host phases want those threads."""
+    say("two contexts on two threads")
+    g = W.knn_graph(*np.random.default_rng(31).integers(0, 1_000_000, (2, 3_000)), EUC_2D, 8)
+    rows = W.kopt_tasks(5, g, np.full(6_000, 5, np.uint8))
+    table = backend.build_kopt_reconnect_table(5)
+    cells, _, _ = O.kopt_costs(g.x, g.y, EUC_2D, 5, rows)
+    witnesses = O.OGraph.from_snapshot(g).witnesses()
+    own = backend.Context(0)
+    s = JvSession(own, g)
+    proof = O.canonical_proof(s.run(100).proof)
+    s.close()
+    own.close()
+    wrong, done = [], threading.Event()
+
+    def large():
+        try:
+            mine = backend.Context(0)
+            batch = KoptBatch(mine)
+            batch.set_work([(batch.add_instance(g), 5, len(rows))], rows)
+            while not done.is_set():
+                batch.run()
+                if not np.array_equal(batch.segment_costs(0), cells):
+                    wrong.append("batch")
+            batch.close()
+            mine.close()
+        except Exception as error:  # noqa: BLE001 - reported by the test
+            wrong.append(error)
+
+    thread = threading.Thread(target=large)
+    thread.start()
+    mine = backend.Context(0)
+    for i in range(15):
+        got, _, _ = backend.evaluate_kopt_template_costs_cuda(g, table, rows[:100 + 50 * i], mine)
+        if not np.array_equal(got, cells[:len(got)]):
+            wrong.append("leaf")
+        if not np.array_equal(backend.find_jv_witnesses(g, mine)[0], witnesses):
+            wrong.append("jv")
+        s = JvSession(mine, g)
+        if O.canonical_proof(s.run(100).proof) != proof:
+            wrong.append("session")
+        s.close()
+    done.set()
+    thread.join()
+    mine.close()
+    assert not wrong
