@@ -394,8 +394,9 @@ struct Context {
 // Copies `bytes` (whole 4-byte words) of device memory to caller memory and
 // waits, after the work queued before it on the context's stream: a kernel
 // writes the words into the context's ring and host threads copy them out
-// as they arrive.
-void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes);
+// as they arrive.  `begun` runs when the first have, with all of that work done.
+void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes,
+                      const std::function<void()>& begun = [] {});
 
 // The rows from row_begin to the next entry's are checked as k-opt task rows
 // of this k on n nodes.

@@ -12,8 +12,10 @@
 //         24m + 20n + 4 + 8A on an exact first fit.
 //   k-opt (src/cuda/kopt_cost.cu:205-295): coordinates keyed by exact
 //         compare of (dimension, distance type, x, y); templates keyed per k
-//         by (generator hash, content); task and cost buffers grow the same
-//         way.
+//         by (generator hash, content).  Rows and cells pass through the
+//         context's ring, so the workspace flag is that of the reference's
+//         buffers, followed by their sizes alone, and the resident bytes are
+//         the device copies and the ring.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -354,9 +356,10 @@ void FindJvCandidates(Context& ctx, const ee_graph_view& g, int32_t* witnesses, 
     u.static_hit = static_hit ? 1 : 0;
     u.workspace_hit = workspace_hit ? 1 : 0;
     u.resident_bytes = JvResidentBytes(c);
-    u.kernel_ms = MsSince(t0);
-    t0 = std::chrono::steady_clock::now();
-    DownloadToCaller(ctx, witnesses, c.d_witnesses.get(), static_cast<size_t>(m) * sizeof(int32_t));
+    DownloadToCaller(ctx, witnesses, c.d_witnesses.get(), static_cast<size_t>(m) * sizeof(int32_t), [&] {
+      u.kernel_ms = MsSince(t0);
+      t0 = std::chrono::steady_clock::now();
+    });
     u.d2h_ms = MsSince(t0);
     break;
   }

@@ -300,7 +300,7 @@ void DownloadCells(Context& ctx, const int64_t* d_cells, size_t count, bool wide
   });
 }
 
-void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes) {
+void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes, const std::function<void()>& begun) {
   if (bytes == 0) return;
   if (dst == nullptr || src == nullptr) throw std::logic_error("download with a NULL buffer");
   if (bytes % 4 != 0) throw std::logic_error("download of partial words");
@@ -320,6 +320,10 @@ void DownloadToCaller(Context& ctx, void* dst, const void* src, size_t bytes) {
     CheckHip(hipGetLastError(), "CopyWords launch");
   }, [&](size_t i, size_t slot) {
     const size_t n = words_of(i);
+    if (i == 0) {
+      io.WaitTile(slot, 0, marks[slot], ctx.stream);
+      begun();
+    }
     const uint32_t* from = reinterpret_cast<const uint32_t*>(io.host()) + slot * slot_words;
     uint32_t* to = static_cast<uint32_t*>(dst) + i * kSlotWords;
     // 64 KiB at a time, on host threads from 512 KiB up

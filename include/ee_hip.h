@@ -124,9 +124,10 @@ typedef struct {
   int32_t static_hit;
   int32_t workspace_hit;
   uint64_t resident_bytes; /* 24m + 20n + 4 + 8A on an exact first fit */
-  double h2d_ms;
-  double kernel_ms;
-  double d2h_ms;
+  double h2d_ms;           /* the dynamic arrays' way in */
+  double kernel_ms;        /* from there to the first witnesses, with the
+                            * comparison of the static part beside the kernel */
+  double d2h_ms;           /* the rest of the witnesses */
 } ee_jv_usage;
 
 /* Replaces cudaee::FindJvCandidatesCuda (src/cuda/jv_cuda.cu:488-566).
@@ -161,12 +162,15 @@ typedef struct {
 typedef struct {
   int32_t snapshot_hit;
   int32_t template_hit;
+  /* Whether an evaluation this large came before, with the reference's growth
+   * rule for its task and cost buffers.  Rows and cells pass through a ring of
+   * fixed size here, so no buffer stands behind it. */
   int32_t workspace_hit;
   int32_t reserved;
-  uint64_t resident_bytes;
-  double h2d_ms;
-  double kernel_ms;
-  double d2h_ms;
+  uint64_t resident_bytes; /* device copies, and the ring in page-locked host memory */
+  double h2d_ms;           /* the rows' staging and the first launches */
+  double kernel_ms;        /* from there to the first tile of the output */
+  double d2h_ms;           /* the rest of the output */
 } ee_kopt_usage;
 
 /* Replaces cudaee::BuildKOptReconnectTable (src/cpu/kopt_search.cpp:1143-1193):
@@ -629,19 +633,23 @@ ee_status ee_jv_fleet_active(const ee_jv_fleet* fleet, uint32_t index, uint8_t* 
 /* ------------------------------------------------------- serving k-opt */
 /* No reference counterpart.  A request loop over device-resident graph
  * snapshots: callers submit leaf-cost queries (one graph, one k, task rows)
- * and JV rechecks (ee_server_submit_jv) from any thread; a worker thread packs whatever has arrived into the next
- * batched launch (continuous batching) as long as the batch stays within the
- * cell and HBM budgets, runs up to `pipeline_depth` batches concurrently on
- * separate streams (a batch's rows, kernels and results overlap with the
- * next; kernels read and write page-locked memory in place), writes each request's cells to the caller's buffer and marks it
- * complete.  Cells are bit-identical to ee_kopt_eval_costs with the canonical
+ * and JV rechecks (ee_server_submit_jv) from any thread; a worker thread packs
+ * whatever has arrived into the next batched launch (continuous batching) as
+ * long as the batch stays within the cell and byte budgets, runs up to
+ * `pipeline_depth` batches concurrently on separate streams (a batch's rows,
+ * kernels and results overlap with the next; kernels read and write
+ * page-locked memory in place), writes each request's cells to the caller's
+ * buffer and marks it complete.  Cells are bit-identical to ee_kopt_eval_costs with the canonical
  * templates.  With max_batch_requests = 1 and pipeline_depth = 1 the server
  * is the plain per-query path: one launch per request, waited for, in
  * arrival order. */
 typedef struct ee_server ee_server;
 
 typedef struct {
-  uint64_t hbm_budget_bytes;   /* device bytes for all in-flight batch buffers */
+  /* Bytes of all batches in flight: 8 a cell and 48 a row, 8 an edge slot.
+   * Their buffers are page-locked host memory, which kernels read and write in
+   * place (5 bytes a cell); device memory holds the snapshots alone. */
+  uint64_t hbm_budget_bytes;
   uint64_t max_batch_cells;    /* cells per launch (a larger request runs alone) */
   uint32_t max_batch_requests; /* requests per launch */
   uint32_t pipeline_depth;     /* batches in flight: 1 or 2 */
@@ -663,7 +671,8 @@ typedef struct {
   uint64_t cells;       /* leaf-cost cells served */
   uint64_t jv_edges;    /* edge slots rechecked */
   uint64_t peak_inflight_bytes;
-  double device_ms;     /* sum of batch kernel times (HIP events) */
+  double device_ms;     /* sum of batch kernel times (HIP events), which hold
+                         * the results' way to host memory */
 } ee_server_stats;
 
 ee_status ee_server_create(ee_ctx* ctx, const ee_server_config* config, ee_server** out);

@@ -422,6 +422,18 @@ def test_jv_call_inputs(ctx, n, neighbors):
     assert not usage.static_hit and usage.workspace_hit
 
 
+def test_jv_phase_times(ctx):
+    """A call's kernel time holds its kernel: on a complete graph (28,680
+    slots that each score 478 neighbours) it is most of the call, and the 0.1
+    MB of witnesses after it the smaller part."""
+    say("jv phase times")
+    g = edges_graph(itertools.combinations(range(240), 2), 240)
+    for _ in range(3):
+        got, usage = backend.find_jv_witnesses(g, ctx)
+    assert np.array_equal(got, O.OGraph.from_snapshot(g).witnesses())
+    assert usage.static_hit and usage.kernel_ms > 2 * usage.d2h_ms > 0
+
+
 @pytest.mark.parametrize("n, neighbors", [(3, 2), (682, 3), (1_023, 3), (1_024, 4), (1_025, 4), (2_049, 5),
                                           (8_193, 6), (50_001, 8)])
 def test_session_snapshot_upload(ctx, n, neighbors):
