@@ -1,7 +1,9 @@
 // Deletion-set producer on the device: the task rows the reference's k-opt
 // cost cursor builds on the host, one per combination of k selectable tour
-// positions, are built by a kernel from the rank of each combination, and
-// fed straight into the plain k-opt evaluation.  No task row crosses PCIe.
+// positions, are built on the device from the rank of each combination: by the
+// cost kernel itself where they are evaluated (ee_kopt.hip), by the producer
+// here where only the rows are wanted.  No task row crosses PCIe on its way
+// in, and out only where the caller asks for rows or positions.
 //
 // Reference: KOptSearchCursor::PrepareNextBlock / PrepareNextK
 // (src/cpu/kopt_search.cpp:2123-2156, 2258-2271), AdvanceCombination

@@ -154,8 +154,8 @@ struct KoptLaunch {
   // row_status non-null: there are no task rows; row r is that of deletion
   // set row_first + r of `cursor`, made by the wavefront that evaluates it,
   // which also writes it to made_tasks[r] and its k positions to
-  // made_positions + k r, in host memory, and 1 to *row_status where the
-  // deleted cost overflows
+  // made_positions + k r, in host memory (either may be null), and 1 to
+  // *row_status where the deleted cost overflows
   KoptCursor cursor;
   uint64_t row_first;
   ee_kopt_task* made_tasks;

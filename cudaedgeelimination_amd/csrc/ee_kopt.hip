@@ -169,8 +169,8 @@ __device__ __forceinline__ void StagePorts(const KoptLaunch& a, const KoptPointe
 
 // Phase A of a tile whose rows are deletion sets of the tour context: lane r
 // makes row r, then the ports' coordinates are gathered as in StagePorts.
-// The rows and positions are staged in LDS and written to host memory in
-// whole words, consecutive lanes to consecutive addresses.
+// The rows and positions a caller wants are staged in LDS and written to host
+// memory in whole words, consecutive lanes to consecutive addresses.
 template <int K, bool kNear, int kOut>
 __device__ __forceinline__ void MakeRows(const KoptLaunch& a, const KoptPointers& bufs, const KoptKLayout& L,
                                          const KoptTile& d, char* wave, int lane) {
@@ -186,10 +186,12 @@ __device__ __forceinline__ void MakeRows(const KoptLaunch& a, const KoptPointers
     if (!CursorRow(a.cursor, K, a.row_first + d.task_index + r, pos, &row)) {
       __hip_atomic_store(a.row_status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    if (a.made_tasks != nullptr) {
 #pragma unroll
-    for (uint32_t p = 0; p < 10; ++p) w_task[r * 12 + p] = static_cast<uint32_t>(row.port_nodes[p]);
-    w_task[r * 12 + 10] = static_cast<uint32_t>(row.deleted_cost);
-    w_task[r * 12 + 11] = static_cast<uint32_t>(static_cast<uint64_t>(row.deleted_cost) >> 32);
+      for (uint32_t p = 0; p < 10; ++p) w_task[r * 12 + p] = static_cast<uint32_t>(row.port_nodes[p]);
+      w_task[r * 12 + 10] = static_cast<uint32_t>(row.deleted_cost);
+      w_task[r * 12 + 11] = static_cast<uint32_t>(static_cast<uint64_t>(row.deleted_cost) >> 32);
+    }
 #pragma unroll
     for (uint32_t p = 0; p < kPorts; ++p) w_node[r * kPorts + p] = row.port_nodes[p];
 #pragma unroll
@@ -208,10 +210,14 @@ __device__ __forceinline__ void MakeRows(const KoptLaunch& a, const KoptPointers
       *reinterpret_cast<longlong2*>(w_port + s * kFarPortBytes) = c;
     }
   }
-  uint32_t* tasks = reinterpret_cast<uint32_t*>(a.made_tasks + d.task_index);
-  for (uint32_t q = static_cast<uint32_t>(lane); q < d.rows * 12; q += kWave) tasks[q] = w_task[q];
-  uint32_t* positions = a.made_positions + static_cast<uint64_t>(d.task_index) * K;
-  for (uint32_t q = static_cast<uint32_t>(lane); q < d.rows * K; q += kWave) positions[q] = w_position[q];
+  if (a.made_tasks != nullptr) {
+    uint32_t* tasks = reinterpret_cast<uint32_t*>(a.made_tasks + d.task_index);
+    for (uint32_t q = static_cast<uint32_t>(lane); q < d.rows * 12; q += kWave) tasks[q] = w_task[q];
+  }
+  if (a.made_positions != nullptr) {
+    uint32_t* positions = a.made_positions + static_cast<uint64_t>(d.task_index) * K;
+    for (uint32_t q = static_cast<uint32_t>(lane); q < d.rows * K; q += kWave) positions[q] = w_position[q];
+  }
   WaveSync();
 }
 

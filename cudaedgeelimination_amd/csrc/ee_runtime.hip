@@ -452,7 +452,8 @@ KoptHits PrepareKoptCaches(Context& ctx, const int64_t* x, const int64_t* y, int
 
 // The rows of one evaluation, cut into launches that pass through the
 // context's page-locked ring.  A launch's slot holds an overflow flag, its
-// task rows (the caller's, or made ones on their way out) and positions, and
+// task rows (the caller's, or made ones on their way out) and positions, where
+// the caller wants them, and
 // its output: mask words, or cells in transfer form (low words, then high
 // bytes on instances that are not near).
 struct KoptChunks {
@@ -461,9 +462,11 @@ struct KoptChunks {
   // tile is 0.3 MB at most.  kPads: the parts of a slot start on 256 bytes.
   static constexpr size_t kPads = 5 * 256;
 
-  KoptChunks(size_t rows, uint32_t tile_rows, size_t position_bytes, size_t low_bytes, size_t high_bytes)
+  // The bytes of a row in each part of a slot; a part may be empty.
+  KoptChunks(size_t rows, uint32_t tile_rows, size_t task_bytes, size_t position_bytes, size_t low_bytes,
+             size_t high_bytes)
       : rows_(rows) {
-    const size_t per_row = sizeof(ee_kopt_task) + position_bytes + low_bytes + high_bytes;
+    const size_t per_row = task_bytes + position_bytes + low_bytes + high_bytes;
     const size_t tiles = (rows + tile_rows - 1) / tile_rows, tile_bytes = tile_rows * per_row;
     const bool whole = tiles <= DirectIo::kSlotTiles && tiles * tile_bytes + kPads <= DirectIo::kBytes;
     const size_t room = whole ? DirectIo::kBytes : DirectIo::kSlotBytes;
@@ -474,7 +477,7 @@ struct KoptChunks {
     const size_t even = (rows + count - 1) / count;
     chunk_rows = std::min(rows, (even + tile_rows - 1) / tile_rows * tile_rows);
     count = (rows + chunk_rows - 1) / chunk_rows;
-    positions_off = rows_off + Align256(chunk_rows * sizeof(ee_kopt_task));
+    positions_off = rows_off + Align256(chunk_rows * task_bytes);
     lo_off = positions_off + Align256(chunk_rows * position_bytes);
     hi_off = lo_off + Align256(chunk_rows * low_bytes);
     slot_bytes = hi_off + Align256(chunk_rows * high_bytes);
@@ -552,7 +555,8 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
   const uint32_t mask_words = (template_count + 31) / 32;
   const KoptTuning tuning = DirectTuning(k, masks != nullptr);
   const uint32_t tile_rows = tuning.rows_per_tile[k - 3];
-  const KoptChunks chunks(task_count, tile_rows, made ? 4 * k : 0, 4 * (masks ? mask_words : template_count),
+  const KoptChunks chunks(task_count, tile_rows, made && rows.out_tasks == nullptr ? 0 : sizeof(ee_kopt_task),
+                          rows.out_positions == nullptr ? 0 : 4 * k, 4 * (masks ? mask_words : template_count),
                           wide ? template_count : 0);
   DirectIo& io = ctx.io;
 
@@ -578,8 +582,10 @@ bool RunDirect(Context& ctx, int32_t n, uint8_t type, uint32_t k, uint32_t templ
       a.row_status = reinterpret_cast<uint32_t*>(device);
       a.cursor = rows.cursor;
       a.row_first = rows.first + chunks.First(chunk);
-      a.made_tasks = reinterpret_cast<ee_kopt_task*>(device + chunks.rows_off);
-      a.made_positions = reinterpret_cast<uint32_t*>(device + chunks.positions_off);
+      if (rows.out_tasks != nullptr) a.made_tasks = reinterpret_cast<ee_kopt_task*>(device + chunks.rows_off);
+      if (rows.out_positions != nullptr) {
+        a.made_positions = reinterpret_cast<uint32_t*>(device + chunks.positions_off);
+      }
     } else {
       const ee_kopt_task* from = rows.tasks + chunks.First(chunk);
       ee_kopt_task* staged = reinterpret_cast<ee_kopt_task*>(io.host() + at + chunks.rows_off);

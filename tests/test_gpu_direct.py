@@ -157,6 +157,37 @@ def test_made_rows_match_oracle(ctx, k, rows, output, box):
             assert not bits[:, improving.shape[1]:].any()
 
 
+@pytest.mark.parametrize("wanted", ["neither", "tasks", "positions"])
+@pytest.mark.parametrize("k, rows, output", [(4, 1, "masks"), (5, 9, "masks"), (5, 30_000, "masks"), (3, 65, "costs"),
+                                             (5, 4_999, "costs"), (5, 12_001, "costs")])
+def test_made_rows_left_out(ctx, k, rows, output, wanted):
+    """Made rows and positions reach host memory only where the caller passes
+    a buffer; the slots then hold more rows, and the results are the same."""
+    say(f"made rows k={k} rows={rows} {output}, wanted: {wanted}")
+    g = graph(rows, 900, EUC_2D, 1 << 30 if rows == 4_999 else 1_000_000)
+    tour = W.tour_context(rows, g, 200, 75)
+    table = backend.build_kopt_reconnect_table(k)
+    whole = backend.evaluate_kopt_cursor_cuda(g, table, tour, k, 3, rows, output, ctx)
+    rows = len(whole.tasks)
+    T = len(table.templates)
+    view, produced = tour.view(), C.c_uint32()
+    out = {"tasks": np.empty(rows, whole.tasks.dtype), "positions": np.empty((rows, k), np.uint32),
+           "costs": np.empty(rows * T, np.int64), "masks": np.empty((rows, (T + 31) // 32), np.uint32)}
+    for array in out.values():
+        array.view(np.uint8)[...] = 0xA5
+    _lib.check(_lib.lib().ee_kopt_cursor_eval(
+        ctx.handle, _lib.ptr(g.x), _lib.ptr(g.y), g.dimension, g.distance_type, C.byref(view), k,
+        _lib.ptr(table.templates), T, table.generator_hash, 3, rows,
+        *(_lib.ptr(out[name]) if name in (wanted, output) else None
+          for name in ("tasks", "positions", "costs", "masks")), C.byref(produced), None))
+    assert produced.value == rows
+    for name, array in out.items():
+        if name in (wanted, output):
+            assert np.array_equal(array, getattr(whole, name))
+        else:
+            assert (array.view(np.uint8) == 0xA5).all()
+
+
 def star(n, hub_degree, seed=3):
     """A k-NN graph with one hub joined to `hub_degree` further nodes."""
     g = graph(seed, n, EUC_2D, 1_000_000)
