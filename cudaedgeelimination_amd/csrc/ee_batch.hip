@@ -18,7 +18,7 @@ namespace {
 
 constexpr uint32_t kTemplateCount[3] = {4, 25, 208};
 // Bumped whenever the k-opt kernel changes, so cached tunings are retuned.
-constexpr int kKernelRevision = 8;
+constexpr int kKernelRevision = 9;
 
 struct Batch {
   explicit Batch(Context* c) : ctx(c) {}

@@ -421,6 +421,29 @@ def test_set_work_without_room(ctx, output):
     batch.close()
 
 
+def test_tunings_of_an_older_kernel_are_retuned(ctx, tmp_path):
+    """A stored tuning is taken under its own key, and not where its key names
+    the kernel's revision 8, before it wrote packed cells and made rows."""
+    say("stored tunings")
+    g = graph(29, 300, EUC_2D, 1_000_000)
+    tasks = W.kopt_tasks(3, g, np.full(64, 4, np.uint8))
+    batch = KoptBatch(ctx)
+    batch.set_work([(batch.add_instance(g), 4, 64)], tasks)
+    cache = tmp_path / "tunings"
+    batch.autotune(1, str(cache))
+    key = cache.read_text().split()[0]
+    assert key.startswith("kopt") and int(key[4:].split("/")[0]) > 8
+    planted = "17 13 11 3 192 0"  # options the search never tries
+    cache.write_text(f"{key} {planted}\n")
+    assert batch.autotune(1, str(cache))["grid"] == 3
+    cache.write_text(f"kopt8/{key.split('/', 1)[1]} {planted}\n")
+    assert batch.autotune(1, str(cache))["grid"] != 3
+    batch.run()
+    want, _, _ = O.kopt_costs(g.x, g.y, EUC_2D, 4, tasks)
+    assert np.array_equal(batch.segment_costs(0), want)
+    batch.close()
+
+
 @pytest.mark.parametrize("n, neighbors", [(4, 3), (41, 6), (700, 10), (60_000, 8)])
 def test_jv_call_inputs(ctx, n, neighbors):
     """The dynamic arrays on their way in (one slot and several; odd counts;
