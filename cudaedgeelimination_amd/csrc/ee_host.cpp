@@ -213,7 +213,6 @@ KoptPlan BuildPlan(uint32_t k, const ee_endpoint_matching* templates, uint32_t c
   return plan;
 }
 
-// ValidateKOptCostTask (src/cpu/kopt_search.cpp:784-807).
 namespace {
 
 // The compiler vectorises both loops; with 256-bit registers one core writes
@@ -248,6 +247,7 @@ void ExpandCells(const uint32_t* lo, const uint8_t* hi, size_t count, int64_t* c
   (avx2 ? ExpandAvx2 : ExpandBase)(lo, hi, count, cells);
 }
 
+// ValidateKOptCostTask (src/cpu/kopt_search.cpp:784-807).
 void ValidateTasks(int32_t n, uint32_t k, const ee_kopt_task* tasks, size_t count) {
   for (size_t r = 0; r < count; ++r) {
     const ee_kopt_task& t = tasks[r];

@@ -201,12 +201,10 @@ struct KoptTileSource {
 void LaunchKoptTiles(const KoptTileSource* sources, uint32_t count, uint64_t tile_count, KoptTile* tiles,
                      hipStream_t stream);
 
-// Number of tiles the segments split into under `tuning`.
-uint64_t KoptCountTiles(const KoptSegment* segments, size_t count, const KoptTuning& tuning);
 // Sets rows_per_tile and tile_begin of every segment, numbering tiles k by k,
-// writes the descriptor of every tile to `tiles` (KoptCountTiles entries; the
-// segments' instances index `instances`; may be null) and the per-k tile
-// ranges to `a`.  Launches of at most kInlineSegments segments also get the
+// writes the descriptor of every tile to `tiles` (as many as the segments
+// split into, ceil(task_count / rows_per_tile) each; the segments' instances
+// index `instances`; may be null) and the per-k tile ranges to `a`.  Launches of at most kInlineSegments segments also get the
 // inline segment table (a->inline_count > 0): their kernels ignore `tiles`,
 // so callers need not upload the descriptors.
 void KoptAssignTiles(KoptSegment* segments, size_t count, const KoptInstance* instances,

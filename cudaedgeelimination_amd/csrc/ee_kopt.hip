@@ -1160,15 +1160,6 @@ size_t KoptPrepareLayout(KoptLaunch* a, const KoptPlan plans[3], const bool pres
   return static_cast<size_t>(plan_bytes) + static_cast<size_t>(wave_bytes) * (tuning.block / kWave);
 }
 
-uint64_t KoptCountTiles(const KoptSegment* segments, size_t count, const KoptTuning& tuning) {
-  uint64_t tiles = 0;
-  for (size_t i = 0; i < count; ++i) {
-    const uint32_t rows = tuning.rows_per_tile[segments[i].k - 3];
-    tiles += (segments[i].task_count + rows - 1) / rows;
-  }
-  return tiles;
-}
-
 void KoptAssignTiles(KoptSegment* segments, size_t count, const KoptInstance* instances,
                      const KoptPlan plans[3], const KoptTuning& tuning, KoptTile* tiles,
                      KoptLaunch* a) {

@@ -542,7 +542,7 @@ KoptTuning DirectTuning(uint32_t k, bool masks) {
 // bounds a block: 61 us for 4,096 k = 5 rows).  Host threads take tiles into
 // the caller's buffers as their marks arrive.  Against an upload, a launch
 // and a download with a wait each: one k = 5 row 56 -> 19 us, 1,237 k = 4
-// rows 63 -> 32 us, 4,096 k = 5 rows 293 -> 121 us, 1,501 wide k = 5 rows
+// rows 63 -> 34 us, 4,096 k = 5 rows 293 -> 121 us, 1,501 wide k = 5 rows
 // 163 -> 83 us, 4,096 made k = 5 rows with their masks 125 -> 60 us.
 // `check` runs on the host while the first launches are on the device; false
 // drops their output and returns false, with nothing delivered.

@@ -184,7 +184,7 @@ void Server::Fail(std::vector<std::shared_ptr<Request>>& batch, const std::strin
   cv_done.notify_all();
 }
 
-// Stages one batch into a slot and enqueues upload, launch and download.
+// Stages one batch into a slot and enqueues its launches.
 bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
   try {
     CheckHip(hipSetDevice(ctx->device), "hipSetDevice");
@@ -456,7 +456,7 @@ void Server::Loop() {
     }
     if (Issue(*free_slot, std::move(batch))) {
       if (slots.size() == 1) {
-        // one slot: the plain path, upload, launch and download in turn
+        // one slot: the plain path, one batch staged, launched and waited for
         Finish(*free_slot);
         continue;
       }

@@ -297,8 +297,8 @@ class KoptServer:
     """Serving loop over device-resident graphs (ee_server_* in ee_hip.h).
 
     batching=True: continuous batching with two pipeline slots;
-    batching=False: the plain per-query path (one request per launch, one
-    synchronous upload / launch / download at a time)."""
+    batching=False: the plain per-query path (one request per launch, each
+    waited for before the next)."""
 
     def __init__(self, ctx: Context, hbm_budget_bytes: int = 1 << 30,
                  max_batch_cells: int = 1 << 21, max_batch_requests: int = 256,
