@@ -186,6 +186,7 @@ void Server::Fail(std::vector<std::shared_ptr<Request>>& batch, const std::strin
 
 // Stages one batch into a slot and enqueues its launches.
 bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
+  bool new_graphs = false, new_jv = false;  // taken off the dirty flags, not yet resident
   try {
     CheckHip(hipSetDevice(ctx->device), "hipSetDevice");
     std::vector<longlong2> xy_copy;
@@ -197,10 +198,12 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
         xy_copy = host_xy;
         inst_copy = instances;
         graphs_dirty = false;
+        new_graphs = true;
       }
       if (jv_dirty) {
         jv_copy = std::make_unique<JvUnion>(jv);
         jv_dirty = false;
+        new_jv = true;
       }
     }
     if (!inst_copy.empty() || jv_copy) {
@@ -212,6 +215,7 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
       d_xy.Upload(xy_copy.data(), xy_copy.size(), slot.stream);
       CheckHip(hipStreamSynchronize(slot.stream), "hipStreamSynchronize");
       worker_instances = std::move(inst_copy);
+      new_graphs = false;
     }
     if (jv_copy) {
       const JvUnion& u = *jv_copy;
@@ -234,6 +238,7 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
       d_jv_edge_ids.Upload(u.edge_ids.data(), u.edge_ids.size(), slot.stream);
       CheckHip(hipStreamSynchronize(slot.stream), "hipStreamSynchronize");
       worker_jv_slots = static_cast<int32_t>(u.uv.size());
+      new_jv = false;
     }
     // leaf-cost requests: one tiled k-opt launch; JV rechecks: one JV launch
     uint64_t rows = 0, cells = 0, tiles = 0, items = 0;
@@ -338,6 +343,12 @@ bool Server::Issue(Slot& slot, std::vector<std::shared_ptr<Request>> batch) {
     return true;
   } catch (const std::exception& e) {
     static_cast<void>(hipStreamSynchronize(slot.stream));  // a launch may still use the slot's memory
+    {
+      // graphs that found no room: the next batch tries again before it launches
+      std::lock_guard<std::mutex> lk(mu);
+      graphs_dirty = graphs_dirty || new_graphs;
+      jv_dirty = jv_dirty || new_jv;
+    }
     Fail(batch, e.what());
     return false;
   }
