@@ -707,21 +707,19 @@ uint64_t CountVerdicts(HtCache& c, uint64_t* offsets) {
   return run;
 }
 
-// As HamiltonReplies below, by verdict bits.  started: the pass is under way.
-void VerdictReplies(Context& ctx, const ee_graph_view& g, int32_t tu, int32_t tv, const int32_t* centers,
-                    size_t count, const VerdictPlan& plan, bool started, uint64_t* offsets, ee_ht_neighbor_pair* replies, uint64_t capacity,
-                    uint64_t* total, ee_ht_usage* u) {
+// As HamiltonReplies below, by the verdict bits of the pass launched at
+// `launched`.
+void VerdictReplies(Context& ctx, std::chrono::steady_clock::time_point launched, uint64_t* offsets,
+                    ee_ht_neighbor_pair* replies, uint64_t capacity, uint64_t* total, ee_ht_usage* u) {
   HtCache& c = ctx.ht;
-  auto t0 = std::chrono::steady_clock::now();
-  if (!started) u->workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count, plan) ? 1 : 0;
   ctx.Sync();
+  u->kernel_ms = MsSince(launched);
+  const auto t0 = std::chrono::steady_clock::now();
   *total = CountVerdicts(c, offsets);
-  u->kernel_ms = MsSince(t0);
   c.current ^= 1;
   c.last_kind = 1;
   c.last_bits = true;
   c.last_total = *total;
-  t0 = std::chrono::steady_clock::now();
   const uint64_t copy = std::min(*total, capacity);
   if (copy > 0) CopyVerdictReplies(c, 0, copy, reinterpret_cast<int32_t*>(replies));
   u->d2h_ms = MsSince(t0);
@@ -752,7 +750,13 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
   VerdictPlan plan;
   if (likely) plan = PlanVerdicts(ctx.ht, centers, count);
   bool started = plan.take;
-  if (started) u.workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count, plan) ? 1 : 0;
+  std::chrono::steady_clock::time_point launched;
+  const auto launch = [&] {
+    u.workspace_hit = LaunchVerdicts(ctx, g.distance_type, tu, tv, centers, count, plan) ? 1 : 0;
+    u.h2d_ms = MsSince(t0);
+    launched = std::chrono::steady_clock::now();
+  };
+  if (started) launch();
   try {
     u.graph_hit = HtGraphMatches(ctx.ht, g) ? 1 : 0;
     if (!u.graph_hit) ValidateHtGraph(g);
@@ -777,8 +781,8 @@ void HamiltonReplies(Context& ctx, const ee_graph_view* graph, int32_t target_u,
   }
   if (!started) plan = PlanVerdicts(c, centers, count);
   if (plan.take) {
-    u.h2d_ms = MsSince(t0);
-    VerdictReplies(ctx, g, tu, tv, centers, count, plan, started, offsets, replies, capacity, total, &u);
+    if (!started) launch();
+    VerdictReplies(ctx, launched, offsets, replies, capacity, total, &u);
     if (usage) *usage = u;
     return;
   }

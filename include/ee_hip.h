@@ -259,9 +259,10 @@ typedef struct {
  * last one's), which grows to at most twice what a call needed and 80 MiB
  * each.  The snapshot must pass the reference's HT graph checks
  * (ht_replies.cu:521-553): a symmetric CSR of exactly the active edges,
- * rows strictly ascending.  usage->h2d_ms covers the checks, beside which the
- * pass over a resident snapshot already runs, usage->kernel_ms the wait for
- * the rest of it, and usage->d2h_ms the writing of the replies. */
+ * rows strictly ascending.  usage->h2d_ms is the time to the first launch
+ * (with the checks and the upload of a snapshot that is not resident),
+ * usage->kernel_ms from there to the end of the passes (the checks of a
+ * resident snapshot run beside them), usage->d2h_ms the offsets and replies. */
 ee_status ee_ht_hamilton_replies(ee_ctx* ctx, const ee_graph_view* graph, int32_t target_u,
                                  int32_t target_v, const int32_t* centers, size_t center_count,
                                  uint64_t* offsets, ee_ht_neighbor_pair* replies, uint64_t capacity,

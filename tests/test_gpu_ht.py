@@ -70,6 +70,21 @@ def test_every_node_of_a_30k_graph(ctx):
     assert len(rep) > 0
 
 
+def test_phase_times_of_a_resident_call(ctx):
+    """The pass goes out before the checks of a resident snapshot: they count
+    beside the kernel, not as the way in."""
+    g = W.config5_graphs(sizes=(30000,))[0]
+    target = (int(g.edge_u[0]), int(g.edge_v[0]))
+    centers = np.setdiff1d(np.arange(g.dimension), target).astype(np.int32)
+    say("ht phase times")
+    times = []
+    for _ in range(6):
+        _, rep, u = backend.evaluate_ht_hamilton_replies_cuda(g, target, centers, ctx)
+        times.append((u.h2d_ms, u.kernel_ms, u.d2h_ms))
+    h2d, kernel, d2h = np.median(np.array(times[1:]), axis=0)
+    assert u.graph_hit and 0 < h2d < kernel and d2h > 0
+
+
 def test_cache_usage_and_checks(ctx, snapshots):
     say("ht cache and checks")
     g = snapshots["uniform300"]
