@@ -558,9 +558,10 @@ void WriteReplies(const HtCache& c, const HtCache::Verdicts& v, const uint64_t* 
 }
 
 // Host threads: writing 19 MB of replies takes 12 about 0.15 ms.  Below
-// kSerialReplies waking them costs more than it saves.
+// kSerialReplies waking them costs more than it saves: 37,500 replies take 17
+// us on one thread, 48,500 21 and 103,000 46; 20, 20 and 25 on 12.
 constexpr unsigned kReplyThreads = 12;
-constexpr uint64_t kSerialReplies = 100000;
+constexpr uint64_t kSerialReplies = 50000;
 
 // Replies [first, first + count) of the last verdicts.
 void CopyVerdictReplies(const HtCache& c, uint64_t first, uint64_t count, int32_t* out) {
@@ -614,8 +615,8 @@ struct VerdictPlan {
 //  - kMeanWords: the form is faster as far as both were measured, from the
 //    smallest calls (one launch and one wait for four and three): whole calls
 //    on k-NN graphs, 300 to 30,000 centers with 3 to 52 words each, 154-5,260
-//    us by three passes and 73-2,020 by bits; complete graphs of 40 to 90
-//    nodes (12 to 62 words) 91-455 and 60-189.  Beyond, replies are hundreds
+//    us by three passes and 71-1,950 by bits; complete graphs of 40 to 90
+//    nodes (12 to 62 words) 91-455 and 60-190.  Beyond, replies are hundreds
 //    of MB, which PCIe carries about as fast as host threads write them.
 //  - kBitsDegree: pair numbers stay exact in the kernel's float root.
 //  - kBitsBytes and kBitsCenters bound what a context keeps page-locked.
@@ -657,8 +658,11 @@ bool LaunchVerdicts(Context& ctx, int type, int32_t tu, int32_t tv, const int32_
   v.stride = plan.stride;
   v.per_wave = plan.per_wave;
   v.count = count;
-  // groups of the host's work: some 512 words, whole wavefronts
-  v.group = std::max<size_t>(4, std::min<size_t>(256, 512 * count / std::max<size_t>(plan.words, 1)) / 4 * 4);
+  // groups of the host's work, whole wavefronts: 256 centers or some 1,024
+  // words (half of that took 5 us more for 30,000 centers, whose groups then
+  // share more of the replies' untouched pages), and as many as threads
+  const size_t most = std::min<size_t>(256, 1024 * count / std::max<size_t>(plan.words, 1));
+  v.group = (std::min(most, (count + kReplyThreads - 1) / kReplyThreads) + 3) / 4 * 4;
   const size_t waves = (count + plan.per_wave - 1) / plan.per_wave;
   const size_t ints = 2 * count + (plan.stride != 0 ? 0 : waves), words = std::max<size_t>(plan.words, 1);
   const bool room = v.centers.count() >= ints && v.bits.count() >= words;
