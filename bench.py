@@ -5,7 +5,8 @@ beside it, the multi-epoch JV workload (60 x 60 drilling-grid lattice, 10-NN).
 
 One step = one evaluation of the whole cost matrix by the resident batched
 path (one kernel launch over all three k segments, inputs already in HBM).
-Prints one JSON line; see the keys below.
+Prints one JSON line; see the keys below.  The legs beside the headline are
+shortened on it (``compact``); stderr has every figure.
 
   python bench.py [--gpus 1] [--steps 20] [--warmup 5] [--no-cpu] [--no-jv]
 """
@@ -316,6 +317,44 @@ def serve_stream(ctx, graphs, pools, requests, is_jv, arrivals, mode: str, burst
     if outputs is not None:
         out["outputs"] = outputs
     return out
+
+
+# of the line, whole; the other legs are shortened
+WHOLE = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+         "vs_baseline", "dtype", "data", "config", "roofline", "cpu_baseline", "parity")
+
+
+def compact(result: dict) -> dict:
+    """The result as one line of some 6 KB: a reader that keeps only the end of
+    the output lost the head of the whole one (21 KB).  The legs beside the
+    headline keep their own figures, to five digits, and of the serving legs
+    each path's latencies per rate and its saturation.  The whole result goes
+    to stderr."""
+    def short(v):
+        return float(f"{v:.5g}") if isinstance(v, float) else v
+
+    def own(leg, nested=False):
+        return {k: own(v) if isinstance(v, dict) else short(v) for k, v in leg.items()
+                if not isinstance(v, list) and (nested or not isinstance(v, dict))}
+
+    def stream(leg):
+        out = {}
+        for p in leg["points"]:
+            out[str(p["qps"])] = {path: [short(v["p50_ms"]), short(v["p99_ms"])] for path, v in p.items()
+                                  if isinstance(v, dict)}
+        out["columns"] = ["p50_ms", "p99_ms"]
+        burst = [p for p in leg["points"] if "results_equal_across_paths" in p]
+        if burst:
+            out["burst_results_equal_across_paths"] = all(p["results_equal_across_paths"] for p in burst)
+        out["saturation_qps"] = {k: v["saturation_qps"] for k, v in (leg.get("saturation") or {}).items()
+                                 if isinstance(v, dict)}
+        if leg.get("leaf_only"):
+            out["leaf_only"] = stream(leg["leaf_only"])
+        return out
+
+    return {k: v if k in WHOLE or not isinstance(v, dict) else stream(v) if k == "serving"
+            else own(v, k in ("cursor", "many_instance", "improving_masks"))
+            for k, v in result.items()}
 
 
 def serving_leg(ctx, qps_list, seconds: float, seed: int = 0xEE000005, jv_share: float = 0.2,
@@ -967,7 +1006,8 @@ def main() -> int:
 
     batch.close()
     ctx.close()
-    print(json.dumps(result), flush=True)
+    log("every figure: " + json.dumps(result))
+    print(json.dumps(compact(result)), flush=True)
     return 0
 
 
