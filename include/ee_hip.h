@@ -69,8 +69,9 @@ ee_status ee_backend_available(int device, char* reason, size_t reason_capacity)
  * else sticky, else the device with the most free memory.  Here the forced
  * ordinal is the `device` argument; device = -1 picks the device with the
  * most free memory.  A context must be used by one host thread at a time.
- * Batches, sessions and servers created on a context must be destroyed
- * before the context. */
+ * Batches, sessions, fleets, servers, queues and leaf pipelines created on a
+ * context must be destroyed before the context (sessions and fleets return
+ * their memory to it). */
 typedef struct ee_ctx ee_ctx;
 ee_status ee_ctx_create(int device, ee_ctx** out);
 void ee_ctx_destroy(ee_ctx* ctx);
